@@ -125,7 +125,7 @@ struct lbm_trainer {
     long long capacity, count;
     float *feat, *target;   // capacity x 10, capacity
     float *w, *m, *v;       // LBM_MLP_TOTAL parameters, Adam moments
-    float *partial, *grad;  // per-wave partial gradients, summed gradient (+ loss)
+    float *partial, *grad;  // per-block partial gradients, summed gradient (+ loss)
     uint32_t max_waves;
     int step;
     int target_mode; // LBM_TARGET_LOCAL or LBM_TARGET_PLANE for lbm_trainer_add_filtered
@@ -2198,7 +2198,7 @@ int lbm_trainer_create(int device, long long capacity, const float *params, lbm_
         hipMalloc((void **)&t->w, MLP_TOTAL * sizeof(float)) != hipSuccess ||
         hipMalloc((void **)&t->m, MLP_NPARAM * sizeof(float)) != hipSuccess ||
         hipMalloc((void **)&t->v, MLP_NPARAM * sizeof(float)) != hipSuccess ||
-        hipMalloc((void **)&t->partial, (size_t)t->max_waves * (MLP_NPARAM + 1) * sizeof(float)) != hipSuccess ||
+        hipMalloc((void **)&t->partial, (size_t)MLP_GRAD_BLOCKS * (MLP_NPARAM + 1) * sizeof(float)) != hipSuccess ||
         hipMalloc((void **)&t->grad, (MLP_NPARAM + 1) * sizeof(float)) != hipSuccess)
         return cleanup(fail(LBM_ERR_NOMEM, "lbm_trainer_create: device allocation failed"));
     if (hipMemcpyAsync(t->w, params, MLP_TOTAL * sizeof(float), hipMemcpyHostToDevice, t->stream) != hipSuccess ||
@@ -2377,7 +2377,7 @@ static int trainer_range(lbm_trainer *t, long long first, long long count, const
     return LBM_OK;
 }
 
-// One gradient pass covers at most max_waves waves of 64 samples.
+// One gradient pass covers at most max_waves times 64 samples.
 static int trainer_batch(lbm_trainer *t, long long batch, const char *fn)
 {
     if ((batch + 63) / 64 > (long long)t->max_waves)

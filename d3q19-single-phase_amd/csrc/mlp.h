@@ -56,31 +56,6 @@ __device__ __forceinline__ float mlp_nut(const float *__restrict__ w, float o)
     return softplus(o) + w[MLP_NUTMIN];
 }
 
-// Network output o for one node's inputs x (already scaled), FP32 on the
-// vector ALUs: the training and prediction kernels' forward pass.
-__device__ __forceinline__ float mlp_forward(const float *__restrict__ w, const float (&x)[MLP_IN])
-{
-    float h1[MLP_H];
-#pragma unroll
-    for (int j = 0; j < MLP_H; j++) {
-        float a = w[MLP_B1 + j];
-#pragma unroll
-        for (int k = 0; k < MLP_IN; k++)
-            a = fmaf(w[MLP_W1 + j * MLP_IN + k], x[k], a);
-        h1[j] = fast_tanh(a);
-    }
-    float o = w[MLP_B3];
-#pragma unroll 4
-    for (int j = 0; j < MLP_H; j++) {
-        float a = w[MLP_B2 + j];
-#pragma unroll
-        for (int k = 0; k < MLP_H; k++)
-            a = fmaf(w[MLP_W2 + j * MLP_H + k], h1[k], a);
-        o = fmaf(w[MLP_W3 + j], fast_tanh(a), o);
-    }
-    return o;
-}
-
 // Shear relaxation rate from the network output.
 __device__ __forceinline__ float mlp_rate(const float *__restrict__ w, float o)
 {
