@@ -14,6 +14,7 @@
 // the result equals the reference's in-place swap algorithm bit for bit.
 #pragma once
 
+#include <algorithm>
 #include <utility>
 
 #include "d3q19_common.h"
@@ -872,23 +873,75 @@ __global__ void __launch_bounds__(BLOCK) k_mass_partials(SumArgs a)
         a.partials[blockIdx.x] = s;
 }
 
-// Plane sums for the statistics of Channel-Flow/saveload.f90:1382-1409:
-// per wall-normal index ix, the sums over the fluid nodes (iy, iz) of
-// ux, uy, uz, ux*uz, ux*uy, uy*uz, ux^2, uy^2, uz^2, rho, rho^2, and their count.
-// Block (blockIdx.x, blockIdx.y) handles ix = blockIdx.y*blockDim.x + tid and
-// rows blockIdx.x, blockIdx.x + gridDim.x, ...; partials[(c*11 + q)*lx + ix].
+// Plane sums run in blocks of blockDim.x wall-normal columns by blockDim.y
+// rows: lane (x, y) of block (chunk, x tile) strides over rows chunk *
+// blockDim.y + y, and the block adds its row lanes in order before it writes
+// its partials.  They are bound by the lattice read (the 192x768x384 channel
+// in FP32 storage, 4.3 GB: 731 us for the statistics, 726 us filtered, 794 us
+// for dissipation_calc, 5.4-5.9 TB/s).  Threads per block, 512 chunks: the
+// statistics' arithmetic hides at any number, and fewer waves read faster
+// (256 threads 731 us, 768 threads 800 us); dissipation_calc needs the waves
+// (1 021 us with 256, 794 us with 768).
+constexpr int PLANE_THREADS = 256, DISS_THREADS = 768;
+
+// Add the row lanes' sums s in order of y and write partial
+// (chunk * Q + q) * nx + ix for ix < nx.  Every thread of the block calls this.
+template <int Q>
+__device__ __forceinline__ void plane_write_partials(double (&s)[Q], uint32_t ix, uint32_t nx, double *partials)
+{
+    __shared__ double part[Q][BLOCK];
+    for (uint32_t y = 1; y < blockDim.y; y++) {
+        if (threadIdx.y == y) {
+#pragma unroll
+            for (int q = 0; q < Q; q++)
+                part[q][threadIdx.x] = s[q];
+        }
+        __syncthreads();
+        if (threadIdx.y == 0) {
+#pragma unroll
+            for (int q = 0; q < Q; q++)
+                s[q] += part[q][threadIdx.x];
+        }
+        __syncthreads();
+    }
+    if (threadIdx.y == 0 && ix < nx) {
+        double *out = partials + (uint64_t)blockIdx.x * Q * nx;
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+            out[(uint64_t)q * nx + ix] = s[q];
+    }
+}
+
+// ux, uy, uz, ux*uz, ux*uy, uy*uz, ux^2, uy^2, uz^2, rho, rho^2 and the count.
+__device__ __forceinline__ void plane_add(double (&s)[NPLANE], double rho, double ux, double uy, double uz)
+{
+    s[0] += ux;
+    s[1] += uy;
+    s[2] += uz;
+    s[3] += ux * uz;
+    s[4] += ux * uy;
+    s[5] += uy * uz;
+    s[6] += ux * ux;
+    s[7] += uy * uy;
+    s[8] += uz * uz;
+    s[9] += rho;
+    s[10] += rho * rho;
+    s[11] += 1.0;
+}
+
+// Plane sums for the statistics of Channel-Flow/saveload.f90:1382-1409: per
+// wall-normal index ix, the sums of plane_add over the fluid nodes (iy, iz);
+// partials[(chunk*NPLANE + q)*lx + ix].
 // SRC 0: field arrays; SRC 1: macrovar(F) of lattice L with rho - rho_off.
 template <int P, int SRC>
-__global__ void __launch_bounds__(BLOCK) k_plane_partials(PlaneArgs a)
+__global__ void __launch_bounds__(PLANE_THREADS) k_plane_partials(PlaneArgs a)
 {
     using S = typename Prec<P>::S;
     using T = typename Prec<P>::T;
     const uint32_t ix = blockIdx.y * blockDim.x + threadIdx.x;
-    if (ix >= a.g.lx)
-        return;
     double s[NPLANE] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const uint32_t rows = a.g.ly * a.g.lz;
-    for (uint32_t row = blockIdx.x; row < rows; row += gridDim.x) {
+    const uint32_t rows = ix < a.g.lx ? a.g.ly * a.g.lz : 0u;
+    for (uint32_t row = blockIdx.x * blockDim.y + threadIdx.y; row < rows; row += gridDim.x * blockDim.y) {
         const uint32_t n = row * a.g.lx + ix;
         if (a.solid && a.solid[n] >= 0)
             continue;
@@ -913,80 +966,56 @@ __global__ void __launch_bounds__(BLOCK) k_plane_partials(PlaneArgs a)
             uz = (double)(uz9 + (T)fz / T(2.));
             rho = (double)(rho9 - (T)a.rho_off);
         }
-        s[0] += ux;
-        s[1] += uy;
-        s[2] += uz;
-        s[3] += ux * uz;
-        s[4] += ux * uy;
-        s[5] += uy * uz;
-        s[6] += ux * ux;
-        s[7] += uy * uy;
-        s[8] += uz * uz;
-        s[9] += rho;
-        s[10] += rho * rho;
-        s[11] += 1.0;
+        plane_add(s, rho, ux, uy, uz);
     }
-    double *out = a.partials + (uint64_t)blockIdx.x * NPLANE * a.g.lx;
-#pragma unroll
-    for (int q = 0; q < NPLANE; q++)
-        out[(uint64_t)q * a.g.lx + ix] = s[q];
+    plane_write_partials(s, ix, a.g.lx, a.partials);
 }
 
 // The same plane sums for the 2x2x2 box-filtered fields on the grid of half
 // the size: coarse node (cx, cy, cz) carries the means of rho and u (macrovar
 // of F, with F/2 and rho_off) over fine nodes (2cx+{0,1}, 2cy+{0,1},
-// 2cz+{0,1}).  Partials are laid out for lx/2 planes.  Even lx, ly, lz.
+// 2cz+{0,1}).  A lane takes one fine column, so its loads are contiguous
+// across the wave, and adds the four fine nodes of a coarse row; its
+// neighbour holds the other column of the coarse node.  (A lane per coarse
+// column, 96 of 128 lanes loading every second value, took 1 242 us on the
+// 192x768x384 channel in FP32.)  Partials are laid out for lx/2 planes.  Even
+// lx, ly, lz.
 template <int P>
-__global__ void __launch_bounds__(BLOCK) k_filtered_plane_partials(PlaneArgs a)
+__global__ void __launch_bounds__(PLANE_THREADS) k_filtered_plane_partials(PlaneArgs a)
 {
     using S = typename Prec<P>::S;
     using T = typename Prec<P>::T;
-    const uint32_t lxc = a.g.lx / 2, lyc = a.g.ly / 2;
-    const uint32_t ic = blockIdx.y * blockDim.x + threadIdx.x;
-    if (ic >= lxc)
-        return;
+    const uint32_t lyc = a.g.ly / 2;
+    const uint32_t ix = blockIdx.y * blockDim.x + threadIdx.x;
     double s[NPLANE] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const uint32_t rows = lyc * (a.g.lz / 2);
-    for (uint32_t row = blockIdx.x; row < rows; row += gridDim.x) {
-        const uint32_t cy = row % lyc, cz = row / lyc;
+    // both lanes of a pair take the same rows: lx is even
+    const uint32_t rows = ix < a.g.lx ? lyc * (a.g.lz / 2) : 0u;
+    for (uint32_t row = blockIdx.x * blockDim.y + threadIdx.y; row < rows; row += gridDim.x * blockDim.y) {
+        const uint32_t cz = row / lyc, cy = row - cz * lyc;
         double rho = 0.0, ux = 0.0, uy = 0.0, uz = 0.0;
         for (uint32_t dz = 0; dz < 2; dz++)
-            for (uint32_t dy = 0; dy < 2; dy++)
-                for (uint32_t dx = 0; dx < 2; dx++) {
-                    const uint32_t n = (2 * ic + dx) + a.g.lx * ((2 * cy + dy) + a.g.ly * (2 * cz + dz));
-                    const Nbr b = make_nbr(n, a.g);
-                    T f[19];
-                    pull_all<P>((const S *)a.L, a.g.N, b, f);
-                    T rho9, ux9, uy9, uz9;
-                    macro_sums(f, rho9, ux9, uy9, uz9);
-                    double fx, fy, fz;
-                    node_force(a.f, a.g, 2 * ic + dx, 2 * cy + dy, 2 * cz + dz, fx, fy, fz);
-                    ux += (double)(ux9 + (T)fx / T(2.));
-                    uy += (double)(uy9 + (T)fy / T(2.));
-                    uz += (double)(uz9 + (T)fz / T(2.));
-                    rho += (double)(rho9 - (T)a.rho_off);
-                }
-        rho *= 0.125;
-        ux *= 0.125;
-        uy *= 0.125;
-        uz *= 0.125;
-        s[0] += ux;
-        s[1] += uy;
-        s[2] += uz;
-        s[3] += ux * uz;
-        s[4] += ux * uy;
-        s[5] += uy * uz;
-        s[6] += ux * ux;
-        s[7] += uy * uy;
-        s[8] += uz * uz;
-        s[9] += rho;
-        s[10] += rho * rho;
-        s[11] += 1.0;
+            for (uint32_t dy = 0; dy < 2; dy++) {
+                const uint32_t n = ix + a.g.lx * ((2 * cy + dy) + a.g.ly * (2 * cz + dz));
+                const Nbr b = make_nbr(n, a.g);
+                T f[19];
+                pull_all<P>((const S *)a.L, a.g.N, b, f);
+                T rho9, ux9, uy9, uz9;
+                macro_sums(f, rho9, ux9, uy9, uz9);
+                double fx, fy, fz;
+                node_force(a.f, a.g, ix, 2 * cy + dy, 2 * cz + dz, fx, fy, fz);
+                ux += (double)(ux9 + (T)fx / T(2.));
+                uy += (double)(uy9 + (T)fy / T(2.));
+                uz += (double)(uz9 + (T)fz / T(2.));
+                rho += (double)(rho9 - (T)a.rho_off);
+            }
+        rho += __shfl_xor(rho, 1);
+        ux += __shfl_xor(ux, 1);
+        uy += __shfl_xor(uy, 1);
+        uz += __shfl_xor(uz, 1);
+        plane_add(s, rho * 0.125, ux * 0.125, uy * 0.125, uz * 0.125);
     }
-    double *out = a.partials + (uint64_t)blockIdx.x * NPLANE * lxc;
-#pragma unroll
-    for (int q = 0; q < NPLANE; q++)
-        out[(uint64_t)q * lxc + ic] = s[q];
+    // the even lane of a pair writes coarse column ix / 2
+    plane_write_partials(s, (ix & 1u) ? a.g.lx : ix / 2, a.g.lx / 2, a.partials);
 }
 
 // ---------------------------------------------------------------------------
@@ -1118,8 +1147,7 @@ __global__ void __launch_bounds__(BLOCK) k_diag_partials(DiagArgs a)
     }
 }
 
-// Per-node strain of dissipation_calc (Channel-Flow/saveload.f90:4677-4776)
-// in the reference's operand order: v[0] = S_ij S_ij and v[1] = S_xy from
+// Per-node strain of dissipation_calc (Channel-Flow/saveload.f90:4677-4776): v[0] = S_ij S_ij and v[1] = S_xy from
 // the non-equilibrium moments, v[2], v[3] the same from the non-equilibrium
 // populations.
 __device__ inline void dissipation_node(const DissArgs &a, const double *f9, double rho9, double ux9, double uy9,
@@ -1161,41 +1189,32 @@ __device__ inline void dissipation_node(const DissArgs &a, const double *f9, dou
     double Szx = -1.5 * neqm15;
     v[0] = Sxx * Sxx + Syy * Syy + Szz * Szz + 2.0 * (Sxy * Sxy + Syz * Syz + Szx * Szx);
     v[1] = Sxy;
-    Sxx = 0.0;
-    Syy = 0.0;
-    Szz = 0.0;
-    Sxy = 0.0;
-    Syz = 0.0;
-    Szx = 0.0;
-    const double usqr = 1.5 * (ux9s + uy9s + uz9s);
-#pragma unroll
-    for (int ip = 1; ip < 19; ip++) {
-        const double wght = ip <= 6 ? a.ww1 : a.ww2;
-        const double edtu = (double)CX[ip] * ux9 + (double)CY[ip] * uy9 + (double)CZ[ip] * uz9;
-        const double feq9 = wght * (rho9 + 3.0 * edtu + 4.5 * (edtu * edtu) - usqr);
-        const double fneq9 = f9[ip] - feq9;
-        Sxx = Sxx + fneq9 * (double)(CX[ip] * CX[ip]);
-        Syy = Syy + fneq9 * (double)(CY[ip] * CY[ip]);
-        Szz = Szz + fneq9 * (double)(CZ[ip] * CZ[ip]);
-        Sxy = Sxy + fneq9 * (double)(CX[ip] * CY[ip]);
-        Syz = Syz + fneq9 * (double)(CY[ip] * CZ[ip]);
-        Szx = Szx + fneq9 * (double)(CZ[ip] * CX[ip]);
-    }
+    // sum_i (f_i - feq_i) c_a c_b in closed form: sum_i feq_i c_a c_b =
+    // delta_ab rho/3 + u_a u_b, from the lattice sums sum w c_a c_b =
+    // delta_ab/3 and sum w c_a c_b c_c c_d = (three pairings)/9.  (The
+    // reference's loop over the 18 directions, about 250 FP64 operations a
+    // node, kept the vector ALUs busier than the memory.)
+    const double sumxy = f9[7] + f9[8] + f9[9] + f9[10], sumxz = f9[11] + f9[12] + f9[13] + f9[14];
+    const double r3 = rho9 / 3.0;
+    Sxx = (sum6 + sumxy + sumxz) - (r3 + ux9s);
+    Syy = (f9[3] + f9[4] + sumxy + sum9) - (r3 + uy9s);
+    Szz = (f9[5] + f9[6] + sumxz + sum9) - (r3 + uz9s);
+    Sxy = evlm10 - eqm10;
+    Syz = evlm11 - eqm11;
+    Szx = evlm12 - eqm12;
     const double m2 = Sxx * Sxx + Syy * Syy + Szz * Szz + 2.0 * (Sxy * Sxy + Syz * Syz + Szx * Szx);
     v[2] = m2 * (a.c15tau * a.c15tau);
     v[3] = Sxy * a.c15tau;
 }
 
-// Plane sums of dissipation_calc: block (chunk, x tile) strides over rows.
+// Plane sums of dissipation_calc, in the blocks of the statistics' plane sums.
 template <int P, int SRC>
-__global__ void __launch_bounds__(BLOCK) k_diss_partials(DissArgs a)
+__global__ void __launch_bounds__(DISS_THREADS) k_diss_partials(DissArgs a)
 {
     const uint32_t ix = blockIdx.y * blockDim.x + threadIdx.x;
-    if (ix >= a.g.lx)
-        return;
     double s[NDISS] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    const uint32_t rows = a.g.ly * a.g.lz;
-    for (uint32_t row = blockIdx.x; row < rows; row += gridDim.x) {
+    const uint32_t rows = ix < a.g.lx ? a.g.ly * a.g.lz : 0u;
+    for (uint32_t row = blockIdx.x * blockDim.y + threadIdx.y; row < rows; row += gridDim.x * blockDim.y) {
         const uint32_t n = row * a.g.lx + ix;
         if (a.solid && a.solid[n] >= 0)
             continue;
@@ -1208,10 +1227,7 @@ __global__ void __launch_bounds__(BLOCK) k_diss_partials(DissArgs a)
         s[3] += v[3];
         s[4] += 1.0;
     }
-    double *out = a.partials + (uint64_t)blockIdx.x * NDISS * a.g.lx;
-#pragma unroll
-    for (int q = 0; q < NDISS; q++)
-        out[(uint64_t)q * a.g.lx + ix] = s[q];
+    plane_write_partials(s, ix, a.g.lx, a.partials);
 }
 
 template <int P>
@@ -1447,25 +1463,35 @@ hipError_t Launch<P>::mass_partials(const SumArgs &a, uint32_t grid, hipStream_t
     return hipGetLastError();
 }
 
+// Block shape of the plane sums for nx wall-normal columns: whole waves of
+// columns, as many row lanes as `threads` holds.
+struct PlaneShape {
+    dim3 grid, blk;
+};
+static inline PlaneShape plane_shape(uint32_t nx, uint32_t rows, uint32_t chunks, uint32_t threads)
+{
+    const uint32_t bx = std::min<uint32_t>(BLOCK, (nx + 63) / 64 * 64);
+    // no row lane without a row: every chunk then has work
+    const uint32_t by = std::max<uint32_t>(1, std::min<uint32_t>(threads / bx, rows / chunks));
+    return PlaneShape{dim3(chunks, (nx + bx - 1) / bx), dim3(bx, by)};
+}
+
 template <int P>
 hipError_t Launch<P>::plane_partials(const PlaneArgs &a, int src, uint32_t chunks, hipStream_t s)
 {
-    const uint32_t bx = a.g.lx >= BLOCK ? BLOCK : ((a.g.lx + 63) / 64) * 64;
-    const dim3 grid(chunks, (a.g.lx + bx - 1) / bx), blk(bx);
+    const PlaneShape p = plane_shape(a.g.lx, a.g.ly * a.g.lz, chunks, PLANE_THREADS);
     if (src == 0)
-        hipLaunchKernelGGL((k_plane_partials<P, 0>), grid, blk, 0, s, a);
+        hipLaunchKernelGGL((k_plane_partials<P, 0>), p.grid, p.blk, 0, s, a);
     else
-        hipLaunchKernelGGL((k_plane_partials<P, 1>), grid, blk, 0, s, a);
+        hipLaunchKernelGGL((k_plane_partials<P, 1>), p.grid, p.blk, 0, s, a);
     return hipGetLastError();
 }
 
 template <int P>
 hipError_t Launch<P>::filtered_plane_partials(const PlaneArgs &a, uint32_t chunks, hipStream_t s)
 {
-    const uint32_t lxc = a.g.lx / 2;
-    const uint32_t bx = lxc >= BLOCK ? BLOCK : ((lxc + 63) / 64) * 64;
-    const dim3 grid(chunks, (lxc + bx - 1) / bx), blk(bx);
-    hipLaunchKernelGGL((k_filtered_plane_partials<P>), grid, blk, 0, s, a);
+    const PlaneShape p = plane_shape(a.g.lx, (a.g.ly / 2) * (a.g.lz / 2), chunks, PLANE_THREADS);
+    hipLaunchKernelGGL((k_filtered_plane_partials<P>), p.grid, p.blk, 0, s, a);
     return hipGetLastError();
 }
 
@@ -1482,12 +1508,11 @@ hipError_t Launch<P>::diag_partials(const DiagArgs &a, int src, uint32_t grid, h
 template <int P>
 hipError_t Launch<P>::dissipation_partials(const DissArgs &a, int src, uint32_t chunks, hipStream_t s)
 {
-    const uint32_t bx = a.g.lx >= BLOCK ? BLOCK : ((a.g.lx + 63) / 64) * 64;
-    const dim3 grid(chunks, (a.g.lx + bx - 1) / bx), blk(bx);
+    const PlaneShape p = plane_shape(a.g.lx, a.g.ly * a.g.lz, chunks, DISS_THREADS);
     if (src == 0)
-        hipLaunchKernelGGL((k_diss_partials<P, 0>), grid, blk, 0, s, a);
+        hipLaunchKernelGGL((k_diss_partials<P, 0>), p.grid, p.blk, 0, s, a);
     else
-        hipLaunchKernelGGL((k_diss_partials<P, 1>), grid, blk, 0, s, a);
+        hipLaunchKernelGGL((k_diss_partials<P, 1>), p.grid, p.blk, 0, s, a);
     return hipGetLastError();
 }
 
