@@ -170,6 +170,14 @@ constexpr double BLOCK_RING_BYTES = 225e6;
 constexpr long BLOCK_MIN_SLABS = 4;
 constexpr long BLOCK_MAX_SLABS = 32;
 
+// Pairs of steps of lattices up to this size run as single steps.  Both
+// lattices, or most of one, then stay in the last-level cache anyway, and the
+// sweep only adds launches and halo slabs.  us per step, sweep against single
+// steps: FP64 10 MB (32x64x32) 11.7 / 6.1, 53 MB 39 / 20, 156 MB 67 / 56, 184
+// MB 82 / 84, 280 MB 103 / 107-111, 478 MB 166 / 178-184; FP32 27 MB 28 / 12,
+// 140 MB 59 / 53-57, 239 MB 92 / 90-93, 295 MB 110 / 112, 359 MB 125 / 132.
+constexpr uint64_t BLOCK_MIN_LATTICE_BYTES = 160000000ull;
+
 // The sweep lbm_create chooses for a lattice of elem-byte values: axis 2 (z)
 // or 1 (y), K slabs per chunk (0: single steps only) and W rows per window
 // (0: whole slabs).  Along each axis K is the number of slabs whose ring of

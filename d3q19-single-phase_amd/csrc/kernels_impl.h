@@ -30,7 +30,8 @@ constexpr int BLOCK = 256;
 // against 68 100); 256 for the plain FP32 step (39 220-39 330 against
 // 37 990-38 800 with 512 on the 2048x1024x512 channel) and the fused closure
 // (96 registers: five 256-thread blocks per CU against two of 512, 248 against
-// 255 us per step on the 96x384x192 channel).  128 was slower.
+// 255 us per step on the 96x384x192 channel).  128 was slower.  These are the
+// largest block sizes; step_threads takes smaller ones for small grids.
 template <int P, int MODE>
 constexpr int step_block() { return ((MODE & 8) != 0 || P == 1) ? 256 : 512; }
 
@@ -201,13 +202,12 @@ __device__ __forceinline__ void node_force(const ForceSpec &s, const Geom &g, ui
     fz = in_band ? gz : fz;
 }
 
-template <int NB>
-__device__ __forceinline__ uint32_t node_index(const Geom &g)
+__device__ __forceinline__ uint32_t node_index(const Geom &g, uint32_t nb)
 {
     uint32_t blk = blockIdx.x;
     if (g.remap)
         blk = xcd_remap(blk, gridDim.x);
-    return blk * NB + threadIdx.x;
+    return blk * nb + threadIdx.x;
 }
 
 // ---------------------------------------------------------------------------
@@ -236,8 +236,7 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
     // every lane stays to the end (a lane past the lattice works on the last
     // node, a particle node on its own slots) and only active lanes store.
     constexpr bool WAVE = (MODE & 8) != 0;
-    constexpr int NB = step_block<P, MODE>();
-    const uint32_t n0 = node_index<NB>(a.g);
+    const uint32_t n0 = node_index(a.g, a.nb);
     bool active = n0 < a.g.N;
     if constexpr (!WAVE) {
         if (!active)
@@ -258,7 +257,7 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
     pull_all<P, (MODE & 32) != 0 ? 1 : ((MODE & 64) != 0 ? 2 : 0)>(src, a.g.N, b, f);
     __shared__ __attribute__((aligned(16))) _Float16 wl[WAVE ? MLP_LDS : 8];
     if constexpr (WAVE) {
-        mlp_stage(a.mlp, wl, threadIdx.x, NB);
+        mlp_stage(a.mlp, wl, threadIdx.x, a.nb);
         __syncthreads();
     }
 
@@ -1240,9 +1239,27 @@ static inline bool use_runs(const StepArgs &a, int mode)
     }
 }
 
-template <int P>
-hipError_t Launch<P>::step(const StepArgs &a, int mode, hipStream_t s)
+// Threads per block of a step over N nodes: the kernel's block size, halved
+// down to one wave while the grid has fewer blocks than the 256 CUs.  A step
+// of a small lattice lasts as long as one wave's chain of loads and
+// arithmetic, so its waves belong on as many SIMDs as there are (32x64x32 in
+// FP64: 6.1 us with 256 threads, 8.1 us with 512; 16x32x32: 4.6 us with 64
+// threads, 6.3 us with 512).  With more blocks than CUs larger ones are
+// faster: waves that share cache lines then share a CU (97x150x83: 84 us with
+// 512 threads, 93 us with 64).
+constexpr uint32_t DEVICE_CUS = 256;
+static inline uint32_t step_threads(uint64_t N, uint32_t largest)
 {
+    uint32_t nb = largest;
+    while (nb > 64 && (N + nb - 1) / nb < DEVICE_CUS)
+        nb /= 2;
+    return nb;
+}
+
+template <int P>
+hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
+{
+    StepArgs a = args;
     if constexpr (!half_storage(P)) {
         if (use_runs<P>(a, mode)) {
             const dim3 grid(nblocks<P>(a.g.N / Vec<P>::W)), blk(BLOCK);
@@ -1253,8 +1270,15 @@ hipError_t Launch<P>::step(const StepArgs &a, int mode, hipStream_t s)
             return hipGetLastError();
         }
     }
-    // one launch geometry per kernel's block size (step_block)
-    auto geo = [&](int nb) { return std::make_pair(dim3((uint32_t)((a.g.N + nb - 1) / nb)), dim3(nb)); };
+    auto launch = [&](auto kernel, uint32_t largest) {
+        a.nb = step_threads(a.g.N, largest);
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)((a.g.N + a.nb - 1) / a.nb)), dim3(a.nb), 0, s, a);
+        return hipGetLastError();
+    };
+#define STEP_CASE(MODE) \
+    case (MODE) & 31: return launch(k_step<P, MODE>, step_block<P, MODE>())
+#define CLOSURE_CASE(MODE) \
+    case (MODE) & 31: return launch(k_step_closure<P, MODE>, step_block<P, MODE>())
     if constexpr (half_storage(P) || P == 1) {
         // 32-bit pull offsets where the lattice allows them: the main loop's
         // modes in 2-byte storage (FP16 1.8-2.5 % faster, FP16C 2.7-2.9 %, on
@@ -1262,39 +1286,20 @@ hipError_t Launch<P>::step(const StepArgs &a, int mode, hipStream_t s)
         // change), and the closure modes, which are issue-bound, in FP32 and
         // 2-byte storage
         if (a.w32 == 1 && a.g.N <= w32_max_n(P)) {
-            switch (mode) {
-            case 0:
-            case 1:
-            case 4:
-            case 16:
-                if constexpr (half_storage(P)) {
-                    if (mode == 0)
-                        hipLaunchKernelGGL((k_step<P, 32>), geo(step_block<P, 32>()).first,
-                                           geo(step_block<P, 32>()).second, 0, s, a);
-                    else if (mode == 1)
-                        hipLaunchKernelGGL((k_step<P, 33>), geo(step_block<P, 33>()).first,
-                                           geo(step_block<P, 33>()).second, 0, s, a);
-                    else if (mode == 4)
-                        hipLaunchKernelGGL((k_step<P, 36>), geo(step_block<P, 36>()).first,
-                                           geo(step_block<P, 36>()).second, 0, s, a);
-                    else
-                        hipLaunchKernelGGL((k_step<P, 48>), geo(step_block<P, 48>()).first,
-                                           geo(step_block<P, 48>()).second, 0, s, a);
-                    return hipGetLastError();
+            if constexpr (half_storage(P)) {
+                switch (mode) {
+                    STEP_CASE(32);
+                    STEP_CASE(33);
+                    STEP_CASE(36);
+                    STEP_CASE(48);
+                default:
+                    break;
                 }
-                break;
-            case 8:
-                hipLaunchKernelGGL((k_step_closure<P, 40>), geo(step_block<P, 40>()).first,
-                                   geo(step_block<P, 40>()).second, 0, s, a);
-                return hipGetLastError();
-            case 12:
-                hipLaunchKernelGGL((k_step_closure<P, 44>), geo(step_block<P, 44>()).first,
-                                   geo(step_block<P, 44>()).second, 0, s, a);
-                return hipGetLastError();
-            case 24:
-                hipLaunchKernelGGL((k_step_closure<P, 56>), geo(step_block<P, 56>()).first,
-                                   geo(step_block<P, 56>()).second, 0, s, a);
-                return hipGetLastError();
+            }
+            switch (mode) {
+                CLOSURE_CASE(40);
+                CLOSURE_CASE(44);
+                CLOSURE_CASE(56);
             default:
                 break;
             }
@@ -1305,77 +1310,39 @@ hipError_t Launch<P>::step(const StepArgs &a, int mode, hipStream_t s)
         // adjacent rows only (step mode + 64)
         if (a.w32 && (a.g.N > w32_max_n(P) || a.w32 == 2) && a.g.N <= W32_ADJ_MAX_N) {
             switch (mode) {
-            case 0:
-                hipLaunchKernelGGL((k_step<P, 64>), geo(step_block<P, 64>()).first, geo(step_block<P, 64>()).second, 0,
-                                   s, a);
-                return hipGetLastError();
-            case 1:
-                hipLaunchKernelGGL((k_step<P, 65>), geo(step_block<P, 65>()).first, geo(step_block<P, 65>()).second, 0,
-                                   s, a);
-                return hipGetLastError();
-            case 4:
-                hipLaunchKernelGGL((k_step<P, 68>), geo(step_block<P, 68>()).first, geo(step_block<P, 68>()).second, 0,
-                                   s, a);
-                return hipGetLastError();
-            case 16:
-                hipLaunchKernelGGL((k_step<P, 80>), geo(step_block<P, 80>()).first, geo(step_block<P, 80>()).second, 0,
-                                   s, a);
-                return hipGetLastError();
+                STEP_CASE(64);
+                STEP_CASE(65);
+                STEP_CASE(68);
+                STEP_CASE(80);
             default:
                 break;
             }
         }
     }
+    if constexpr (P != 0) { // the closure runs in FP32 arithmetic only
+        switch (mode) {
+            CLOSURE_CASE(8);
+            CLOSURE_CASE(12);
+            CLOSURE_CASE(24);
+        default:
+            break;
+        }
+    }
     switch (mode) {
-    case 0:
-        hipLaunchKernelGGL((k_step<P, 0>), geo(step_block<P, 0>()).first, geo(step_block<P, 0>()).second, 0, s, a);
-        break;
-    case 1:
-        hipLaunchKernelGGL((k_step<P, 1>), geo(step_block<P, 1>()).first, geo(step_block<P, 1>()).second, 0, s, a);
-        break;
-    case 2:
-        hipLaunchKernelGGL((k_step<P, 2>), geo(step_block<P, 2>()).first, geo(step_block<P, 2>()).second, 0, s, a);
-        break;
-    case 4:
-        hipLaunchKernelGGL((k_step<P, 4>), geo(step_block<P, 4>()).first, geo(step_block<P, 4>()).second, 0, s, a);
-        break;
-    case 5:
-        hipLaunchKernelGGL((k_step<P, 5>), geo(step_block<P, 5>()).first, geo(step_block<P, 5>()).second, 0, s, a);
-        break;
-    case 6:
-        hipLaunchKernelGGL((k_step<P, 6>), geo(step_block<P, 6>()).first, geo(step_block<P, 6>()).second, 0, s, a);
-        break;
-    case 8:
-        if constexpr (P == 0)
-            return hipErrorInvalidValue;
-        else
-            hipLaunchKernelGGL((k_step_closure<P, 8>), geo(step_block<P, 8>()).first, geo(step_block<P, 8>()).second, 0, s, a);
-        break;
-    case 12:
-        if constexpr (P == 0)
-            return hipErrorInvalidValue;
-        else
-            hipLaunchKernelGGL((k_step_closure<P, 12>), geo(step_block<P, 12>()).first, geo(step_block<P, 12>()).second, 0, s, a);
-        break;
-    case 16:
-        hipLaunchKernelGGL((k_step<P, 16>), geo(step_block<P, 16>()).first, geo(step_block<P, 16>()).second, 0, s, a);
-        break;
-    case 17:
-        hipLaunchKernelGGL((k_step<P, 17>), geo(step_block<P, 17>()).first, geo(step_block<P, 17>()).second, 0, s, a);
-        break;
-    case 18:
-        hipLaunchKernelGGL((k_step<P, 18>), geo(step_block<P, 18>()).first, geo(step_block<P, 18>()).second, 0, s, a);
-        break;
-    case 24:
-        if constexpr (P == 0)
-            return hipErrorInvalidValue;
-        else
-            hipLaunchKernelGGL((k_step_closure<P, 24>), geo(step_block<P, 24>()).first, geo(step_block<P, 24>()).second, 0, s, a);
-        break;
+        STEP_CASE(0);
+        STEP_CASE(1);
+        STEP_CASE(2);
+        STEP_CASE(4);
+        STEP_CASE(5);
+        STEP_CASE(6);
+        STEP_CASE(16);
+        STEP_CASE(17);
+        STEP_CASE(18);
     default:
         return hipErrorInvalidValue;
     }
-    return hipGetLastError();
+#undef STEP_CASE
+#undef CLOSURE_CASE
 }
 
 template <int P>

@@ -108,6 +108,7 @@ struct lbm_channel {
     uint32_t bK;        // two-step blocked sweep: slabs per chunk (0 = single steps only)
     int baxis;          // its sweep axis: 2 = z (slabs lx*ly), 1 = y (slabs lx*lz)
     uint32_t bW;        // rows per window of its slabs (0 = whole slabs)
+    bool bskip;         // the lattice is small: pairs run as single steps although bK > 0
     int bforced;        // lbm_run_forcingp also pairs steps whose force varies over the nodes
     void *bring, *bhead; // its slab ring and head buffer (allocated on first use)
     bool ave_pending;   // lbm_run_particles: avedensity due once the next bounce-back has run
@@ -608,6 +609,10 @@ int lbm_create(const lbm_config *cfg, lbm_channel **out)
         h->baxis = bc.axis;
         h->bK = bc.K;
         h->bW = bc.W;
+        // small lattices are faster in single steps; setting the sweep's
+        // variables asks for the sweep at any size
+        h->bskip = N * 19 * h->elem <= BLOCK_MIN_LATTICE_BYTES && !getenv("LBM_BLOCK_AXIS") &&
+                   !getenv("LBM_BLOCK_PLANES") && !getenv("LBM_BLOCK_ROWS");
         // LBM_BLOCK_FORCED=1: pairs under a force evaluated per node too.
         // Off by default: on the 192x768x384 channel such pairs took 3.33 ms
         // per FP64 step against 3.10 ms for single steps (the per-node force
@@ -1130,8 +1135,8 @@ int lbm_avedensity(lbm_channel *h, double *rhomean)
 // density offset, one uniform force, no particles, no closure.
 static bool block_ready(const lbm_channel *h)
 {
-    return h->bK > 0 && h->ms == FROM_CUR && h->rho_off == 0.0 && !h->part && !h->mlp && h->fc.tab == nullptr &&
-           same_force(h->fm, h->fc);
+    return h->bK > 0 && !h->bskip && h->ms == FROM_CUR && h->rho_off == 0.0 && !h->part && !h->mlp &&
+           h->fc.tab == nullptr && same_force(h->fm, h->fc);
 }
 
 // The force of one step of a pair: collision force fc, fields formed with fm
@@ -1218,7 +1223,8 @@ int lbm_run_forcingp(lbm_channel *h, int istep0, int nsteps, int npforcing, doub
         // no density offset, no particles or closure, and one uniform force
         // (or, with bforced, any forces, evaluated per node)
         bool paired = false;
-        if (nsteps - s >= 2 && h->bK > 0 && h->ms == FROM_CUR && h->rho_off == 0.0 && !h->part && !h->mlp) {
+        if (nsteps - s >= 2 && h->bK > 0 && !h->bskip && h->ms == FROM_CUR && h->rho_off == 0.0 && !h->part &&
+            !h->mlp) {
             const ForceSpec fc0 = h->fc, fm0 = h->fm;
             rc = main_loop_force(h, istep + 1, npforcing, force_in_y, fy_forcing);
             if (rc)
