@@ -62,15 +62,21 @@ inline uint32_t block_ring_rows(const Geom &g, int axis, uint32_t W)
     return block_windowed(g, axis, W) ? W + 2 : block_geom(g, axis).nr;
 }
 
-// Ring slots and buffer sizes in elements (slabs of lx * ring rows nodes).
+// Ring slots, elements of one population of a ring slab (lx * ring rows nodes,
+// rounded up to whole waves so that slabs start on cache lines) and buffer
+// sizes in elements.
 inline uint32_t block_ring_slots(uint32_t K) { return K + 2; }
+inline uint64_t block_ring_slab(const Geom &g, int axis, uint32_t W)
+{
+    return slab_padded(g.lx * block_ring_rows(g, axis, W));
+}
 inline uint64_t block_ring_elems(const Geom &g, int axis, uint32_t K, uint32_t W = 0)
 {
-    return 19ull * block_ring_slots(K) * g.lx * block_ring_rows(g, axis, W);
+    return 19ull * block_ring_slots(K) * block_ring_slab(g, axis, W);
 }
 inline uint64_t block_head_elems(const Geom &g, int axis, uint32_t W = 0)
 {
-    return 19ull * 2 * g.lx * block_ring_rows(g, axis, W);
+    return 19ull * 2 * block_ring_slab(g, axis, W);
 }
 
 // The force of one of the two steps of a pair: rates with the uniform force
@@ -83,19 +89,20 @@ struct StepForce {
 };
 
 // Launch list of one pair: step t with force f0, step t+1 with force f1,
-// whole slabs (W = 0) or row windows of W rows.
+// whole slabs (W = 0) or row windows of W rows; the lattices' population
+// stride (0: the node count).
 inline std::vector<BlockArgs> block_schedule(const Geom &g, int axis, const StepForce &f0, const StepForce &f1,
                                              uint32_t K, uint32_t W, void *lat_in, void *lat_out, void *ring,
-                                             void *head)
+                                             void *head, uint64_t lat_stride = 0)
 {
+    const uint64_t ls = lat_stride ? lat_stride : g.N;
     const BlockGeom bg = block_geom(g, axis);
     const uint32_t ns = bg.ns, nr = bg.nr, slots = block_ring_slots(K);
     const bool win = block_windowed(g, axis, W);
-    const uint32_t rr = block_ring_rows(g, axis, W);
-    const uint64_t rslab = (uint64_t)g.lx * rr; // nodes of a ring slab
-    const PlaneStore full_in = {lat_in, g.N, ns, make_fastdiv(ns), bg.lat_slab_stride, bg.lat_row_stride, nullptr, 0,
+    const uint64_t rslab = block_ring_slab(g, axis, W);
+    const PlaneStore full_in = {lat_in, ls, ns, make_fastdiv(ns), bg.lat_slab_stride, bg.lat_row_stride, nullptr, 0,
                                 0, 0};
-    const PlaneStore full_out = {lat_out, g.N, ns, make_fastdiv(ns), bg.lat_slab_stride, bg.lat_row_stride, nullptr, 0,
+    const PlaneStore full_out = {lat_out, ls, ns, make_fastdiv(ns), bg.lat_slab_stride, bg.lat_row_stride, nullptr, 0,
                                  0, 0};
     const PlaneStore ring_only = {ring, slots * rslab, slots, make_fastdiv(slots), rslab, g.lx, nullptr, 0, 0, 0};
     PlaneStore ring_head = ring_only;
@@ -173,10 +180,11 @@ constexpr long BLOCK_MAX_SLABS = 32;
 // Pairs of steps of lattices up to this size run as single steps.  Both
 // lattices, or most of one, then stay in the last-level cache anyway, and the
 // sweep only adds launches and halo slabs.  us per step, sweep against single
-// steps: FP64 10 MB (32x64x32) 11.7 / 6.1, 53 MB 39 / 20, 156 MB 67 / 56, 184
-// MB 82 / 84, 280 MB 103 / 107-111, 478 MB 166 / 178-184; FP32 27 MB 28 / 12,
-// 140 MB 59 / 53-57, 239 MB 92 / 90-93, 295 MB 110 / 112, 359 MB 125 / 132.
-constexpr uint64_t BLOCK_MIN_LATTICE_BYTES = 160000000ull;
+// steps: FP64 10 MB (32x64x32) 11.7 / 6.1, 53 MB 40 / 24, 184 MB (97x150x83)
+// 81 / 74, 280 MB 106 / 107, 342 MB 126 / 129, 478 MB 172 / 189; FP32 27 MB
+// 28 / 13, 140 MB 60 / 56, 239 MB 93 / 90-101, 294 MB 111 / 107, 538 MB 185 /
+// 194.
+constexpr uint64_t BLOCK_MIN_LATTICE_BYTES = 300000000ull;
 
 // The sweep lbm_create chooses for a lattice of elem-byte values: axis 2 (z)
 // or 1 (y), K slabs per chunk (0: single steps only) and W rows per window

@@ -55,7 +55,8 @@ __device__ __forceinline__ const typename Prec<P>::S *elem(const typename Prec<P
     return elem<P>(const_cast<typename Prec<P>::S *>(row), node);
 }
 
-// F_I(x): streamed population of direction I at node x.  The bounce-back
+// F_I(x): streamed population of direction I at node x; N is the population
+// stride Geom::S here and in the functions below.  The bounce-back
 // choice is made with masks, not branches, so every load issues back to back.
 // Loads are plain (cached): the +-x shifted reads of neighbouring waves share
 // cache lines.  W32 = 1 (N <= w32_max_n(P)): a pull with c_x != 0 addresses
@@ -88,7 +89,7 @@ __device__ __forceinline__ typename Prec<P>::T pull(const typename Prec<P>::S *_
             constexpr int M = I < OPP[I] ? I : OPP[I];
             uint64_t row_m = (uint64_t)M * N;
             uint32_t d_i = (uint32_t)(I - M) * (uint32_t)N, d_o = (uint32_t)(OPP[I] - M) * (uint32_t)N;
-            // wave-uniform (N is the kernel argument Geom::N), kept in scalar
+            // wave-uniform (N is the kernel argument Geom::S), kept in scalar
             // registers as below
             __asm__("" : "+s"(row_m));
             __asm__("" : "+s"(d_i));
@@ -105,7 +106,7 @@ __device__ __forceinline__ typename Prec<P>::T pull(const typename Prec<P>::S *_
             // of two scalar row offsets into a per-lane 64-bit multiply of a
             // selected index (quarter-rate; FP16 storage is issue-bound).
             // The "s" operands require N to be wave-uniform: every caller
-            // passes the kernel argument Geom::N.
+            // passes the kernel argument Geom::S.
             __asm__("" : "+s"(row_i));
             __asm__("" : "+s"(row_o));
             return Prec<P>::template to_T<I>(*elem<P>(L + (w ? row_o : row_i), node));
@@ -254,7 +255,7 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
     // the 19 loads issue first; the closure's weights are staged while they
     // are in flight
     T f[19];
-    pull_all<P, (MODE & 32) != 0 ? 1 : ((MODE & 64) != 0 ? 2 : 0)>(src, a.g.N, b, f);
+    pull_all<P, (MODE & 32) != 0 ? 1 : ((MODE & 64) != 0 ? 2 : 0)>(src, a.g.S, b, f);
     __shared__ __attribute__((aligned(16))) _Float16 wl[WAVE ? MLP_LDS : 8];
     if constexpr (WAVE) {
         mlp_stage(a.mlp, wl, threadIdx.x, a.nb);
@@ -333,7 +334,7 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
         if (!active)
             return;
     }
-    store_all<P>(dst, a.g.N, n, f);
+    store_all<P>(dst, a.g.S, n, f);
 }
 
 template <int P, int MODE>
@@ -484,7 +485,7 @@ __global__ void __launch_bounds__(BLOCK) k_closure_eval(StepArgs a, uint64_t n_b
     }
     const Nbr b = make_nbr(n, a.g);
     T f[19];
-    pull_all<P>((const S *)a.src, a.g.N, b, f);
+    pull_all<P>((const S *)a.src, a.g.S, b, f);
     Rates<T> r = rates_as<T>(a.r);
     uint32_t ix, iy, iz;
     node_coords(n, a.g, ix, iy, iz);
@@ -637,7 +638,7 @@ __global__ void __launch_bounds__(BLOCK) k_step_run(StepArgs a)
     const bool last_lane = (lane == 63u) || (t + 1 >= nruns);
 
     T F[VW][19];
-    pull_run_all<P>((const S *)a.src, a.g.N, b, whi_last, active, first_lane, last_lane, F,
+    pull_run_all<P>((const S *)a.src, a.g.S, b, whi_last, active, first_lane, last_lane, F,
                     std::make_integer_sequence<int, 19>{});
     if (!active)
         return;
@@ -660,7 +661,7 @@ __global__ void __launch_bounds__(BLOCK) k_step_run(StepArgs a)
             mrt_collide_delta(F[k], rho9, ux9, uy9, uz9, drho, T(0), T(0), T(0), r);
         }
     }
-    store_run_all<P>((S *)a.dst, a.g.N, n0, F, std::make_integer_sequence<int, 19>{});
+    store_run_all<P>((S *)a.dst, a.g.S, n0, F, std::make_integer_sequence<int, 19>{});
 }
 
 // macrovar / rhoupdat / materialisation of the fields of lattice L.
@@ -676,7 +677,7 @@ __global__ void __launch_bounds__(BLOCK) k_macro(MacroArgs a)
     if (n < a.g.N) {
         const Nbr b = make_nbr(n, a.g);
         T f[19];
-        pull_all<P>((const S *)a.L, a.g.N, b, f);
+        pull_all<P>((const S *)a.L, a.g.S, b, f);
         T rho9, ux9, uy9, uz9;
         macro_sums(f, rho9, ux9, uy9, uz9);
         if constexpr (WHAT == 0) {
@@ -730,7 +731,7 @@ __global__ void __launch_bounds__(BLOCK) k_gather(CopyArgs a)
     if (base + threadIdx.x < a.count) {
         const Nbr b = make_nbr((uint32_t)n, a.g);
         T f[19];
-        pull_all<P>((const S *)a.L, a.g.N, b, f);
+        pull_all<P>((const S *)a.L, a.g.S, b, f);
 #pragma unroll
         for (int i = 0; i < 19; i++)
             tile[i][threadIdx.x] = (double)f[i];
@@ -763,7 +764,7 @@ __global__ void __launch_bounds__(BLOCK) k_scatter(CopyArgs a)
 #pragma unroll
         for (int i = 0; i < 19; i++)
             f[i] = (T)tile[i][threadIdx.x];
-        scatter_all<P>((S *)a.L, a.g.N, b, f);
+        scatter_all<P>((S *)a.L, a.g.S, b, f);
     }
 }
 
@@ -795,7 +796,7 @@ __global__ void __launch_bounds__(BLOCK) k_initpop(InitArgs a)
 #undef D3Q19_EQ
     a.rho[n] = 0.0;
     const Nbr b = make_nbr(n, a.g);
-    scatter_all<P>((S *)a.L, a.g.N, b, f);
+    scatter_all<P>((S *)a.L, a.g.S, b, f);
 }
 
 // Deterministic block sum: each thread's partial, reduced in a fixed tree.
@@ -834,7 +835,7 @@ __global__ void __launch_bounds__(BLOCK) k_rho_partials(SumArgs a)
         } else {
             const Nbr b = make_nbr((uint32_t)n, a.g);
             T f[19];
-            pull_all<P>((const S *)a.L, a.g.N, b, f);
+            pull_all<P>((const S *)a.L, a.g.S, b, f);
             T rho9, ux9, uy9, uz9;
             macro_sums(f, rho9, ux9, uy9, uz9);
             acc += (double)rho9;
@@ -866,7 +867,7 @@ __global__ void __launch_bounds__(BLOCK) k_mass_partials(SumArgs a)
     double acc = 0.0;
     for (uint64_t n = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; n < a.g.N; n += (uint64_t)gridDim.x * BLOCK)
         if (!a.solid || a.solid[n] < 0)
-            acc += node_mass<P>((const S *)a.L, a.g.N, n, std::make_integer_sequence<int, 19>{});
+            acc += node_mass<P>((const S *)a.L, a.g.S, n, std::make_integer_sequence<int, 19>{});
     const double s = block_sum(acc);
     if (threadIdx.x == 0)
         a.partials[blockIdx.x] = s;
@@ -953,7 +954,7 @@ __global__ void __launch_bounds__(PLANE_THREADS) k_plane_partials(PlaneArgs a)
         } else {
             const Nbr b = make_nbr(n, a.g);
             T f[19];
-            pull_all<P>((const S *)a.L, a.g.N, b, f);
+            pull_all<P>((const S *)a.L, a.g.S, b, f);
             T rho9, ux9, uy9, uz9;
             macro_sums(f, rho9, ux9, uy9, uz9);
             uint32_t cx, cy, cz;
@@ -997,7 +998,7 @@ __global__ void __launch_bounds__(PLANE_THREADS) k_filtered_plane_partials(Plane
                 const uint32_t n = ix + a.g.lx * ((2 * cy + dy) + a.g.ly * (2 * cz + dz));
                 const Nbr b = make_nbr(n, a.g);
                 T f[19];
-                pull_all<P>((const S *)a.L, a.g.N, b, f);
+                pull_all<P>((const S *)a.L, a.g.S, b, f);
                 T rho9, ux9, uy9, uz9;
                 macro_sums(f, rho9, ux9, uy9, uz9);
                 double fx, fy, fz;
@@ -1044,7 +1045,7 @@ __device__ __forceinline__ void node_fields(const void *L, const double *rho_a, 
         if (f9) {
             const Nbr b = make_nbr(n, g);
             T f[19];
-            pull_all<P>((const S *)L, g.N, b, f);
+            pull_all<P>((const S *)L, g.S, b, f);
 #pragma unroll
             for (int i = 0; i < 19; i++)
                 f9[i] = (double)f[i];
@@ -1052,7 +1053,7 @@ __device__ __forceinline__ void node_fields(const void *L, const double *rho_a, 
     } else {
         const Nbr b = make_nbr(n, g);
         T f[19];
-        pull_all<P>((const S *)L, g.N, b, f);
+        pull_all<P>((const S *)L, g.S, b, f);
         T rho9, ux9, uy9, uz9;
         macro_sums(f, rho9, ux9, uy9, uz9);
         uint32_t cx, cy, cz;
@@ -1285,7 +1286,7 @@ hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
         // the 192x768x384 channel; FP32's memory-bound step measured no
         // change), and the closure modes, which are issue-bound, in FP32 and
         // 2-byte storage
-        if (a.w32 == 1 && a.g.N <= w32_max_n(P)) {
+        if (a.w32 == 1 && a.g.S <= w32_max_n(P)) {
             if constexpr (half_storage(P)) {
                 switch (mode) {
                     STEP_CASE(32);
@@ -1308,7 +1309,7 @@ hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
     if constexpr (half_storage(P)) {
         // above 2^29 nodes (the 2048x1024x512 channel), the pulls between
         // adjacent rows only (step mode + 64)
-        if (a.w32 && (a.g.N > w32_max_n(P) || a.w32 == 2) && a.g.N <= W32_ADJ_MAX_N) {
+        if (a.w32 && (a.g.S > w32_max_n(P) || a.w32 == 2) && a.g.S <= W32_ADJ_MAX_N) {
             switch (mode) {
                 STEP_CASE(64);
                 STEP_CASE(65);

@@ -569,6 +569,7 @@ int lbm_create(const lbm_config *cfg, lbm_channel **out)
     h->g.lz = c.lz;
     h->g.plane = (uint32_t)c.lx * c.ly;
     h->g.N = N;
+    h->g.S = padded_stride(N, h->elem);
     h->g.dlx = make_fastdiv(c.lx);
     h->g.dly = make_fastdiv(c.ly);
     h->g.remap = 0;
@@ -637,7 +638,7 @@ int lbm_create(const lbm_config *cfg, lbm_channel **out)
     hipError_t e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
     if (e != hipSuccess)
         return cleanup(fail(LBM_ERR_HIP, "hipStreamCreate failed: %s", hipGetErrorString(e)));
-    const size_t lat_bytes = (size_t)N * 19 * h->elem;
+    const size_t lat_bytes = (size_t)h->g.S * 19 * h->elem;
     for (int k = 0; k < 2; k++) {
         e = hipMalloc(&h->lat[k], lat_bytes);
         if (e != hipSuccess)
@@ -1175,7 +1176,7 @@ static int run_pair_with(lbm_channel *h, const StepForce &f0, const StepForce &f
     }
     const auto launches =
         block_schedule(h->g, h->baxis, f0, f1, h->bK, h->bW, h->lat[h->cur], h->lat[1 - h->cur], h->bring,
-                       h->bhead);
+                       h->bhead, h->g.S);
     for (const BlockArgs &a : launches) {
         int rc = dispatch_err(PREC_CALL(h, step_planes, a, h->baxis, h->stream), "collision (blocked sweep)");
         if (rc)
@@ -1737,7 +1738,7 @@ int lbm_device_bytes(lbm_channel *h, size_t *bytes)
 {
     if (!h || !bytes)
         return fail(LBM_ERR_ARG, "lbm_device_bytes: null argument");
-    size_t b = 2 * (size_t)h->g.N * 19 * h->elem;
+    size_t b = 2 * (size_t)h->g.S * 19 * h->elem;
     if (h->mac[0])
         b += 4 * (size_t)h->g.N * sizeof(double);
     if (h->stage)
@@ -1772,11 +1773,11 @@ int lbm_block_rows(lbm_channel *h, int *rows)
 // population-major (out[i*count + k] = P_i(n0 + k)).
 static int download_post_range(lbm_channel *h, uint64_t n0, uint64_t count, double *out)
 {
-    const uint64_t N = h->g.N;
+    const uint64_t S = h->g.S;
     const unsigned char *L = (const unsigned char *)h->lat[h->cur];
     if (h->prec == LBM_FP64) {
         for (int i = 0; i < 19; i++)
-            HIP_TRY(hipMemcpyAsync(out + (size_t)i * count, L + ((size_t)i * N + n0) * sizeof(double),
+            HIP_TRY(hipMemcpyAsync(out + (size_t)i * count, L + ((size_t)i * S + n0) * sizeof(double),
                                    count * sizeof(double), hipMemcpyDeviceToHost, h->stream));
         HIP_TRY(hipStreamSynchronize(h->stream));
         return LBM_OK;
@@ -1784,7 +1785,7 @@ static int download_post_range(lbm_channel *h, uint64_t n0, uint64_t count, doub
     // FP32/FP16/FP16C: widen on the host, population by population
     std::vector<unsigned char> buf(count * h->elem);
     for (int i = 0; i < 19; i++) {
-        HIP_TRY(hipMemcpyAsync(buf.data(), L + ((size_t)i * N + n0) * h->elem, count * h->elem,
+        HIP_TRY(hipMemcpyAsync(buf.data(), L + ((size_t)i * S + n0) * h->elem, count * h->elem,
                                hipMemcpyDeviceToHost, h->stream));
         HIP_TRY(hipStreamSynchronize(h->stream));
         double *o = out + (size_t)i * count;

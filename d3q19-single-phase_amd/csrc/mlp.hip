@@ -46,7 +46,7 @@ __global__ void __launch_bounds__(256) k_filter(FilterArgs a)
                 const uint32_t n = (2 * cx + dx) + a.gf.lx * ((2 * cy + dy) + a.gf.ly * (2 * cz + dz));
                 const Nbr b = make_nbr(n, a.gf);
                 T f[19];
-                pull_all<P>((const S *)a.L, a.gf.N, b, f);
+                pull_all<P>((const S *)a.L, a.gf.S, b, f);
                 T rho9, ux9, uy9, uz9;
                 macro_sums(f, rho9, ux9, uy9, uz9);
                 const double ux = (double)ux9 + 0.5 * a.fx, uy = (double)uy9 + 0.5 * a.fy,

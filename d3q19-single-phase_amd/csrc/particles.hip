@@ -342,7 +342,7 @@ __global__ void __launch_bounds__(PBLOCK) k_p_ibb(PartGeom pg, PartState ps, voi
     const int p = blockIdx.y;
     const int nl = ps.link_count[p];
     S *L = (S *)Lv;
-    const uint64_t N = pg.g.N;
+    const uint64_t N = pg.g.S; // population stride
     for (int k = blockIdx.x * PBLOCK + threadIdx.x; k < nl; k += gridDim.x * PBLOCK)
         ibb_link<P>(pg, ps, L, N, p, k);
 }
@@ -580,7 +580,7 @@ __global__ void __launch_bounds__(64) k_p_refill(PartGeom pg, PartState ps, void
 {
     using S = typename Prec<P>::S;
     S *L = (S *)Lv;
-    const uint64_t N = pg.g.N;
+    const uint64_t N = pg.g.S; // population stride
     const int p = blockIdx.y;
     const int nf = ps.fill_count[p];
     const int l = threadIdx.x;
