@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "blocked.h"
+#include "hostcopy.h"
 #include "kernels.h"
 #include "lbm.h"
 #include "particles.h"
@@ -58,7 +59,7 @@ enum MacroState { FROM_CUR = 0, FROM_PREV = 1, ARRAYS = 2 };
 constexpr uint32_t RED_BLOCKS = 2048;   // partial sums per reduction
 constexpr uint32_t DIAG_BLOCKS = 1024;  // partials per quantity of diag
 constexpr uint32_t PLANE_CHUNKS = 512;  // row chunks for plane sums
-constexpr uint64_t COPY_NODES = 1u << 20; // nodes per upload/download chunk
+constexpr size_t STAGE_BYTES = HOST_WORKERS * HOST_DEPTH * HOST_SLICE; // device side of the copy slices
 
 // Scratch of lbm_mass_sum_noalloc: the per-block partial sums of the mass
 // reduction, 16 KiB per GPU, held until the process ends.  Host code never passes `scratch` itself
@@ -96,7 +97,7 @@ struct lbm_channel {
     long long stat_n;
     double *fstat_acc;  // NPLANE*(lx/2) running sums of the box-filtered fields (allocated on first use)
     long long fstat_n;
-    double *stage;      // COPY_NODES*19 doubles
+    char *stage;        // STAGE_BYTES: one device slice for every slot of the host copies
     hipEvent_t ev[2];
     struct Part *part;  // rigid particles (nullptr without)
     hipStream_t pstream; // lbm_run_particles: the force sums and beads_move beside the collision
@@ -561,6 +562,7 @@ int lbm_create(const lbm_config *cfg, lbm_channel **out)
 
     lbm_channel *h = new lbm_channel();
     memset(h, 0, sizeof(*h));
+    host_pool().retain();
     h->cfg = c;
     h->prec = c.precision;
     h->elem = c.precision == LBM_FP64 ? 8 : (c.precision == LBM_FP32 ? 4 : 2);
@@ -604,7 +606,7 @@ int lbm_create(const lbm_config *cfg, lbm_channel **out)
             block_choice(h->g, h->elem, h->elem != 2, BLOCK_RING_BYTES, BLOCK_MIN_SLABS, getenv("LBM_BLOCK_AXIS"),
                          getenv("LBM_BLOCK_PLANES"), getenv("LBM_BLOCK_ROWS"));
         if (bc.bad) {
-            delete h;
+            (void)lbm_destroy(h);
             return fail(LBM_ERR_ARG, "lbm_create: invalid value of %s", bc.bad);
         }
         h->baxis = bc.axis;
@@ -623,7 +625,7 @@ int lbm_create(const lbm_config *cfg, lbm_channel **out)
         // LBM_DEFER=0: collision_MRT launches at once (no per-call pairing)
         const char *kd = getenv("LBM_DEFER");
         if (kd && strcmp(kd, "0") != 0 && strcmp(kd, "1") != 0) {
-            delete h;
+            (void)lbm_destroy(h);
             return fail(LBM_ERR_ARG, "lbm_create: invalid value of LBM_DEFER (0 or 1)");
         }
         h->defer = (kd && strcmp(kd, "0") == 0) ? 0 : 1;
@@ -718,6 +720,7 @@ int lbm_destroy(lbm_channel *h)
         (void)hipEventDestroy(h->ev[1]);
     if (h->stream)
         (void)hipStreamDestroy(h->stream);
+    host_pool().release();
     delete h;
     return LBM_OK;
 }
@@ -767,40 +770,137 @@ static int ensure_stage(lbm_channel *h)
 {
     if (h->stage)
         return LBM_OK;
-    hipError_t e = hipMalloc((void **)&h->stage, COPY_NODES * 19 * sizeof(double));
+    hipError_t e = hipMalloc((void **)&h->stage, STAGE_BYTES);
     if (e != hipSuccess)
         return fail(LBM_ERR_NOMEM, "hipMalloc of the copy staging buffer failed: %s", hipGetErrorString(e));
     return LBM_OK;
 }
+
+extern "C++" {
+namespace {
+
+// Nodes [0, N) in slices of at most slice_bytes of node_bytes each.
+struct NodeSlices {
+    uint64_t N, per;
+    size_t node_bytes;
+    NodeSlices(uint64_t n, size_t nb, size_t slice_bytes) : N(n), per(slice_bytes / nb / 256 * 256), node_bytes(nb) {}
+    size_t count() const { return (size_t)((N + per - 1) / per); }
+    uint64_t first(size_t k) const { return k * per; }
+    uint64_t nodes(size_t k) const { return std::min<uint64_t>(per, N - k * per); }
+    size_t bytes(size_t k) const { return (size_t)nodes(k) * node_bytes; }
+};
+
+// Per-node values made on the device slice by slice (launch(first, nodes,
+// device slice)) into the host array out.
+template <class Launch>
+int nodes_to_host(lbm_channel *h, void *out, size_t node_bytes, const char *what, Launch launch)
+{
+    const int rc = ensure_stage(h);
+    if (rc)
+        return rc;
+    char *const host = (char *)out;
+    const hipStream_t s = h->stream;
+    HIP_TRY(hipStreamSynchronize(s));
+    HostPool &pool = host_pool();
+    std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
+    hipError_t e = hipSuccess;
+    if (h->g.N * node_bytes >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device)) {
+        const NodeSlices sl(h->g.N, node_bytes, HOST_SLICE);
+        e = host_slices_out(
+            pool, h->cfg.device, s, sl.count(), host_workers(h->g.N * node_bytes),
+            [&](size_t k, int slot, char *pinned) {
+                char *dev = h->stage + slot * HOST_SLICE;
+                const hipError_t le = launch(sl.first(k), sl.nodes(k), dev);
+                return le != hipSuccess ? le : hipMemcpyAsync(pinned, dev, sl.bytes(k), hipMemcpyDeviceToHost, s);
+            },
+            [&](size_t k, const char *pinned) { memcpy(host + sl.first(k) * node_bytes, pinned, sl.bytes(k)); });
+    } else {
+        const NodeSlices sl(h->g.N, node_bytes, STAGE_BYTES);
+        for (size_t k = 0; k < sl.count() && e == hipSuccess; k++) {
+            e = launch(sl.first(k), sl.nodes(k), h->stage);
+            if (e == hipSuccess)
+                e = hipMemcpyAsync(host + sl.first(k) * node_bytes, h->stage, sl.bytes(k), hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess)
+                e = hipStreamSynchronize(s);
+        }
+    }
+    if (e != hipSuccess)
+        return fail(LBM_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
+    return LBM_OK;
+}
+
+// The host array `in` to the device slice by slice, launch consuming each.
+template <class Launch>
+int nodes_from_host(lbm_channel *h, const void *in, size_t node_bytes, const char *what, Launch launch)
+{
+    const int rc = ensure_stage(h);
+    if (rc)
+        return rc;
+    const char *const host = (const char *)in;
+    const hipStream_t s = h->stream;
+    HIP_TRY(hipStreamSynchronize(s));
+    HostPool &pool = host_pool();
+    std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
+    hipError_t e = hipSuccess;
+    if (h->g.N * node_bytes >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device)) {
+        const NodeSlices sl(h->g.N, node_bytes, HOST_SLICE);
+        e = host_slices_in(
+            pool, h->cfg.device, s, sl.count(), host_workers(h->g.N * node_bytes),
+            [&](size_t k, char *pinned) { memcpy(pinned, host + sl.first(k) * node_bytes, sl.bytes(k)); },
+            [&](size_t k, int slot, const char *pinned) {
+                char *dev = h->stage + slot * HOST_SLICE;
+                const hipError_t ce = hipMemcpyAsync(dev, pinned, sl.bytes(k), hipMemcpyHostToDevice, s);
+                return ce != hipSuccess ? ce : launch(sl.first(k), sl.nodes(k), dev);
+            });
+    } else {
+        const NodeSlices sl(h->g.N, node_bytes, STAGE_BYTES);
+        for (size_t k = 0; k < sl.count() && e == hipSuccess; k++) {
+            e = hipMemcpyAsync(h->stage, host + sl.first(k) * node_bytes, sl.bytes(k), hipMemcpyHostToDevice, s);
+            if (e == hipSuccess)
+                e = launch(sl.first(k), sl.nodes(k), h->stage);
+        }
+        if (e == hipSuccess)
+            e = hipStreamSynchronize(s);
+    }
+    if (e != hipSuccess)
+        return fail(LBM_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
+    return LBM_OK;
+}
+
+// Whole arrays between host and device; null host pointers are skipped.
+int copy_parts(lbm_channel *h, const HostPart *parts, int n, bool down, const char *what)
+{
+    const hipError_t e = host_copy(h->cfg.device, h->stream, parts, n, down);
+    if (e != hipSuccess)
+        return fail(LBM_ERR_HIP, "%s: copy failed: %s", what, hipGetErrorString(e));
+    return LBM_OK;
+}
+
+} // namespace
+} // extern "C++"
 
 int lbm_upload_f(lbm_channel *h, const double *f)
 {
     CHECK_H(h);
     if (!f)
         return fail(LBM_ERR_ARG, "lbm_upload_f: null f");
-    int rc = ensure_stage(h);
-    if (rc)
-        return rc;
     // the reference's arrays keep their values when f is replaced
     if (!h->fresh && h->ms != ARRAYS) {
-        rc = materialize(h);
+        const int rc = materialize(h);
         if (rc)
             return rc;
     }
-    for (uint64_t n0 = 0; n0 < h->g.N; n0 += COPY_NODES) {
-        const uint64_t cnt = std::min<uint64_t>(COPY_NODES, h->g.N - n0);
-        HIP_TRY(hipMemcpyAsync(h->stage, f + n0 * 19, cnt * 19 * sizeof(double), hipMemcpyHostToDevice, h->stream));
+    const int rc = nodes_from_host(h, f, 19 * sizeof(double), "lbm_upload_f", [h](uint64_t n0, uint64_t cnt, char *dev) {
         CopyArgs a;
         a.g = h->g;
         a.L = h->lat[h->cur];
-        a.aos = h->stage;
+        a.aos = (double *)dev;
         a.n0 = n0;
         a.count = cnt;
-        rc = dispatch_err(PREC_CALL(h, scatter, a, h->stream), "upload scatter");
-        if (rc)
-            return rc;
-    }
-    HIP_TRY(hipStreamSynchronize(h->stream));
+        return PREC_CALL(h, scatter, a, h->stream);
+    });
+    if (rc)
+        return rc;
     h->have_prev = false;
     return LBM_OK;
 }
@@ -810,24 +910,15 @@ int lbm_download_f(lbm_channel *h, double *f)
     CHECK_H(h);
     if (!f)
         return fail(LBM_ERR_ARG, "lbm_download_f: null f");
-    int rc = ensure_stage(h);
-    if (rc)
-        return rc;
-    for (uint64_t n0 = 0; n0 < h->g.N; n0 += COPY_NODES) {
-        const uint64_t cnt = std::min<uint64_t>(COPY_NODES, h->g.N - n0);
+    return nodes_to_host(h, f, 19 * sizeof(double), "lbm_download_f", [h](uint64_t n0, uint64_t cnt, char *dev) {
         CopyArgs a;
         a.g = h->g;
         a.L = h->lat[h->cur];
-        a.aos = h->stage;
+        a.aos = (double *)dev;
         a.n0 = n0;
         a.count = cnt;
-        rc = dispatch_err(PREC_CALL(h, gather, a, h->stream), "download gather");
-        if (rc)
-            return rc;
-        HIP_TRY(hipMemcpyAsync(f + n0 * 19, h->stage, cnt * 19 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-        HIP_TRY(hipStreamSynchronize(h->stream));
-    }
-    return LBM_OK;
+        return PREC_CALL(h, gather, a, h->stream);
+    });
 }
 
 int lbm_set_force(lbm_channel *h, double fx, double fy, double fz)
@@ -911,10 +1002,12 @@ int lbm_set_macros(lbm_channel *h, const double *rho, const double *ux, const do
     if (rc)
         return rc;
     const double *src[4] = {rho, ux, uy, uz};
+    HostPart parts[4];
     for (int k = 0; k < 4; k++)
-        if (src[k])
-            HIP_TRY(hipMemcpyAsync(h->mac[k], src[k], h->g.N * sizeof(double), hipMemcpyHostToDevice, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
+        parts[k] = HostPart{const_cast<double *>(src[k]), h->mac[k], h->g.N * sizeof(double)};
+    rc = copy_parts(h, parts, 4, false, "lbm_set_macros");
+    if (rc)
+        return rc;
     h->fresh = false;
     return LBM_OK;
 }
@@ -1062,11 +1155,10 @@ int lbm_macrovar(lbm_channel *h, double *rho, double *ux, double *uy, double *uz
     int rc = compute_fields(h, h->cur);
     if (rc)
         return rc;
+    HostPart parts[4];
     for (int k = 0; k < 4; k++)
-        if (dst[k])
-            HIP_TRY(hipMemcpyAsync(dst[k], h->mac[k], h->g.N * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    return LBM_OK;
+        parts[k] = HostPart{dst[k], h->mac[k], h->g.N * sizeof(double)};
+    return copy_parts(h, parts, 4, true, "lbm_macrovar");
 }
 
 int lbm_rhoupdat(lbm_channel *h, double *rhoerrmax)
@@ -1520,11 +1612,9 @@ int lbm_vortcalc(lbm_channel *h, double *ox, double *oy, double *oz)
                        (const double *)h->mac[1], (const double *)h->mac[2], (const double *)h->mac[3], solid_of(h),
                        omg, d, d + h->g.N, d + 2 * h->g.N);
     e = hipGetLastError();
-    double *dst[3] = {ox, oy, oz};
-    for (int k = 0; k < 3 && e == hipSuccess; k++)
-        e = hipMemcpyAsync(dst[k], d + (size_t)k * h->g.N, bytes, hipMemcpyDeviceToHost, h->stream);
+    const HostPart parts[3] = {{ox, d, bytes}, {oy, d + h->g.N, bytes}, {oz, d + 2 * h->g.N, bytes}};
     if (e == hipSuccess)
-        e = hipStreamSynchronize(h->stream);
+        e = host_copy(h->cfg.device, h->stream, parts, 3, true);
     (void)hipFree(d);
     if (e != hipSuccess)
         return fail(LBM_ERR_HIP, "lbm_vortcalc: %s", hipGetErrorString(e));
@@ -1742,7 +1832,7 @@ int lbm_device_bytes(lbm_channel *h, size_t *bytes)
     if (h->mac[0])
         b += 4 * (size_t)h->g.N * sizeof(double);
     if (h->stage)
-        b += COPY_NODES * 19 * sizeof(double);
+        b += STAGE_BYTES;
     if (h->bring)
         b += (block_ring_elems(h->g, h->baxis, h->bK, h->bW) + block_head_elems(h->g, h->baxis, h->bW)) * h->elem;
     b += (2 * RED_BLOCKS + (size_t)PLANE_CHUNKS * NPLANE * h->g.lx + 2 + 2 * NPLANE * (size_t)h->g.lx) * sizeof(double) + 8;
@@ -1769,41 +1859,61 @@ int lbm_block_rows(lbm_channel *h, int *rows)
     return LBM_OK;
 }
 
+// `count` stored values of population i at `v` as FP64.
+static void widen(const lbm_channel *h, int i, const void *v, uint64_t count, double *o)
+{
+    if (h->prec == LBM_FP64) {
+        memcpy(o, v, count * sizeof(double));
+    } else if (h->prec == LBM_FP32) {
+        const float *x = (const float *)v;
+        for (uint64_t n = 0; n < count; n++)
+            o[n] = x[n];
+    } else if (h->prec == LBM_FP16) {
+        const _Float16 *x = (const _Float16 *)v;
+        const double sc = i == 0 ? 0.25 : (i <= 6 ? 1.0 / 16.0 : 1.0 / 32.0);
+        for (uint64_t n = 0; n < count; n++)
+            o[n] = (double)(float)x[n] * sc;
+    } else {
+        const uint16_t *x = (const uint16_t *)v;
+        const float sc = FP16C_UP / fp16_scale_rt(i);
+        for (uint64_t n = 0; n < count; n++)
+            o[n] = (double)(fp16c_unpack(x[n]) * sc);
+    }
+}
+
 // Nodes [n0, n0 + count) of the stored post-collision lattice as FP64,
-// population-major (out[i*count + k] = P_i(n0 + k)).
+// population-major (out[i*count + k] = P_i(n0 + k)), widened on the host.
 static int download_post_range(lbm_channel *h, uint64_t n0, uint64_t count, double *out)
 {
     const uint64_t S = h->g.S;
     const unsigned char *L = (const unsigned char *)h->lat[h->cur];
-    if (h->prec == LBM_FP64) {
-        for (int i = 0; i < 19; i++)
-            HIP_TRY(hipMemcpyAsync(out + (size_t)i * count, L + ((size_t)i * S + n0) * sizeof(double),
-                                   count * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-        HIP_TRY(hipStreamSynchronize(h->stream));
+    const hipStream_t s = h->stream;
+    HIP_TRY(hipStreamSynchronize(s));
+    HostPool &pool = host_pool();
+    std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
+    if (19 * count * h->elem >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device)) {
+        const uint64_t per = HOST_SLICE / h->elem, m = (count + per - 1) / per; // slices of a population
+        const hipError_t e = host_slices_out(
+            pool, h->cfg.device, s, 19 * m, host_workers(19 * count * sizeof(double)),
+            [&](size_t k, int, char *pinned) {
+                const uint64_t i = k / m, at = k % m * per;
+                return hipMemcpyAsync(pinned, L + (i * S + n0 + at) * h->elem,
+                                      std::min<uint64_t>(per, count - at) * h->elem, hipMemcpyDeviceToHost, s);
+            },
+            [&](size_t k, const char *pinned) {
+                const uint64_t i = k / m, at = k % m * per;
+                widen(h, (int)i, pinned, std::min<uint64_t>(per, count - at), out + i * count + at);
+            });
+        if (e != hipSuccess)
+            return fail(LBM_ERR_HIP, "lattice download: %s", hipGetErrorString(e));
         return LBM_OK;
     }
-    // FP32/FP16/FP16C: widen on the host, population by population
     std::vector<unsigned char> buf(count * h->elem);
     for (int i = 0; i < 19; i++) {
         HIP_TRY(hipMemcpyAsync(buf.data(), L + ((size_t)i * S + n0) * h->elem, count * h->elem,
-                               hipMemcpyDeviceToHost, h->stream));
-        HIP_TRY(hipStreamSynchronize(h->stream));
-        double *o = out + (size_t)i * count;
-        if (h->prec == LBM_FP32) {
-            const float *v = (const float *)buf.data();
-            for (uint64_t n = 0; n < count; n++)
-                o[n] = v[n];
-        } else if (h->prec == LBM_FP16) {
-            const _Float16 *v = (const _Float16 *)buf.data();
-            const double sc = i == 0 ? 0.25 : (i <= 6 ? 1.0 / 16.0 : 1.0 / 32.0);
-            for (uint64_t n = 0; n < count; n++)
-                o[n] = (double)(float)v[n] * sc;
-        } else {
-            const uint16_t *v = (const uint16_t *)buf.data();
-            const float sc = FP16C_UP / fp16_scale_rt(i);
-            for (uint64_t n = 0; n < count; n++)
-                o[n] = (double)(fp16c_unpack(v[n]) * sc);
-        }
+                               hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        widen(h, i, buf.data(), count, out + (size_t)i * count);
     }
     return LBM_OK;
 }
@@ -2130,9 +2240,8 @@ int lbm_particles_solid(lbm_channel *h, int *solid)
     CHECK_P(h);
     if (!solid)
         return fail(LBM_ERR_ARG, "lbm_particles_solid: null output");
-    HIP_TRY(hipMemcpyAsync(solid, h->part->ps.solid, h->g.N * sizeof(int), hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    return LBM_OK;
+    const HostPart part = {solid, h->part->ps.solid, h->g.N * sizeof(int)};
+    return copy_parts(h, &part, 1, true, "lbm_particles_solid");
 }
 
 int lbm_closure_set(lbm_channel *h, const float *params, double ystar)
@@ -2185,26 +2294,10 @@ static int closure_eval(lbm_channel *h, float *out, int what, const char *name)
     a.mlp = h->mlp;
     a.inv_ystar = h->mlp_inv_ystar;
     a.yscale = h->mlp_yscale;
-    const int width = what == 0 ? MLP_IN : 1;
-    float *buf = nullptr;
-    const uint64_t chunk = std::min<uint64_t>(COPY_NODES, h->g.N);
-    HIP_TRY(hipMalloc((void **)&buf, chunk * width * sizeof(float)));
-    int rc = LBM_OK;
-    for (uint64_t n0 = 0; n0 < h->g.N && rc == LBM_OK; n0 += chunk) {
-        const uint64_t cnt = std::min<uint64_t>(chunk, h->g.N - n0);
-        rc = dispatch_err(PREC_CALL(h, closure_eval, a, n0, cnt, buf, what, h->stream), name);
-        if (rc == LBM_OK) {
-            hipError_t e = hipMemcpyAsync(out + n0 * width, buf, cnt * width * sizeof(float), hipMemcpyDeviceToHost,
-                                          h->stream);
-            if (e == hipSuccess)
-                e = hipStreamSynchronize(h->stream);
-            if (e != hipSuccess)
-                rc = fail(LBM_ERR_HIP, "%s: copy failed: %s", name, hipGetErrorString(e));
-        }
-    }
-    (void)hipStreamSynchronize(h->stream);
-    (void)hipFree(buf);
-    return rc;
+    const size_t node_bytes = (what == 0 ? MLP_IN : 1) * sizeof(float);
+    return nodes_to_host(h, out, node_bytes, name, [&](uint64_t n0, uint64_t cnt, char *dev) {
+        return PREC_CALL(h, closure_eval, a, n0, cnt, (float *)dev, what, h->stream);
+    });
 }
 
 int lbm_closure_inputs(lbm_channel *h, float *feat) { return closure_eval(h, feat, 0, "lbm_closure_inputs"); }
@@ -2239,6 +2332,7 @@ int lbm_trainer_create(int device, long long capacity, const float *params, lbm_
     HIP_TRY(hipSetDevice(device));
     lbm_trainer *t = new lbm_trainer();
     memset(t, 0, sizeof(*t));
+    host_pool().retain();
     t->device = device;
     t->capacity = capacity;
     t->max_waves = 1u << 16;
@@ -2278,6 +2372,7 @@ int lbm_trainer_destroy(lbm_trainer *t)
             (void)hipFree(p);
     if (t->stream)
         (void)hipStreamDestroy(t->stream);
+    host_pool().release();
     delete t;
     return LBM_OK;
 }
@@ -2401,11 +2496,10 @@ int lbm_trainer_add_samples(lbm_trainer *t, const float *features, const float *
     CHECK_T(t);
     if (!features || !targets || n < 0 || t->count + n > t->capacity)
         return fail(LBM_ERR_ARG, "lbm_trainer_add_samples: bad arguments or capacity exceeded");
-    HIP_TRY(hipMemcpyAsync(t->feat + (size_t)t->count * MLP_IN, features, (size_t)n * MLP_IN * sizeof(float),
-                           hipMemcpyHostToDevice, t->stream));
-    HIP_TRY(hipMemcpyAsync(t->target + t->count, targets, (size_t)n * sizeof(float), hipMemcpyHostToDevice,
-                           t->stream));
-    HIP_TRY(hipStreamSynchronize(t->stream));
+    const HostPart parts[2] = {
+        {const_cast<float *>(features), t->feat + (size_t)t->count * MLP_IN, (size_t)n * MLP_IN * sizeof(float)},
+        {const_cast<float *>(targets), t->target + t->count, (size_t)n * sizeof(float)}};
+    HIP_TRY(host_copy(t->device, t->stream, parts, 2, false));
     t->count += n;
     return LBM_OK;
 }
@@ -2415,13 +2509,9 @@ int lbm_trainer_samples(lbm_trainer *t, long long *n, float *features, float *ta
     CHECK_T(t);
     if (n)
         *n = t->count;
-    if (features)
-        HIP_TRY(hipMemcpyAsync(features, t->feat, (size_t)t->count * MLP_IN * sizeof(float), hipMemcpyDeviceToHost,
-                               t->stream));
-    if (targets)
-        HIP_TRY(hipMemcpyAsync(targets, t->target, (size_t)t->count * sizeof(float), hipMemcpyDeviceToHost,
-                               t->stream));
-    HIP_TRY(hipStreamSynchronize(t->stream));
+    const HostPart parts[2] = {{features, t->feat, (size_t)t->count * MLP_IN * sizeof(float)},
+                               {targets, t->target, (size_t)t->count * sizeof(float)}};
+    HIP_TRY(host_copy(t->device, t->stream, parts, 2, true));
     return LBM_OK;
 }
 
