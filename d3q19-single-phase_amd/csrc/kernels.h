@@ -74,6 +74,9 @@ struct StepArgs {
     ForceSpec fm;      // mode bit 16: force that the fused fields u = j + F/2 are formed with
 };
 
+// Slots of rhoupdat's maximum, a cache line apart.
+constexpr uint32_t ERR_SLOTS = 64, ERR_STRIDE = 8;
+
 struct MacroArgs {
     Geom g;
     const void *L;

@@ -666,7 +666,9 @@ __global__ void __launch_bounds__(BLOCK) k_step_run(StepArgs a)
 
 // macrovar / rhoupdat / materialisation of the fields of lattice L.
 // WHAT 0: rho, ux, uy, uz = macrovar(F) with rho - rho_off.
-// WHAT 1: rho = sum F (rhoupdat); max |rho_new - rho_old| into *errbits.
+// WHAT 1: rho = sum F (rhoupdat); max |rho_new - rho_old| into errbits, one of
+// ERR_SLOTS per block: on a single word the blocks' atomics took turns (64x192x96
+// in FP64, 4 608 blocks: 63 us with one word, 36 us with 64).
 template <int P, int WHAT>
 __global__ void __launch_bounds__(BLOCK) k_macro(MacroArgs a)
 {
@@ -714,7 +716,7 @@ __global__ void __launch_bounds__(BLOCK) k_macro(MacroArgs a)
             unsigned long long m = wmax[0];
             for (int w = 1; w < BLOCK / 64; w++)
                 m = wmax[w] > m ? wmax[w] : m;
-            atomicMax(a.errbits, m);
+            atomicMax(a.errbits + (blockIdx.x % ERR_SLOTS) * ERR_STRIDE, m);
         }
     }
 }

@@ -92,7 +92,7 @@ struct lbm_channel {
     hipStream_t stream;
     double *partials;   // 2*RED_BLOCKS doubles, then PLANE_CHUNKS*NPLANE*lx doubles
     double *red_out;    // 2 doubles + NPLANE*lx doubles of final sums
-    unsigned long long *errbits;
+    unsigned long long *errbits; // ERR_SLOTS maxima of rhoupdat
     double *stat_acc;   // NPLANE*lx running sums
     long long stat_n;
     double *fstat_acc;  // NPLANE*(lx/2) running sums of the box-filtered fields (allocated on first use)
@@ -654,7 +654,7 @@ int lbm_create(const lbm_config *cfg, lbm_channel **out)
     if (hipMalloc((void **)&h->partials, part * sizeof(double)) != hipSuccess ||
         hipMalloc((void **)&h->red_out, (2 + NPLANE * (size_t)c.lx) * sizeof(double)) != hipSuccess ||
         hipMalloc((void **)&h->stat_acc, NPLANE * (size_t)c.lx * sizeof(double)) != hipSuccess ||
-        hipMalloc((void **)&h->errbits, sizeof(unsigned long long)) != hipSuccess)
+        hipMalloc((void **)&h->errbits, ERR_SLOTS * ERR_STRIDE * sizeof(unsigned long long)) != hipSuccess)
         return cleanup(fail(LBM_ERR_NOMEM, "hipMalloc of reduction scratch failed"));
     e = hipMemsetAsync(h->stat_acc, 0, NPLANE * (size_t)c.lx * sizeof(double), h->stream);
     if (e == hipSuccess)
@@ -1168,7 +1168,7 @@ int lbm_rhoupdat(lbm_channel *h, double *rhoerrmax)
     int rc = materialize(h);
     if (rc)
         return rc;
-    HIP_TRY(hipMemsetAsync(h->errbits, 0, sizeof(unsigned long long), h->stream));
+    HIP_TRY(hipMemsetAsync(h->errbits, 0, ERR_SLOTS * ERR_STRIDE * sizeof(unsigned long long), h->stream));
     MacroArgs a;
     a.g = h->g;
     a.L = h->lat[h->cur];
@@ -1184,9 +1184,11 @@ int lbm_rhoupdat(lbm_channel *h, double *rhoerrmax)
         return rc;
     h->fresh = false;
     if (rhoerrmax) {
-        unsigned long long bits = 0;
-        HIP_TRY(hipMemcpyAsync(&bits, h->errbits, sizeof(bits), hipMemcpyDeviceToHost, h->stream));
+        unsigned long long slots[ERR_SLOTS * ERR_STRIDE], bits = 0;
+        HIP_TRY(hipMemcpyAsync(slots, h->errbits, sizeof(slots), hipMemcpyDeviceToHost, h->stream));
         HIP_TRY(hipStreamSynchronize(h->stream));
+        for (uint32_t k = 0; k < ERR_SLOTS; k++)
+            bits = std::max(bits, slots[k * ERR_STRIDE]);
         memcpy(rhoerrmax, &bits, sizeof(double));
     }
     return LBM_OK;
