@@ -144,6 +144,13 @@ __device__ __forceinline__ void store_all(typename Prec<P>::S *__restrict__ L, u
     store_all_impl<P>(L, N, n, f, std::make_integer_sequence<int, 19>{});
 }
 
+template <int P, int... Is>
+__device__ __forceinline__ void store_all_cached(typename Prec<P>::S *__restrict__ L, uint64_t N, uint32_t n,
+                                                 const typename Prec<P>::T (&f)[19], std::integer_sequence<int, Is...>)
+{
+    ((*elem<P>(L + (uint64_t)Is * N, n) = Prec<P>::template to_S<Is>(f[Is])), ...);
+}
+
 // Scatter the streamed value F_I(x) back to the post-collision slot it came
 // from (the inverse of pull).
 template <int P, int... Is>
@@ -228,6 +235,7 @@ __device__ __forceinline__ uint32_t node_index(const Geom &g, uint32_t nb)
 // N <= 2^28): the pulls with c_x != 0 take 32-bit offsets (pull<P, I, 1>);
 // the same loads, fewer instructions.  MODE + 64: 2-byte storage with
 // N <= 2^30: the pulls between adjacent rows only (pull<P, I, 2>).
+// MODE + 128: cached instead of non-temporal stores.
 template <int P, int MODE>
 __device__ __forceinline__ void step_node(const StepArgs &a)
 {
@@ -334,7 +342,10 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
         if (!active)
             return;
     }
-    store_all<P>(dst, a.g.S, n, f);
+    if constexpr ((MODE & 128) != 0)
+        store_all_cached<P>(dst, a.g.S, n, f, std::make_integer_sequence<int, 19>{});
+    else
+        store_all<P>(dst, a.g.S, n, f);
 }
 
 template <int P, int MODE>
@@ -698,7 +709,7 @@ __global__ void __launch_bounds__(BLOCK) k_macro(MacroArgs a)
         }
     }
     if constexpr (WHAT == 1) {
-        // max over the block, then one atomic per block, all on the bit
+        // max over the block, then one atomic per block on its slot, all on the bit
         // patterns: non-negative doubles order like their unsigned bit
         // patterns, and a NaN with the sign cleared (fabs) orders above
         // +inf, so a NaN anywhere becomes the result instead of being
@@ -1259,6 +1270,16 @@ static inline uint32_t step_threads(uint64_t N, uint32_t largest)
     return nb;
 }
 
+// 2-byte storage stores through the cache while the last-level cache holds
+// both lattices: a wave's non-temporal store of one population is a single
+// 128-byte line, and a step over a resident lattice then waits for memory
+// (FP16, 46 MB 97x150x83: 29.3 us non-temporal, 19.8 us cached; 70 MB
+// 96x192x100: 33.2 / 27.1 us; 125 MB 109x201x150: 64.0 / 44.4 us; 269 MB
+// 96x384x192: 101 / 107 us; 717 MB 271 / 276 us).  A branch on a kernel
+// argument instead of the step mode cost the large lattices 2.5 %.  FP64 and
+// FP32 measured no difference.
+constexpr uint64_t CACHED_STORE_BYTES = 256000000ull;
+
 template <int P>
 hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
 {
@@ -1290,6 +1311,16 @@ hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
         // 2-byte storage
         if (a.w32 == 1 && a.g.S <= w32_max_n(P)) {
             if constexpr (half_storage(P)) {
+                if (2 * 19 * a.g.S * sizeof(typename Prec<P>::S) <= CACHED_STORE_BYTES) {
+                    switch (mode) {
+                        STEP_CASE(160);
+                        STEP_CASE(161);
+                        STEP_CASE(164);
+                        STEP_CASE(176);
+                    default:
+                        break;
+                    }
+                }
                 switch (mode) {
                     STEP_CASE(32);
                     STEP_CASE(33);
