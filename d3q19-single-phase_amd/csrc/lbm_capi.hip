@@ -2188,9 +2188,12 @@ int lbm_run_particles(lbm_channel *h, int istep0, int nsteps)
         if (nave > 0 && istep % nave == 0)
             h->ave_pending = true;
         HIP_TRY(hipStreamWaitEvent(h->stream, h->pev[1], 0));
-        rc = dispatch_err(part_classify(pt->pg, pt->ps, 0, h->stream), "beads_links");
-        if (!rc)
-            rc = lbm_beads_filling(h);
+        void *lat = h->lat[h->cur];
+        e = h->prec == LBM_FP64   ? PartLaunch<0>::classify_refill(pt->pg, pt->ps, lat, h->stream)
+            : h->prec == LBM_FP32 ? PartLaunch<1>::classify_refill(pt->pg, pt->ps, lat, h->stream)
+            : h->prec == LBM_FP16 ? PartLaunch<2>::classify_refill(pt->pg, pt->ps, lat, h->stream)
+                                  : PartLaunch<3>::classify_refill(pt->pg, pt->ps, lat, h->stream);
+        rc = dispatch_err(e, "beads_links and beads_filling");
         if (rc)
             return rc;
     }

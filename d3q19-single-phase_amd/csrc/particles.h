@@ -123,6 +123,8 @@ template <int P>
 struct PartLaunch {
     static hipError_t ibb(const PartGeom &pg, const PartState &ps, void *L, hipStream_t s);
     static hipError_t refill(const PartGeom &pg, const PartState &ps, void *L, hipStream_t s);
+    // part_classify (not the first) and refill together
+    static hipError_t classify_refill(const PartGeom &pg, const PartState &ps, void *L, hipStream_t s);
 };
 
 hipError_t part_classify(const PartGeom &pg, const PartState &ps, int first, hipStream_t s);
