@@ -177,37 +177,73 @@ __device__ __forceinline__ void node_coords(uint32_t n, const Geom &g, uint32_t 
     iy = q - iz * g.ly;
 }
 
+// The factors of FORCINGP's field at node (ix, iy, iz), from the tables of one
+// coordinate each.
+struct ForceFactors {
+    double sg, x1, x2, cy, sy, cz, sz;
+    bool in_band;
+    __device__ __forceinline__ ForceFactors(const double *tab, const Geom &g, uint32_t ix, uint32_t iy, uint32_t iz)
+    {
+        // every table value loads at once (both bands' y factors), so no load
+        // waits for the band flag; the selects pick what the band needs
+        const double *xt = tab + 3 * ix;
+        const double *yt = tab + 3 * g.lx + 4 * iy;
+        const double *zt = tab + 3 * g.lx + 4 * g.ly + 2 * iz;
+        const double band = xt[0];
+        x1 = xt[1];
+        x2 = xt[2];
+        const double c1 = yt[0], s1 = yt[1], c2 = yt[2], s2 = yt[3];
+        cz = zt[0];
+        sz = zt[1];
+        const bool first = band == 1.0;
+        sg = first ? 1.0 : -1.0;
+        cy = first ? c1 : c2;
+        sy = first ? s1 : s2;
+        in_band = band != 0.0;
+    }
+    // The force of s in the operand order of Channel-Flow/collision.f90:571-576
+    // and 591-596; band 2's leading minus is carried by the first factor,
+    // which changes no bit of the product.
+    __device__ __forceinline__ void force(const ForceSpec &s, double &fx, double &fy, double &fz) const
+    {
+#pragma clang fp contract(off)
+        const double gx = (((sg * s.a) * x1) * cy) * cz;
+        const double gy = s.fy * (1.0 + (((-sg * s.b) * x2) * sy) * cz);
+        const double gz = (((sg * s.c) * x2) * cy) * sz;
+        fx = in_band ? gx : s.fx;
+        fy = in_band ? gy : s.fy;
+        fz = in_band ? gz : s.fz;
+    }
+};
+
 // Body force of s at node (ix, iy, iz), the value the reference's force
-// arrays hold there.  The FORCINGP products keep the operand order of
-// Channel-Flow/collision.f90:571-576 and 591-596; band 2's leading minus is
-// carried by the first factor, which changes no bit of the product.
+// arrays hold there.
 __device__ __forceinline__ void node_force(const ForceSpec &s, const Geom &g, uint32_t ix, uint32_t iy, uint32_t iz,
                                            double &fx, double &fy, double &fz)
 {
-#pragma clang fp contract(off)
     fx = s.fx;
     fy = s.fy;
     fz = s.fz;
     if (s.tab == nullptr)
         return;
-    // every table value loads at once (both bands' y factors), so no load
-    // waits for the band flag; the selects pick what the band needs
-    const double *xt = s.tab + 3 * ix;
-    const double *yt = s.tab + 3 * g.lx + 4 * iy;
-    const double *zt = s.tab + 3 * g.lx + 4 * g.ly + 2 * iz;
-    const double band = xt[0], x1 = xt[1], x2 = xt[2];
-    const double c1 = yt[0], s1 = yt[1], c2 = yt[2], s2 = yt[3];
-    const double cz = zt[0], sz = zt[1];
-    const bool first = band == 1.0;
-    const double sg = first ? 1.0 : -1.0;
-    const double cy = first ? c1 : c2, sy = first ? s1 : s2;
-    const double gx = (((sg * s.a) * x1) * cy) * cz;
-    const double gy = s.fy * (1.0 + (((-sg * s.b) * x2) * sy) * cz);
-    const double gz = (((sg * s.c) * x2) * cy) * sz;
-    const bool in_band = band != 0.0;
-    fx = in_band ? gx : fx;
-    fy = in_band ? gy : fy;
-    fz = in_band ? gz : fz;
+    ForceFactors(s.tab, g, ix, iy, iz).force(s, fx, fy, fz);
+}
+
+// Both forces of a step whose force varies over the nodes: fc for the
+// collision, fm for the fused fields.  Under FORCINGP the two differ in their
+// amplitudes only, so the factors are loaded and selected once (two separate
+// evaluations: 18 loads and twice the selects per node).
+__device__ __forceinline__ void node_forces(const ForceSpec &fc, const ForceSpec &fm, const Geom &g, uint32_t ix,
+                                            uint32_t iy, uint32_t iz, double (&c)[3], double (&m)[3])
+{
+    if (fc.tab != nullptr && fc.tab == fm.tab) {
+        const ForceFactors t(fc.tab, g, ix, iy, iz);
+        t.force(fc, c[0], c[1], c[2]);
+        t.force(fm, m[0], m[1], m[2]);
+    } else {
+        node_force(fc, g, ix, iy, iz, c[0], c[1], c[2]);
+        node_force(fm, g, ix, iy, iz, m[0], m[1], m[2]);
+    }
 }
 
 __device__ __forceinline__ uint32_t node_index(const Geom &g, uint32_t nb)
@@ -275,17 +311,18 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
     if constexpr ((MODE & 16) != 0) {
         uint32_t ix, iy, iz;
         node_coords(n, a.g, ix, iy, iz);
-        double x, y, z;
-        node_force(a.fc, a.g, ix, iy, iz, x, y, z);
-        r.fx = (T)x;
-        r.fy = (T)y;
-        r.fz = (T)z;
+        double c[3], m[3];
         if constexpr ((MODE & 3) != 2) {
-            node_force(a.fm, a.g, ix, iy, iz, x, y, z);
-            fmx = (T)x;
-            fmy = (T)y;
-            fmz = (T)z;
+            node_forces(a.fc, a.fm, a.g, ix, iy, iz, c, m);
+            fmx = (T)m[0];
+            fmy = (T)m[1];
+            fmz = (T)m[2];
+        } else {
+            node_force(a.fc, a.g, ix, iy, iz, c[0], c[1], c[2]);
         }
+        r.fx = (T)c[0];
+        r.fy = (T)c[1];
+        r.fz = (T)c[2];
     }
 
     T rho9, ux9, uy9, uz9;
@@ -439,15 +476,14 @@ __global__ void __launch_bounds__((plane_block<P, NT>())) k_step_planes(BlockArg
     T fmx = rt.fx, fmy = rt.fy, fmz = rt.fz; // force in u = j + F/2 of the fused fields
     if constexpr (FP != 0) {
         const uint32_t iy = AXIS == 2 ? br.rg : sb, iz = AXIS == 2 ? sb : br.rg;
-        double x, y, z;
-        node_force(a.fc, a.g, ix, iy, iz, x, y, z);
-        rt.fx = (T)x;
-        rt.fy = (T)y;
-        rt.fz = (T)z;
-        node_force(a.fm, a.g, ix, iy, iz, x, y, z);
-        fmx = (T)x;
-        fmy = (T)y;
-        fmz = (T)z;
+        double c[3], m[3];
+        node_forces(a.fc, a.fm, a.g, ix, iy, iz, c, m);
+        rt.fx = (T)c[0];
+        rt.fy = (T)c[1];
+        rt.fz = (T)c[2];
+        fmx = (T)m[0];
+        fmy = (T)m[1];
+        fmz = (T)m[2];
     }
     T rho9, ux9, uy9, uz9;
     macro_sums(f, rho9, ux9, uy9, uz9);

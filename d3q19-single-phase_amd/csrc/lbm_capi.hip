@@ -616,12 +616,13 @@ int lbm_create(const lbm_config *cfg, lbm_channel **out)
         // variables asks for the sweep at any size
         h->bskip = N * 19 * h->elem <= BLOCK_MIN_LATTICE_BYTES && !getenv("LBM_BLOCK_AXIS") &&
                    !getenv("LBM_BLOCK_PLANES") && !getenv("LBM_BLOCK_ROWS");
-        // LBM_BLOCK_FORCED=1: pairs under a force evaluated per node too.
-        // Off by default: on the 192x768x384 channel such pairs took 3.33 ms
-        // per FP64 step against 3.10 ms for single steps (the per-node force
-        // costs the latency-bound sweep what the HBM-bound step hides).
+        // Pairs under a force evaluated per node run as sweeps too
+        // (LBM_BLOCK_FORCED=0: as single steps).  With both steps' forces
+        // from one set of factors (node_forces) that is the faster form: us
+        // per step on 96x384x192, FP64 361 against 394 for single steps, FP32
+        // 191 / 199; on 192x768x384 2 869 / 3 081 and 1 403 / 1 607.
         const char *kf = getenv("LBM_BLOCK_FORCED");
-        h->bforced = (kf && strcmp(kf, "1") == 0) ? 1 : 0;
+        h->bforced = (kf && strcmp(kf, "0") == 0) ? 0 : 1;
         // LBM_DEFER=0: collision_MRT launches at once (no per-call pairing)
         const char *kd = getenv("LBM_DEFER");
         if (kd && strcmp(kd, "0") != 0 && strcmp(kd, "1") != 0) {
@@ -1316,7 +1317,7 @@ int lbm_run_forcingp(lbm_channel *h, int istep0, int nsteps, int npforcing, doub
             return rc;
         // a pair as one blocked sweep: fused fields of the current lattice,
         // no density offset, no particles or closure, and one uniform force
-        // (or, with bforced, any forces, evaluated per node)
+        // or, with bforced, any forces, evaluated per node
         bool paired = false;
         if (nsteps - s >= 2 && h->bK > 0 && !h->bskip && h->ms == FROM_CUR && h->rho_off == 0.0 && !h->part &&
             !h->mlp) {

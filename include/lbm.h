@@ -110,9 +110,9 @@ int lbm_forcingp(lbm_channel *h, int istep, double force_in_y);
  * istep0 + nsteps: lbm_forcingp(istep, force_in_y) while istep < npforcing,
  * lbm_set_force(0, fy_forcing, 0) at istep == npforcing (FORCING, with
  * fy_forcing = force_in_y*force_mag), then collision_MRT and macrovar.  Pairs
- * of steps under one uniform force run as one blocked sweep (see lbm_run);
- * FORCINGP steps run one by one, or also in pairs with the force evaluated
- * per node when LBM_BLOCK_FORCED=1 at lbm_create (measured slower).  Results
+ * of steps under one uniform force run as one blocked sweep (see lbm_run),
+ * pairs of FORCINGP steps too, with the force evaluated per node in both
+ * steps (LBM_BLOCK_FORCED=0 at lbm_create runs them one by one).  Results
  * equal those calls one by one, bit for bit.  No reference counterpart as
  * one call: it batches the driver's loop. */
 int lbm_run_forcingp(lbm_channel *h, int istep0, int nsteps, int npforcing, double force_in_y,
