@@ -30,10 +30,12 @@ constexpr int BLOCK = 256;
 // against 68 100); 256 for the plain FP32 step (39 220-39 330 against
 // 37 990-38 800 with 512 on the 2048x1024x512 channel) and the fused closure
 // (96 registers: five 256-thread blocks per CU against two of 512, 248 against
-// 255 us per step on the 96x384x192 channel).  128 was slower.  These are the
-// largest block sizes; step_threads takes smaller ones for small grids.
+// 255 us per step on the 96x384x192 channel) and the cached stores of 2-byte
+// storage (41.6 against 48.7-53.7 us on 96x256x128).  128 was slower.  These
+// are the largest block sizes; step_threads takes smaller ones for small
+// grids.
 template <int P, int MODE>
-constexpr int step_block() { return ((MODE & 8) != 0 || P == 1) ? 256 : 512; }
+constexpr int step_block() { return ((MODE & (8 | 128)) != 0 || P == 1) ? 256 : 512; }
 
 // Element `node` of a population row, addressed as the row base plus a 32-bit
 // byte offset when that cannot wrap: 2-byte storage, whose rows hold fewer than
@@ -1297,10 +1299,15 @@ static inline bool use_runs(const StepArgs &a, int mode)
 // threads, 6.3 us with 512).  With more blocks than CUs larger ones are
 // faster: waves that share cache lines then share a CU (97x150x83: 84 us with
 // 512 threads, 93 us with 64).
+// FP64 blocks of 512 threads pay off on the largest grids only (us per step,
+// 256 / 512 threads: 1.0 M nodes 60.3 / 63.3, 7.1 M 393 / 397, 28 M 1 556 / 1
+// 573, 57 M 3 108 / 3 100).
 constexpr uint32_t DEVICE_CUS = 256;
+constexpr uint64_t FP64_LARGE_N = 40000000;
+template <int P>
 static inline uint32_t step_threads(uint64_t N, uint32_t largest)
 {
-    uint32_t nb = largest;
+    uint32_t nb = P == 0 && N < FP64_LARGE_N ? std::min<uint32_t>(largest, 256) : largest;
     while (nb > 64 && (N + nb - 1) / nb < DEVICE_CUS)
         nb /= 2;
     return nb;
@@ -1331,7 +1338,7 @@ hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
         }
     }
     auto launch = [&](auto kernel, uint32_t largest) {
-        a.nb = step_threads(a.g.N, largest);
+        a.nb = step_threads<P>(a.g.N, largest);
         hipLaunchKernelGGL(kernel, dim3((uint32_t)((a.g.N + a.nb - 1) / a.nb)), dim3(a.nb), 0, s, a);
         return hipGetLastError();
     };
