@@ -62,13 +62,20 @@ inline uint32_t block_ring_rows(const Geom &g, int axis, uint32_t W)
     return block_windowed(g, axis, W) ? W + 2 : block_geom(g, axis).nr;
 }
 
-// Ring slots, elements of one population of a ring slab (lx * ring rows nodes,
-// rounded up to whole waves so that slabs start on cache lines) and buffer
-// sizes in elements.
+// Nodes of a z slab modulo a wave (BlockArgs::res), 0 for y slabs and row
+// windows, whose rows are not contiguous in the lattice.
+inline uint32_t block_residue(const Geom &g, int axis, uint32_t W)
+{
+    return axis == 2 && !block_windowed(g, axis, W) ? g.lx * g.ly % WAVE_LANES : 0u;
+}
+
+// Ring slots, elements of one population of a ring slab (lx * ring rows nodes
+// and their shift, rounded up to whole waves so that slots start on cache
+// lines) and buffer sizes in elements.
 inline uint32_t block_ring_slots(uint32_t K) { return K + 2; }
 inline uint64_t block_ring_slab(const Geom &g, int axis, uint32_t W)
 {
-    return slab_padded(g.lx * block_ring_rows(g, axis, W));
+    return slab_padded(g.lx * block_ring_rows(g, axis, W) + (block_residue(g, axis, W) ? WAVE_LANES - 1 : 0u));
 }
 inline uint64_t block_ring_elems(const Geom &g, int axis, uint32_t K, uint32_t W = 0)
 {
@@ -100,11 +107,12 @@ inline std::vector<BlockArgs> block_schedule(const Geom &g, int axis, const Step
     const uint32_t ns = bg.ns, nr = bg.nr, slots = block_ring_slots(K);
     const bool win = block_windowed(g, axis, W);
     const uint64_t rslab = block_ring_slab(g, axis, W);
+    const uint32_t res = block_residue(g, axis, W);
     const PlaneStore full_in = {lat_in, ls, ns, make_fastdiv(ns), bg.lat_slab_stride, bg.lat_row_stride, nullptr, 0,
-                                0, 0};
+                                0, 0, 0};
     const PlaneStore full_out = {lat_out, ls, ns, make_fastdiv(ns), bg.lat_slab_stride, bg.lat_row_stride, nullptr, 0,
-                                 0, 0};
-    const PlaneStore ring_only = {ring, slots * rslab, slots, make_fastdiv(slots), rslab, g.lx, nullptr, 0, 0, 0};
+                                 0, 0, 0};
+    const PlaneStore ring_only = {ring, slots * rslab, slots, make_fastdiv(slots), rslab, g.lx, nullptr, 0, 0, 0, res};
     PlaneStore ring_head = ring_only;
     ring_head.head = head;
     ring_head.head_stride = 2 * rslab;
@@ -132,6 +140,9 @@ inline std::vector<BlockArgs> block_schedule(const Geom &g, int axis, const Step
         a.slab = g.lx * rw.nrw;
         a.slabp = slab_padded(a.slab);
         a.dslabp = make_fastdiv(a.slabp);
+        a.res = res;
+        a.slabt = slab_padded(a.slab + (res ? WAVE_LANES - 1 : 0u));
+        a.dslabt = make_fastdiv(a.slabt);
         a.r = f.r;
         a.fc = f.fc;
         a.fm = f.fm;
@@ -177,14 +188,23 @@ constexpr double BLOCK_RING_BYTES = 225e6;
 constexpr long BLOCK_MIN_SLABS = 4;
 constexpr long BLOCK_MAX_SLABS = 32;
 
-// Pairs of steps of lattices up to this size run as single steps.  Both
-// lattices, or most of one, then stay in the last-level cache anyway, and the
-// sweep only adds launches and halo slabs.  us per step, sweep against single
-// steps: FP64 10 MB (32x64x32) 11.7 / 6.1, 53 MB 40 / 24, 184 MB (97x150x83)
-// 81 / 74, 280 MB 106 / 107, 342 MB 126 / 129, 478 MB 172 / 189; FP32 27 MB
-// 28 / 13, 140 MB 60 / 56, 239 MB 93 / 90-101, 294 MB 111 / 107, 538 MB 185 /
-// 194.
+// Pairs of steps run as single steps when the lattice is small or the sweep's
+// chunks are.
+//
+// A lattice of up to BLOCK_MIN_LATTICE_BYTES, or most of one, stays in the
+// last-level cache anyway, and the sweep only adds launches and halo slabs.
+// us per step, sweep against single steps: FP64 10 MB (32x64x32) 11.7 / 6.1,
+// 53 MB 40 / 24, 184 MB (97x150x83) 81 / 74, 280 MB 106 / 107, 342 MB 126 /
+// 129, 478 MB 172 / 189; FP32 27 MB 28 / 13, 140 MB 60 / 56, 239 MB 93 /
+// 90-101, 294 MB 111 / 107, 538 MB 185 / 194.
+//
+// A chunk of K slabs of less than BLOCK_MIN_CHUNK_BYTES (K is at most 32) makes
+// launches too short to hide their start and end: FP64 66 MB (45x301x180) 150
+// / 135, 75 MB 198 / 190, 126 MB 207 / 217, 188 MB 292 / 325; FP32 33 MB
+// (45x301x180) 95 / 73, 63 MB 116 / 107, 81 MB 297 / 281, 94 MB 163 / 159-271 /
+// 274, 172 MB 464 / 475, 186 MB 502 / 529.
 constexpr uint64_t BLOCK_MIN_LATTICE_BYTES = 300000000ull;
+constexpr uint64_t BLOCK_MIN_CHUNK_BYTES = 90000000ull;
 
 // The sweep lbm_create chooses for a lattice of elem-byte values: axis 2 (z)
 // or 1 (y), K slabs per chunk (0: single steps only) and W rows per window

@@ -142,6 +142,7 @@ struct PlaneStore {
     uint64_t head_stride;
     int32_t head_lo;
     uint32_t head_n;
+    uint32_t res; // slab s starts (s * res) % WAVE_LANES elements into its slot (BlockArgs::res)
 };
 
 // Slab s of a store: buffer, population stride, element offset of the slab
@@ -159,36 +160,50 @@ __host__ __device__ inline uint32_t ring_slot(const PlaneStore &st, uint32_t s)
     return s - fdiv(s, st.dslots) * st.ring_slots;
 }
 
+constexpr uint32_t WAVE_LANES = 64;
+
+// Elements by which slab s starts past a multiple of WAVE_LANES.
+__host__ __device__ inline uint32_t slab_shift(uint32_t res, uint32_t s) { return (s * res) & (WAVE_LANES - 1); }
+
 // Slab s as a reader sees it.
 __host__ __device__ inline PlaneRef plane_read(const PlaneStore &st, uint32_t s)
 {
     const uint32_t h = s - (uint32_t)st.head_lo; // wraps for s < head_lo
     if (st.head != nullptr && h < st.head_n)
-        return PlaneRef{st.head, st.head_stride, (uint64_t)h * st.slab_stride, st.row_stride};
-    return PlaneRef{st.ring, st.ring_stride, (uint64_t)ring_slot(st, s) * st.slab_stride, st.row_stride};
+        return PlaneRef{st.head, st.head_stride, (uint64_t)h * st.slab_stride + slab_shift(st.res, s), st.row_stride};
+    return PlaneRef{st.ring, st.ring_stride, (uint64_t)ring_slot(st, s) * st.slab_stride + slab_shift(st.res, s),
+                    st.row_stride};
 }
 
 // Slab s as a writer stores it: always its ring slot, and also the head copy
 // when s is a head slab (plane_write_head; buf = nullptr otherwise).
 __host__ __device__ inline PlaneRef plane_write(const PlaneStore &st, uint32_t s)
 {
-    return PlaneRef{st.ring, st.ring_stride, (uint64_t)ring_slot(st, s) * st.slab_stride, st.row_stride};
+    return PlaneRef{st.ring, st.ring_stride, (uint64_t)ring_slot(st, s) * st.slab_stride + slab_shift(st.res, s),
+                    st.row_stride};
 }
 
 __host__ __device__ inline PlaneRef plane_write_head(const PlaneStore &st, uint32_t s)
 {
     const uint32_t h = s - (uint32_t)st.head_lo;
     if (st.head != nullptr && h < st.head_n)
-        return PlaneRef{st.head, st.head_stride, (uint64_t)h * st.slab_stride, st.row_stride};
+        return PlaneRef{st.head, st.head_stride, (uint64_t)h * st.slab_stride + slab_shift(st.res, s), st.row_stride};
     return PlaneRef{nullptr, 0, 0, 0};
 }
 
 // One launch of the blocked sweep: one time step (fused macrovar, mode 0) of
 // slabs s0, s0+1, ..., s0+count-1 (taken modulo ns), gathering from `src` and
-// storing into `dst` (non-temporal stores when nt).  Thread t works on node
-// t % slabp of the launch's slab t / slabp: slabs are padded to whole waves
-// (slabp = slab rounded up to a multiple of 64), so every wave lies in one
-// slab and the slab's buffers and offsets are the same for all its lanes.
+// storing into `dst` (non-temporal stores when nt).  Slabs are padded to whole
+// waves (slabp = slab rounded up to a multiple of 64), so every wave lies in
+// one slab and the slab's buffers and offsets are the same for all its lanes.
+// Thread t works on node t % slabt - slab_shift(res, s) of the launch's slab t /
+// slabt.  When whole z slabs of lx * ly nodes do not fill cache lines, res is
+// that count modulo 64 and slabt leaves room for the shift: a wave's nodes
+// then start on a line of the lattice, and of the ring, whose slots hold each
+// slab at the same shift.  Without it every wave stored two partial lines a
+// population (us per step without / with, single steps: 191x401x255 FP64 1 160
+// / 964, 1 081; FP32 565 / 502, 529; 98x301x201 FP64 335 / 316, 337).
+// Otherwise res = 0 and slabt = slabp.
 // per_node: the body force is evaluated at every node as in step mode 16
 // (fc for the collision, fm for the fused fields u = j + F/2); otherwise it
 // is r.fx, r.fy, r.fz for both.
@@ -208,6 +223,8 @@ struct BlockArgs {
     uint32_t slab;       // nodes computed per slab, lx * nrw
     uint32_t slabp;      // slab rounded up to a whole number of waves
     FastDiv dslabp;      // division by slabp
+    uint32_t slabt, res; // threads per slab and the slabs' residue
+    FastDiv dslabt;      // division by slabt
     int32_t s0;
     uint32_t count;
     PlaneStore src, dst;
@@ -216,8 +233,6 @@ struct BlockArgs {
     int per_node;
     int nt;
 };
-
-constexpr uint32_t WAVE_LANES = 64;
 
 inline uint32_t slab_padded(uint32_t slab) { return (slab + WAVE_LANES - 1) / WAVE_LANES * WAVE_LANES; }
 

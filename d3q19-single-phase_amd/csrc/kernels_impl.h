@@ -460,13 +460,15 @@ __global__ void __launch_bounds__((plane_block<P, NT>())) k_step_planes(BlockArg
     const uint32_t t = blockIdx.x * plane_block<P, NT>() + threadIdx.x;
     // the wave's slab, uniform across its lanes (slabs are padded to whole
     // waves), so the slab buffers and offsets below stay in scalar registers
-    const uint32_t sl = __builtin_amdgcn_readfirstlane(fdiv(t, a.dslabp));
-    const uint32_t w = t - sl * a.slabp;
-    if (sl >= a.count || w >= a.slab)
+    const uint32_t sl = __builtin_amdgcn_readfirstlane(fdiv(t, a.dslabt));
+    if (sl >= a.count)
+        return;
+    const uint32_t sb = block_plane(a, sl);
+    const uint32_t w = t - sl * a.slabt - slab_shift(a.res, sb); // wraps below the shift
+    if (w >= a.slab)
         return;
     const BlockRow br = block_row(a, w);
     const uint32_t ix = br.ix;
-    const uint32_t sb = block_plane(a, sl);
     PlaneRef pl[3];
     block_planes(a, sb, pl);
     const BlockLane l = block_lane(ix, br.rs, a.src_nr, (uint32_t)a.src.row_stride, a.g.lx);
@@ -1426,7 +1428,7 @@ template <int P>
 hipError_t Launch<P>::step_planes(const BlockArgs &a, int axis, hipStream_t s)
 {
     const uint32_t PB = a.nt ? plane_block<P, 1>() : plane_block<P, 0>();
-    const dim3 grid((uint32_t)(((uint64_t)a.slabp * a.count + PB - 1) / PB)), blk(PB);
+    const dim3 grid((uint32_t)(((uint64_t)a.slabt * a.count + PB - 1) / PB)), blk(PB);
     const int v = (axis == 2 ? 4 : axis == 1 ? 0 : -8) + (a.nt ? 2 : 0) + (a.per_node ? 1 : 0);
     switch (v) {
     case 0: hipLaunchKernelGGL((k_step_planes<P, 1, 0, 0>), grid, blk, 0, s, a); break;

@@ -602,8 +602,14 @@ int lbm_create(const lbm_config *cfg, lbm_channel **out)
         // by default for 2-byte storage, whose step is bound by arithmetic
         // (FP16: measured 66 300 MLUPS blocked, 32 to a chunk, against 72 000
         // single-step).
+        // Rows that are not whole cache lines are swept along z: z slabs are
+        // contiguous, so their waves can start on lines (BlockArgs::res).
+        const char *axis = getenv("LBM_BLOCK_AXIS");
+        if (!axis && c.lx * h->elem % 128 != 0 && (uint64_t)c.lx * c.ly * 19 * h->elem * (BLOCK_MIN_SLABS + 2) <=
+                                                      (uint64_t)BLOCK_RING_BYTES)
+            axis = "z";
         const BlockChoice bc =
-            block_choice(h->g, h->elem, h->elem != 2, BLOCK_RING_BYTES, BLOCK_MIN_SLABS, getenv("LBM_BLOCK_AXIS"),
+            block_choice(h->g, h->elem, h->elem != 2, BLOCK_RING_BYTES, BLOCK_MIN_SLABS, axis,
                          getenv("LBM_BLOCK_PLANES"), getenv("LBM_BLOCK_ROWS"));
         if (bc.bad) {
             (void)lbm_destroy(h);
@@ -612,10 +618,12 @@ int lbm_create(const lbm_config *cfg, lbm_channel **out)
         h->baxis = bc.axis;
         h->bK = bc.K;
         h->bW = bc.W;
-        // small lattices are faster in single steps; setting the sweep's
-        // variables asks for the sweep at any size
-        h->bskip = N * 19 * h->elem <= BLOCK_MIN_LATTICE_BYTES && !getenv("LBM_BLOCK_AXIS") &&
-                   !getenv("LBM_BLOCK_PLANES") && !getenv("LBM_BLOCK_ROWS");
+        // small lattices and chunks are faster in single steps; setting the
+        // sweep's variables asks for the sweep at any size
+        const uint64_t chunk_rows = bc.W ? bc.W : block_geom(h->g, bc.axis).nr;
+        h->bskip = (N * 19 * h->elem <= BLOCK_MIN_LATTICE_BYTES ||
+                    bc.K * chunk_rows * c.lx * 19 * h->elem < BLOCK_MIN_CHUNK_BYTES) &&
+                   !getenv("LBM_BLOCK_AXIS") && !getenv("LBM_BLOCK_PLANES") && !getenv("LBM_BLOCK_ROWS");
         // Pairs under a force evaluated per node run as sweeps too
         // (LBM_BLOCK_FORCED=0: as single steps).  With both steps' forces
         // from one set of factors (node_forces) that is the faster form: us

@@ -177,9 +177,10 @@ int lbm_avedensity(lbm_channel *h, double *rhomean);
  * the single-step path's bit for bit.  The environment variables
  * LBM_BLOCK_AXIS=z|y and LBM_BLOCK_PLANES (read by lbm_create) set the axis
  * and the slabs per chunk (at most 32), 0 turns the sweep off; lbm_block_info
- * and lbm_block_rows report the choice.  Lattices of at most 300 MB run their
- * steps one by one, which measures faster there, unless one of the sweep's
- * variables is set. */
+ * and lbm_block_rows report the choice.  Lattices of at most 300 MB, and those whose
+ * slabs are so small that a chunk holds less than 90 MB, run their steps one
+ * by one, which measures faster there, unless one of the sweep's variables is
+ * set. */
 int lbm_run(lbm_channel *h, int nsteps);
 
 /* Sum of all populations in FP64 (mass monitor; the sum is invariant under

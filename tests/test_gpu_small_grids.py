@@ -1,8 +1,9 @@
 """GPU tests of the main loop on small lattices, whose pairs of steps run as
 single steps in smaller blocks: grids around each block size (64 threads up to
-512, with and without a remainder), FP64, bit for bit against the oracle; and
-the per-call pairing with the sweep asked for, which such lattices no longer
-take by themselves."""
+512, with and without a remainder), FP64, bit for bit against the oracle; the
+per-call pairing with the sweep asked for, which such lattices no longer take
+by themselves; and the sweep along z slabs of every residue modulo a wave,
+bit for bit against single steps."""
 import numpy as np
 import pytest
 
@@ -66,3 +67,26 @@ def test_per_call_pairs_with_the_sweep_asked_for(monkeypatch, prec):
                     c.stats_accumulate()  # launches what is deferred
         assert np.array_equal(bits(paired.download_post()), bits(single.download_post()))
         assert np.array_equal(bits(paired.statistc2()), bits(single.statistc2()))
+
+
+# lx * ly modulo 64: 0, 1, 32, 63 and others; slabs below a wave and of several
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("lx,ly,lz,k", [(16, 8, 9, 3), (5, 13, 11, 2), (12, 8, 7, 3), (7, 9, 12, 4), (3, 7, 5, 5),
+                                        (13, 11, 10, 1), (33, 31, 17, 6), (9, 7, 1, 1), (9, 7, 2, 2)])
+def test_sweep_of_slabs_that_do_not_fill_waves(monkeypatch, prec, lx, ly, lz, k):
+    u = workloads.laminar_parabola_noise(lx, ly, lz, seed=10)
+    monkeypatch.setenv("LBM_BLOCK_AXIS", "z")
+    monkeypatch.setenv("LBM_BLOCK_PLANES", str(k))
+    swept = d3q19.Channel(lx, ly, lz, prec)
+    monkeypatch.setenv("LBM_BLOCK_PLANES", "0")
+    single = d3q19.Channel(lx, ly, lz, prec)
+    with swept, single:
+        for c in (swept, single):
+            _start(c, u)
+            c.run(6)
+            c.run_forcingp(6, 4, 9)
+        a, b = swept.download_post(), single.download_post()
+    if prec == "fp64":
+        assert np.array_equal(bits(a), bits(b))
+    else:  # FMA contraction may differ between the kernels: an ulp of the largest value
+        assert np.max(np.abs(a - b)) <= 1e-6 * np.max(np.abs(b))
