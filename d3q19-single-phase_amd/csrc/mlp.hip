@@ -148,12 +148,12 @@ __global__ void __launch_bounds__(256) k_features(FeatArgs a)
 // over samples, so their operands have the hidden unit in the lane: those
 // pass through LDS (TS floats a sample: 16-byte stores, conflict-free reads).
 //
-// Bound: 69 matrix instructions of 64 cycles a group of 32 samples (a
-// gradient), 32 tanh and LDS traffic beside them; the samples (44 B each) stay
-// in cache.  Twenty iterations of 65 536 samples with the parameters' and a
-// prediction's download: 466 us, against 5 763 with one lane per sample on
-// the vector ALUs (48 us) and one thread per parameter adding 1 024 partials
-// (231 us an iteration).
+// Bound: 53 matrix instructions of 64 cycles and 16 of 32 (the gradient of W1,
+// whose ten columns and b1 fill a 16-wide product) a group of 32 samples, with
+// 32 tanh and the LDS traffic between them; the samples (44 B each) stay in
+// cache.  An iteration of 65 536 samples takes 15.2 us, 287 us with one lane
+// per sample on the vector ALUs (48 us) and one thread per parameter adding 1
+// 024 partials (231 us).
 constexpr int GROUP = 32;
 constexpr int MLP_WAVES = 4;             // waves per block
 constexpr int TS = 36;                   // LDS stride of a sample's 32 values
@@ -232,28 +232,41 @@ k_mlp_grad(const float *__restrict__ w, const float *__restrict__ feat, const fl
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, j = lane & 31, h = lane >> 5;
     float *const th1 = lds[wv], *const tg2 = th1 + GROUP * TS, *const tg1 = tg2 + GROUP * TS,
                  *const th3 = tg1 + GROUP * TS, *const tx = th3 + GROUP * TS;
+    const float inv_count = 1.0f / (float)count;
+    const uint32_t groups = (count + GROUP - 1) / GROUP, waves = gridDim.x * MLP_WAVES;
+    // the lane's sample of group g: half its inputs and the target, loaded one
+    // group ahead (the first with the weights)
+    auto sample = [&](uint32_t g, float (&x)[5], float &y) {
+        const uint32_t s = g * GROUP + j;
+        const bool valid = s < count; // also false past the last group
+#pragma unroll
+        for (int t = 0; t < 5; t++)
+            x[t] = valid ? feat[((uint64_t)first + s) * MLP_IN + 5 * h + t] : 0.0f;
+        y = valid ? target[(uint64_t)first + s] : 0.0f;
+    };
+    float xn[5], yn;
+    sample(blockIdx.x * MLP_WAVES + wv, xn, yn);
     MlpRegs n;
     n.load(w, j, h);
     float a2t[16]; // columns of W2: the transposed product of the back-propagation
 #pragma unroll
     for (int t = 0; t < 16; t++)
         a2t[t] = w[MLP_W2 + mfma_row(t, h) * MLP_H + j];
-    const float inv_count = 1.0f / (float)count;
-    const uint32_t groups = (count + GROUP - 1) / GROUP, waves = gridDim.x * MLP_WAVES;
 
-    mlp_float16 dw2, dw1;
+    mlp_float16 dw2;
+    mlp_float4 dw1[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
 #pragma unroll
     for (int r = 0; r < 16; r++)
-        dw2[r] = dw1[r] = 0.0f;
+        dw2[r] = 0.0f;
     float db2 = 0.0f, dw3 = 0.0f, db3 = 0.0f, loss = 0.0f;
     for (uint32_t g = blockIdx.x * MLP_WAVES + wv; g < groups; g += waves) {
-        const uint32_t s = g * GROUP + j;
-        const bool valid = s < count;
+        const bool valid = g * GROUP + j < count;
         float x[5];
 #pragma unroll
         for (int t = 0; t < 5; t++)
-            x[t] = valid ? feat[((uint64_t)first + s) * MLP_IN + 5 * h + t] : 0.0f;
-        const float y = valid ? target[(uint64_t)first + s] : 0.0f;
+            x[t] = xn[t];
+        const float y = yn;
+        sample(g + waves, xn, yn);
         mlp_float16 h1, h2;
         const float o = n.forward(x, h1, h2);
         const float err = mlp_nut(w, o) - y;
@@ -292,12 +305,19 @@ k_mlp_grad(const float *__restrict__ w, const float *__restrict__ feat, const fl
 #pragma unroll
         for (int t = 0; t < 16; t++) {
             const int k = 2 * t + h; // samples k of the group
-            const float ga = tg2[k * TS + j], gb = tg1[k * TS + j];
-            const float xb = j <= MLP_IN ? tx[k * TX + (j <= MLP_IN ? j : 0)] : 0.0f;
+            const float ga = tg2[k * TS + j];
             dw2 = __builtin_amdgcn_mfma_f32_32x32x2f32(ga, th1[k * TS + j], dw2, 0, 0, 0);
-            dw1 = __builtin_amdgcn_mfma_f32_32x32x2f32(gb, xb, dw1, 0, 0, 0);
             db2 += ga;
             dw3 += th3[k * TS + j];
+        }
+        // v_mfma_f32_16x16x4_f32: A[i][k], B[k][j] in lane 16 k + i, 16 k + j
+        const int c16 = lane & 15, k16 = lane >> 4;
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            const int k = 4 * t + k16;
+            const float xb = c16 <= MLP_IN ? tx[k * TX + (c16 <= MLP_IN ? c16 : 0)] : 0.0f;
+            dw1[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(tg1[k * TS + c16], xb, dw1[0], 0, 0, 0);
+            dw1[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(tg1[k * TS + 16 + c16], xb, dw1[1], 0, 0, 0);
         }
     }
 
@@ -316,10 +336,14 @@ k_mlp_grad(const float *__restrict__ w, const float *__restrict__ feat, const fl
     for (int r = 0; r < 16; r++) {
         const int i = mfma_row(r, h);
         out[MLP_W2 + i * MLP_H + j] = dw2[r];
-        if (j < MLP_IN)
-            out[MLP_W1 + i * MLP_IN + j] = dw1[r];
-        else if (j == MLP_IN)
-            out[MLP_B1 + i] = dw1[r];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++) { // D of 16x16: column lane % 16, row 4 (lane / 16) + q % 4
+        const int i = 16 * (q >> 2) + 4 * (lane >> 4) + (q & 3), c = lane & 15;
+        if (c < MLP_IN)
+            out[MLP_W1 + i * MLP_IN + c] = dw1[q >> 2][q & 3];
+        else if (c == MLP_IN)
+            out[MLP_B1 + i] = dw1[q >> 2][q & 3];
     }
     if (h == 0) {
         out[MLP_B2 + j] = db2;
@@ -465,12 +489,16 @@ hipError_t mlp_plane_targets(uint32_t lx, uint32_t ly, uint32_t lz, const float 
 }
 
 // Blocks for `count` samples: a wave for every group of 32 up to a block per
-// CU, beyond that several groups to a wave (65 536 samples: 13.3 us with 256
-// blocks, 14.0 us with 512, whose weights and partials cost more).
+// CU, beyond that several groups to a wave.  From eight groups a wave on, two
+// blocks per CU: their matrix and vector instructions overlap, which then
+// outweighs loading the weights and writing the partials twice (us an
+// iteration, one / two blocks: 65 536 samples 15.2 / 16.4, 131 072 22.5 / 23.3,
+// 262 144 36.8 / 35.5, 524 288 65.8 / 59.6).
 static uint32_t mlp_blocks(uint32_t count)
 {
     const uint32_t groups = (count + GROUP - 1) / GROUP;
-    return std::min<uint32_t>((groups + MLP_WAVES - 1) / MLP_WAVES, MLP_GRAD_BLOCKS);
+    const uint32_t most = groups >= 8 * MLP_WAVES * (MLP_GRAD_BLOCKS / 2) ? MLP_GRAD_BLOCKS : MLP_GRAD_BLOCKS / 2;
+    return std::min<uint32_t>((groups + MLP_WAVES - 1) / MLP_WAVES, most);
 }
 
 hipError_t mlp_grad(const float *w, const float *feat, const float *target, uint32_t first, uint32_t count,

@@ -41,9 +41,9 @@ struct MlpLaunch {
     static hipError_t filter(const FilterArgs &a, hipStream_t s);
 };
 
-// Blocks of a gradient pass: `partial` holds a gradient and a loss
+// Most blocks of a gradient pass: `partial` holds a gradient and a loss
 // (MLP_NPARAM + 1 floats) for each.
-constexpr uint32_t MLP_GRAD_BLOCKS = 256;
+constexpr uint32_t MLP_GRAD_BLOCKS = 512;
 
 hipError_t mlp_features(const FeatArgs &a, hipStream_t s);
 hipError_t mlp_grad(const float *w, const float *feat, const float *target, uint32_t first, uint32_t count,

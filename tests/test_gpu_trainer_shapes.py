@@ -1,6 +1,7 @@
 """GPU test of the trainer's gradient and prediction at the edges of their
-work split: a wave takes 32 samples at a time, a block four waves, and from
-65 536 samples on a wave takes several groups.
+work split: a wave takes 32 samples at a time, a block four waves, a wave takes
+several groups from 32 768 samples on, and from 262 113 there are two blocks
+per CU.
 
 Tolerance: the targets lie well above the predictions, so no parameter's sum
 over the samples loses digits by cancellation beyond its own size; a sample's
@@ -17,7 +18,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("first,count", [(0, 1), (3, 31), (0, 32), (5, 33), (0, 127), (1, 128), (7, 129), (0, 4097),
-                                         (11, 65535), (0, 65536), (2, 65537), (9, 131073), (0, 200001)])
+                                         (11, 65535), (0, 65536), (2, 65537), (9, 131073), (0, 200001),
+                                         (1, 262113), (0, 262144), (3, 300007)])
 def test_gradient_and_prediction_at_split_edges(first, count):
     rng = np.random.default_rng(count)
     p = d3q19.closure_params(seed=5)
