@@ -69,6 +69,7 @@ struct StepArgs {
     int runs;          // 1: modes 0 and 1 of FP64/FP32 take the vector-run kernel when lx allows
     int w32;           // 1: 32-bit pull offsets when N allows (step mode + 32, or + 64 between adjacent
                        // rows above 2^29 nodes in 2-byte storage); 2: + 64 wherever N <= 2^30
+    int to_kept;       // 1: dst is the lattice that single steps may keep in the last-level cache
     uint32_t nb;       // threads per block (set by Launch<P>::step)
     ForceSpec fc;      // mode bit 16: collision force (r.fx, r.fy, r.fz are then unused)
     ForceSpec fm;      // mode bit 16: force that the fused fields u = j + F/2 are formed with

@@ -57,6 +57,16 @@ __device__ __forceinline__ const typename Prec<P>::S *elem(const typename Prec<P
     return elem<P>(const_cast<typename Prec<P>::S *>(row), node);
 }
 
+// A load of one population, non-temporal when NT.
+template <int NT, typename S>
+__device__ __forceinline__ S load_pop(const S *p)
+{
+    if constexpr (NT != 0)
+        return __builtin_nontemporal_load(p);
+    else
+        return *p;
+}
+
 // F_I(x): streamed population of direction I at node x; N is the population
 // stride Geom::S here and in the functions below.  The bounce-back
 // choice is made with masks, not branches, so every load issues back to back.
@@ -72,7 +82,7 @@ constexpr uint64_t W32_MAX_N = 1ull << 29;
 constexpr uint64_t w32_max_n(int P) { return half_storage(P) ? W32_MAX_N : (P == 1 ? (1ull << 28) : 0); }
 constexpr uint64_t W32_ADJ_MAX_N = 1ull << 30;
 
-template <int P, int I, int W32 = 0>
+template <int P, int I, int W32 = 0, int NT = 0>
 __device__ __forceinline__ typename Prec<P>::T pull(const typename Prec<P>::S *__restrict__ L, uint64_t N,
                                                     const Nbr &b)
 {
@@ -85,7 +95,8 @@ __device__ __forceinline__ typename Prec<P>::T pull(const typename Prec<P>::S *_
         const uint32_t node = w ? b.n : src_of<I>(b);
         if constexpr (P == 0) {
             // memory-bound: this form measured 1.4 % faster than the one below
-            return Prec<P>::template to_T<I>(L[(w ? (uint64_t)OPP[I] * N : (uint64_t)I * N) + node]);
+            return Prec<P>::template to_T<I>(
+                load_pop<NT>(L + ((w ? (uint64_t)OPP[I] * N : (uint64_t)I * N) + node)));
         } else if constexpr (W32 == 1 || (W32 == 2 && (OPP[I] - I == 1 || I - OPP[I] == 1))) {
             static_assert(half_storage(P) || P == 1, "32-bit pull offsets are for FP32 and 2-byte storage");
             constexpr int M = I < OPP[I] ? I : OPP[I];
@@ -101,7 +112,7 @@ __device__ __forceinline__ typename Prec<P>::T pull(const typename Prec<P>::S *_
             using S = typename Prec<P>::S;
             const uint32_t off = w ? b.n + d_o : src_of<I>(b) + d_i;
             return Prec<P>::template to_T<I>(
-                *(const S *)((const char *)(L + row_m) + off * (uint32_t)sizeof(S)));
+                load_pop<NT>((const S *)((const char *)(L + row_m) + off * (uint32_t)sizeof(S))));
         } else {
             uint64_t row_i = (uint64_t)I * N, row_o = (uint64_t)OPP[I] * N;
             // opaque to the optimiser, which would otherwise turn the select
@@ -111,25 +122,25 @@ __device__ __forceinline__ typename Prec<P>::T pull(const typename Prec<P>::S *_
             // passes the kernel argument Geom::S.
             __asm__("" : "+s"(row_i));
             __asm__("" : "+s"(row_o));
-            return Prec<P>::template to_T<I>(*elem<P>(L + (w ? row_o : row_i), node));
+            return Prec<P>::template to_T<I>(load_pop<NT>(elem<P>(L + (w ? row_o : row_i), node)));
         }
     } else {
-        return Prec<P>::template to_T<I>(*elem<P>(L + (uint64_t)I * N, src_of<I>(b)));
+        return Prec<P>::template to_T<I>(load_pop<NT>(elem<P>(L + (uint64_t)I * N, src_of<I>(b))));
     }
 }
 
-template <int P, int W32, int... Is>
+template <int P, int W32, int NT, int... Is>
 __device__ __forceinline__ void pull_all_impl(const typename Prec<P>::S *__restrict__ L, uint64_t N, const Nbr &b,
                                               typename Prec<P>::T (&f)[19], std::integer_sequence<int, Is...>)
 {
-    ((f[Is] = pull<P, Is, W32>(L, N, b)), ...);
+    ((f[Is] = pull<P, Is, W32, NT>(L, N, b)), ...);
 }
 
-template <int P, int W32 = 0>
+template <int P, int W32 = 0, int NT = 0>
 __device__ __forceinline__ void pull_all(const typename Prec<P>::S *__restrict__ L, uint64_t N, const Nbr &b,
                                          typename Prec<P>::T (&f)[19])
 {
-    pull_all_impl<P, W32>(L, N, b, f, std::make_integer_sequence<int, 19>{});
+    pull_all_impl<P, W32, NT>(L, N, b, f, std::make_integer_sequence<int, 19>{});
 }
 
 template <int P, int... Is>
@@ -273,7 +284,8 @@ __device__ __forceinline__ uint32_t node_index(const Geom &g, uint32_t nb)
 // N <= 2^28): the pulls with c_x != 0 take 32-bit offsets (pull<P, I, 1>);
 // the same loads, fewer instructions.  MODE + 64: 2-byte storage with
 // N <= 2^30: the pulls between adjacent rows only (pull<P, I, 2>).
-// MODE + 128: cached instead of non-temporal stores.
+// MODE + 128: cached instead of non-temporal stores; MODE + 256:
+// non-temporal loads (step_policy).
 template <int P, int MODE>
 __device__ __forceinline__ void step_node(const StepArgs &a)
 {
@@ -301,7 +313,7 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
     // the 19 loads issue first; the closure's weights are staged while they
     // are in flight
     T f[19];
-    pull_all<P, (MODE & 32) != 0 ? 1 : ((MODE & 64) != 0 ? 2 : 0)>(src, a.g.S, b, f);
+    pull_all<P, (MODE & 32) != 0 ? 1 : ((MODE & 64) != 0 ? 2 : 0), (MODE & 256) != 0>(src, a.g.S, b, f);
     __shared__ __attribute__((aligned(16))) _Float16 wl[WAVE ? MLP_LDS : 8];
     if constexpr (WAVE) {
         mlp_stage(a.mlp, wl, threadIdx.x, a.nb);
@@ -1315,15 +1327,38 @@ static inline uint32_t step_threads(uint64_t N, uint32_t largest)
     return nb;
 }
 
-// 2-byte storage stores through the cache while the last-level cache holds
-// both lattices: a wave's non-temporal store of one population is a single
-// 128-byte line, and a step over a resident lattice then waits for memory
-// (FP16, 46 MB 97x150x83: 29.3 us non-temporal, 19.8 us cached; 70 MB
-// 96x192x100: 33.2 / 27.1 us; 125 MB 109x201x150: 64.0 / 44.4 us; 269 MB
-// 96x384x192: 101 / 107 us; 717 MB 271 / 276 us).  A branch on a kernel
-// argument instead of the step mode cost the large lattices 2.5 %.  FP64 and
-// FP32 measured no difference.
-constexpr uint64_t CACHED_STORE_BYTES = 256000000ull;
+// How a single step uses the caches, by the bytes of a lattice.
+// * Both lattices fit into the 256 MB last-level cache: stores go through it
+//   (mode + 128), and no traffic leaves it.
+// * One lattice fits (FP64, FP32): the handle's second one is kept there.  The
+//   step that writes it reads the other with non-temporal loads and stores
+//   through the cache (mode + 384); the next one reads it back from there and
+//   sends its own stores past the cache.  Memory carries half the traffic.
+//   2-byte storage, issue-bound at that size, measured no difference.
+// * Larger: non-temporal stores, and so too where both lattices just fill the
+//   8 XCDs' L2s (32 MB), whose dirty lines a step's end would write back.
+// us per step, FP64 non-temporal / cached stores: 2 MB 4.3 / 4.0, 10 MB 5.4 /
+// 5.7, 16 MB 8.0 / 9.6, 27 MB 13.7 / 11.5, 53 MB 23.4 / 19.7, 100 MB 38.6 /
+// 31.3; and one lattice kept: 156 MB 59.4 / 54.1 / 49.3, 179 MB 71.1 / 72.0 /
+// 56.8, 239 MB 89.5 / 92.4 / 77.9, 280 MB 103.9 / 107.3 / 98.9, 366 MB 137 /
+// 140 / 148.  FP32: 13 MB 7.3 / 8.0, 17 MB 9.2 / 8.5, 27 MB 13.2 / 11.0, 90 MB
+// 38.2 / 28.3, 119 MB 45.1 / 39.9; 140 MB 57.3 / 54.9 / 47.2, 183 MB 73.8 / 74
+// / 65.1, 239 MB 90.7 / 92 / 77.7, 374 MB 136 / 141 / 155.  FP16: 9 MB 6.6 /
+// 7.5, 46 MB 29.3 / 19.8, 125 MB 64.0 / 44.4, 269 MB 101 / 107.  A branch on a
+// kernel argument instead of the step mode cost large FP16 lattices 2.5 %.
+constexpr uint64_t L2S_LOW_BYTES = 12000000ull, L2S_BYTES = 33500000ull;
+constexpr uint64_t LLC_BYTES = 260000000ull, LLC_ONE_BYTES = 300000000ull;
+enum StepPolicy { POLICY_STREAM = 0, POLICY_CACHED = 1, POLICY_FILL = 2 };
+template <int P>
+static inline StepPolicy step_policy(const StepArgs &a)
+{
+    const uint64_t lattice = 19 * a.g.S * sizeof(typename Prec<P>::S);
+    if (2 * lattice <= LLC_BYTES)
+        return 2 * lattice > L2S_LOW_BYTES && 2 * lattice < L2S_BYTES ? POLICY_STREAM : POLICY_CACHED;
+    if (!half_storage(P) && a.to_kept && lattice <= LLC_ONE_BYTES)
+        return POLICY_FILL;
+    return POLICY_STREAM;
+}
 
 template <int P>
 hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
@@ -1344,8 +1379,6 @@ hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
         hipLaunchKernelGGL(kernel, dim3((uint32_t)((a.g.N + a.nb - 1) / a.nb)), dim3(a.nb), 0, s, a);
         return hipGetLastError();
     };
-#define STEP_CASE(MODE) \
-    case (MODE) & 31: return launch(k_step<P, MODE>, step_block<P, MODE>())
     // the closure's blocks stage the weights: fewer, whole blocks also on
     // small grids (43 k nodes: 6.8 us with 256 threads, 8.3 us with 128)
     auto launch_closure = [&](auto kernel) {
@@ -1353,6 +1386,17 @@ hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
         hipLaunchKernelGGL(kernel, dim3((uint32_t)((a.g.N + a.nb - 1) / a.nb)), dim3(a.nb), 0, s, a);
         return hipGetLastError();
     };
+    const StepPolicy policy = step_policy<P>(a);
+#define STEP_CASE(MODE) \
+    case (MODE) & 31: return launch(k_step<P, MODE>, step_block<P, MODE>())
+#define POLICY_CASE(MODE)                                                                      \
+    case (MODE) & 31:                                                                          \
+        if constexpr (!half_storage(P)) {                                                      \
+            if (policy == POLICY_FILL)                                                         \
+                return launch(k_step<P, (MODE) + 384>, step_block<P, 128>());                  \
+        }                                                                                      \
+        return policy == POLICY_CACHED ? launch(k_step<P, (MODE) + 128>, step_block<P, 128>()) \
+                                       : launch(k_step<P, MODE>, step_block<P, MODE>())
 #define CLOSURE_CASE(MODE) \
     case (MODE) & 31: return launch_closure(k_step_closure<P, MODE>)
     if constexpr (half_storage(P) || P == 1) {
@@ -1363,21 +1407,11 @@ hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
         // 2-byte storage
         if (a.w32 == 1 && a.g.S <= w32_max_n(P)) {
             if constexpr (half_storage(P)) {
-                if (2 * 19 * a.g.S * sizeof(typename Prec<P>::S) <= CACHED_STORE_BYTES) {
-                    switch (mode) {
-                        STEP_CASE(160);
-                        STEP_CASE(161);
-                        STEP_CASE(164);
-                        STEP_CASE(176);
-                    default:
-                        break;
-                    }
-                }
                 switch (mode) {
-                    STEP_CASE(32);
-                    STEP_CASE(33);
-                    STEP_CASE(36);
-                    STEP_CASE(48);
+                    POLICY_CASE(32);
+                    POLICY_CASE(33);
+                    POLICY_CASE(36);
+                    POLICY_CASE(48);
                 default:
                     break;
                 }
@@ -1414,19 +1448,36 @@ hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
             break;
         }
     }
-    switch (mode) {
-        STEP_CASE(0);
-        STEP_CASE(1);
-        STEP_CASE(2);
-        STEP_CASE(4);
-        STEP_CASE(5);
-        STEP_CASE(6);
-        STEP_CASE(16);
-        STEP_CASE(17);
-        STEP_CASE(18);
-    default:
-        return hipErrorInvalidValue;
+    if constexpr (!half_storage(P)) {
+        switch (mode) {
+            POLICY_CASE(0);
+            POLICY_CASE(1);
+            POLICY_CASE(2);
+            POLICY_CASE(4);
+            POLICY_CASE(5);
+            POLICY_CASE(6);
+            POLICY_CASE(16);
+            POLICY_CASE(17);
+            POLICY_CASE(18);
+        default:
+            return hipErrorInvalidValue;
+        }
+    } else {
+        switch (mode) {
+            STEP_CASE(0);
+            STEP_CASE(1);
+            STEP_CASE(2);
+            STEP_CASE(4);
+            STEP_CASE(5);
+            STEP_CASE(6);
+            STEP_CASE(16);
+            STEP_CASE(17);
+            STEP_CASE(18);
+        default:
+            return hipErrorInvalidValue;
+        }
     }
+#undef POLICY_CASE
 #undef STEP_CASE
 #undef CLOSURE_CASE
 }

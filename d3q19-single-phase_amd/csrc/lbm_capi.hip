@@ -379,6 +379,7 @@ int launch_step(lbm_channel *h)
     a.yscale = h->mlp_yscale;
     a.runs = h->runs;
     a.w32 = h->w32;
+    a.to_kept = h->cur == 0;
     if (h->mlp) {
         if (mode & 3) // the closure runs with fused fields only
             return fail(LBM_ERR_STATE, "collision: the learned closure needs fields from macrovar");
