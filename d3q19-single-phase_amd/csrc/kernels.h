@@ -73,6 +73,11 @@ struct StepArgs {
     uint32_t nb;       // threads per block (set by Launch<P>::step)
     ForceSpec fc;      // mode bit 16: collision force (r.fx, r.fy, r.fz are then unused)
     ForceSpec fm;      // mode bit 16: force that the fused fields u = j + F/2 are formed with
+    // mode 2 with errbits set: rhoupdat first, rho stored to rho_out; nothing is
+    // stored when stop is given and *stop is not 0
+    double *rho_out;
+    unsigned long long *errbits;
+    const unsigned long long *stop;
 };
 
 // Slots of rhoupdat's maximum, a cache line apart.

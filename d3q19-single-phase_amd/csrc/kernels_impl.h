@@ -267,6 +267,32 @@ __device__ __forceinline__ uint32_t node_index(const Geom &g, uint32_t nb)
     return blk * nb + threadIdx.x;
 }
 
+// rhoupdat's max |rho_new - rho_old| over a block of nb threads (err >= 0 or
+// NaN in each of them) into one of ERR_SLOTS words: on a single word the
+// blocks' atomics took turns (64x192x96 in FP64, 4 608 blocks: 63 us with one
+// word, 36 us with 64).  All on the bit patterns: non-negative doubles order
+// like their unsigned bit patterns, and a NaN with the sign cleared (fabs)
+// orders above +inf, so a NaN anywhere becomes the result instead of being
+// dropped as fmax would drop it.
+__device__ __forceinline__ void block_err_max(double err, uint32_t nb, unsigned long long *errbits)
+{
+    unsigned long long u = (unsigned long long)__double_as_longlong(err);
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long v = (unsigned long long)__shfl_xor((long long)u, o);
+        u = v > u ? v : u;
+    }
+    __shared__ unsigned long long wmax[16];
+    if ((threadIdx.x & 63) == 0)
+        wmax[threadIdx.x >> 6] = u;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long m = wmax[0];
+        for (uint32_t w = 1; w < nb / 64; w++)
+            m = wmax[w] > m ? wmax[w] : m;
+        atomicMax(errbits + (blockIdx.x % ERR_SLOTS) * ERR_STRIDE, m);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // One time step: gather F_k, macroscopic fields, MRT collision, store P_{k+1}.
 // MODE 0: rho, u from F_k (macrovar fused); MODE 1: same with rho - rho_off
@@ -286,6 +312,10 @@ __device__ __forceinline__ uint32_t node_index(const Geom &g, uint32_t nb)
 // N <= 2^30: the pulls between adjacent rows only (pull<P, I, 2>).
 // MODE + 128: cached instead of non-temporal stores; MODE + 256:
 // non-temporal loads (step_policy).
+// MODE 2 + 512: an iteration of the pre-relaxation, rhoupdat and the step in
+// one pass (rho is set to sum F, its largest change goes to errbits), and
+// without effect once *stop is set.  The pulls of the step are the ones that
+// rhoupdat needs: apart, both read the lattice.
 template <int P, int MODE>
 __device__ __forceinline__ void step_node(const StepArgs &a)
 {
@@ -294,10 +324,10 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
     // The closure's network runs on the matrix cores over whole waves: there
     // every lane stays to the end (a lane past the lattice works on the last
     // node, a particle node on its own slots) and only active lanes store.
-    constexpr bool WAVE = (MODE & 8) != 0;
+    constexpr bool WAVE = (MODE & 8) != 0, RHO = (MODE & 512) != 0;
     const uint32_t n0 = node_index(a.g, a.nb);
     bool active = n0 < a.g.N;
-    if constexpr (!WAVE) {
+    if constexpr (!WAVE && !RHO) {
         if (!active)
             return;
     }
@@ -341,7 +371,17 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
 
     T rho9, ux9, uy9, uz9;
     T jx = T(0), jy = T(0), jz = T(0);
-    if constexpr ((MODE & 3) == 2) {
+    double err = 0.0, rnew = 0.0;
+    if constexpr (RHO) {
+        static_assert((MODE & 31) == 2, "the pre-relaxation steps with stored fields");
+        active = active && !(a.stop && *a.stop);
+        macro_sums(f, rho9, jx, jy, jz);
+        rnew = (double)rho9;
+        err = active ? fabs(rnew - a.rho[n]) : 0.0;
+        ux9 = (T)a.ux[n];
+        uy9 = (T)a.uy[n];
+        uz9 = (T)a.uz[n];
+    } else if constexpr ((MODE & 3) == 2) {
         rho9 = (T)a.rho[n];
         ux9 = (T)a.ux[n];
         uy9 = (T)a.uy[n];
@@ -373,7 +413,7 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
             djz = uz9 - (jz + r.fz / T(2.));
         }
         if constexpr ((MODE & 3) == 2) {
-            T rf, jx, jy, jz;
+            T rf;
             macro_sums(f, rf, jx, jy, jz);
             drho = rho9 - rf;
             djx = ux9 - (jx + r.fx / T(2.));
@@ -389,10 +429,14 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
             mrt_collide_delta(f, rho9, ux9, uy9, uz9, drho, djx, djy, djz, r);
         }
     }
-    if constexpr (WAVE || (MODE & 4) != 0) {
+    if constexpr (RHO)
+        block_err_max(err, a.nb, a.errbits);
+    if constexpr (WAVE || RHO || (MODE & 4) != 0) {
         if (!active)
             return;
     }
+    if constexpr (RHO)
+        a.rho_out[n] = rnew;
     if constexpr ((MODE & 128) != 0)
         store_all_cached<P>(dst, a.g.S, n, f, std::make_integer_sequence<int, 19>{});
     else
@@ -729,9 +773,7 @@ __global__ void __launch_bounds__(BLOCK) k_step_run(StepArgs a)
 
 // macrovar / rhoupdat / materialisation of the fields of lattice L.
 // WHAT 0: rho, ux, uy, uz = macrovar(F) with rho - rho_off.
-// WHAT 1: rho = sum F (rhoupdat); max |rho_new - rho_old| into errbits, one of
-// ERR_SLOTS per block: on a single word the blocks' atomics took turns (64x192x96
-// in FP64, 4 608 blocks: 63 us with one word, 36 us with 64).
+// WHAT 1: rho = sum F (rhoupdat); max |rho_new - rho_old| into errbits.
 template <int P, int WHAT>
 __global__ void __launch_bounds__(BLOCK) k_macro(MacroArgs a)
 {
@@ -761,26 +803,7 @@ __global__ void __launch_bounds__(BLOCK) k_macro(MacroArgs a)
         }
     }
     if constexpr (WHAT == 1) {
-        // max over the block, then one atomic per block on its slot, all on the bit
-        // patterns: non-negative doubles order like their unsigned bit
-        // patterns, and a NaN with the sign cleared (fabs) orders above
-        // +inf, so a NaN anywhere becomes the result instead of being
-        // dropped as fmax would drop it
-        unsigned long long u = (unsigned long long)__double_as_longlong(err);
-        for (int o = 32; o > 0; o >>= 1) {
-            const unsigned long long v = (unsigned long long)__shfl_xor((long long)u, o);
-            u = v > u ? v : u;
-        }
-        __shared__ unsigned long long wmax[BLOCK / 64];
-        if ((threadIdx.x & 63) == 0)
-            wmax[threadIdx.x >> 6] = u;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            unsigned long long m = wmax[0];
-            for (int w = 1; w < BLOCK / 64; w++)
-                m = wmax[w] > m ? wmax[w] : m;
-            atomicMax(a.errbits + (blockIdx.x % ERR_SLOTS) * ERR_STRIDE, m);
-        }
+        block_err_max(err, BLOCK, a.errbits);
     }
 }
 
@@ -1399,6 +1422,11 @@ hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
                                        : launch(k_step<P, MODE>, step_block<P, MODE>())
 #define CLOSURE_CASE(MODE) \
     case (MODE) & 31: return launch_closure(k_step_closure<P, MODE>)
+    if (mode == 2 && a.errbits) {
+        return policy == POLICY_CACHED ? launch(k_step<P, 642>, step_block<P, 128>())
+               : policy == POLICY_FILL && !half_storage(P) ? launch(k_step<P, 898>, step_block<P, 128>())
+                                                           : launch(k_step<P, 514>, step_block<P, 514>());
+    }
     if constexpr (half_storage(P) || P == 1) {
         // 32-bit pull offsets where the lattice allows them: the main loop's
         // modes in 2-byte storage (FP16 1.8-2.5 % faster, FP16C 2.7-2.9 %, on

@@ -70,6 +70,7 @@ _SIGS = {
     "lbm_set_velocity_separable": [_H, ctypes.c_int, _D, _D, _D],
     "lbm_collision_mrt": [_H],
     "lbm_macrovar": [_H, _D, _D, _D, _D],
+    "lbm_prerelax": [_H, ctypes.c_double, ctypes.c_int, ctypes.POINTER(ctypes.c_int), _D],
     "lbm_rhoupdat": [_H, ctypes.POINTER(ctypes.c_double)],
     "lbm_avedensity": [_H, ctypes.POINTER(ctypes.c_double)],
     "lbm_run": [_H, ctypes.c_int],
@@ -352,13 +353,14 @@ class Channel:
     def prerelax(self, rhoepsl=1.0e-5, maxiter=15000):
         """Pre-relaxation loop of Channel-Flow/main.f90:70-90 (u held fixed).
         Returns (iterations, last max|drho|)."""
-        istep = 0
+        istep, errs, done = 0, np.empty(64), ctypes.c_int()
         while True:
-            err = self.rhoupdat()
-            self.collision_MRT()
-            if err <= rhoepsl or istep > maxiter:
-                return istep, err
-            istep += 1
+            n = int(min(errs.size, max(1, maxiter + 2 - istep)))
+            _call("lbm_prerelax", self._h, rhoepsl, n, ctypes.byref(done), _ptr(errs))
+            istep += done.value
+            err = float(errs[done.value - 1])
+            if err <= rhoepsl or istep - 1 > maxiter:
+                return istep - 1, err
 
     def mass(self):
         v = ctypes.c_double()

@@ -7,6 +7,7 @@
 !   collision_MRT  -> lbm_collision_mrt   (collision.f90:24-273, exchange :281-372)
 !   macrovar       -> lbm_macrovar        (collision.f90:378-463)
 !   rhoupdat       -> lbm_rhoupdat        (collision.f90:469-480)
+!   prerelax       -> lbm_prerelax        (the loop of main.f90:70-90)
 !   avedensity     -> lbm_avedensity      (collision.f90:487-513)
 !   FORCING        -> lbm_set_force       (collision.f90:515-527)
 !   FORCINGP       -> lbm_forcingp        (collision.f90:529-602)
@@ -86,6 +87,19 @@
       implicit none
       call lbm_check(lbm_rhoupdat(lbm, rhoerrmax), 'rhoupdat')
       end subroutine rhoupdat
+
+      ! Up to niter iterations of the pre-relaxation loop (rhoupdat, then
+      ! collision_MRT; main.f90:70-90), ending at the convergence limit rhoepsl:
+      ! their number and each one's max |drho|.
+      subroutine prerelax(niter, done, errs)
+      use channel_vars
+      implicit none
+      integer, intent(in) :: niter
+      integer, intent(out) :: done
+      real(8), intent(out) :: errs(niter)
+      call lbm_check(lbm_prerelax(lbm, rhoepsl, niter, done, errs), 'prerelax')
+      rhoerrmax = errs(done)
+      end subroutine prerelax
 
       subroutine avedensity
       use channel_vars

@@ -104,6 +104,15 @@
           type(c_ptr), value :: h, rho, ux, uy, uz
         end function
 
+        integer(c_int) function lbm_prerelax(h, rhoepsl, niter, done, rhoerrmax) bind(C, name="lbm_prerelax")
+          import :: c_int, c_ptr, c_double
+          type(c_ptr), value :: h
+          real(c_double), value :: rhoepsl
+          integer(c_int), value :: niter
+          integer(c_int), intent(out) :: done
+          real(c_double), intent(out) :: rhoerrmax(*)
+        end function
+
         integer(c_int) function lbm_rhoupdat(h, rhoerrmax) bind(C, name="lbm_rhoupdat")
           import :: c_int, c_ptr, c_double
           type(c_ptr), value :: h

@@ -12,7 +12,8 @@
       character(len=300) :: nml
       integer :: u, ios, nrun
       integer(8) :: t0, t1, rate
-      real(8) :: time_max, mass
+      real(8) :: time_max, mass, errs(64)
+      integer :: i, ndone
 
       nml = 'channel.nml'
       if (command_argument_count() >= 1) call get_command_argument(1, nml)
@@ -39,9 +40,11 @@
           call initpop
           istep = 0
           do
-            call rhoupdat
-            call collision_MRT
-            write(*,*) istep, rhoerrmax
+            call prerelax(min(size(errs), 15002 - istep), ndone, errs)
+            do i = 1, ndone
+              write(*,*) istep + i - 1, errs(i)
+            end do
+            istep = istep + ndone - 1
             if (rhoerrmax <= rhoepsl .or. istep > 15000) then
               write(*,*) 'final relaxation => ', istep, rhoerrmax
               exit
