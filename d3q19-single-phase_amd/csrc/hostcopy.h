@@ -3,21 +3,23 @@
 //
 // A pageable hipMemcpyAsync is staged by one thread inside the runtime (17
 // GB/s down, 29 GB/s up here, 4 GB/s down into pages not touched yet).  Here
-// the array moves in slices: the copy engine fills or drains one pinned slot
-// while host threads copy others to or from the array, so the link's rate is
-// the bound (45 GB/s with 4 MiB slices, 20 us of each slice being the copy's
-// start; 512 MB down: 31 ms before, 11.5 ms).  Two threads keep up with the
-// link; more share the page faults of a new array (184 MB: 46 ms before,
-// 13 ms).
+// the array moves in slices: a kernel fills or drains one pinned slot over
+// the link while host threads copy others to or from the array, so the link's
+// rate is the bound: 50 GB/s down and 51 up, 45 and 41 when the copy engine
+// moved the slices (kernels that make the values, macrovar and the checkpoint,
+// store into the slots themselves).  1.81 GB of fields: 40.9 -> 36.2 ms; 11.2
+// MB 480 -> 340 us.
+// Two threads keep up with the link; more share the page faults of a new array.
 //
-// The pinned slots belong to the process, not to a handle: HOST_WORKERS x
-// HOST_DEPTH slots of HOST_SLICE bytes (48 MiB), allocated by the first large
-// copy and freed with the last handle (host_pool_retain / release).  One copy
-// uses them at a time; a copy that finds them taken by another thread, or
+// The pinned slots belong to the process, not to a handle: up to HOST_WORKERS
+// x HOST_DEPTH slots of HOST_SLICE bytes (48 MiB), each allocated by the first
+// copy that needs it and freed with the last handle (retain / release).  One
+// copy uses them at a time; a copy that finds them taken by another thread, or
 // cannot allocate them, goes the plain way.
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 #include <string.h>
 
 #include <algorithm>
@@ -29,7 +31,23 @@ namespace d3q19 {
 
 constexpr int HOST_WORKERS = 6, HOST_DEPTH = 2;
 constexpr size_t HOST_SLICE = 4u << 20;
-constexpr size_t HOST_MIN = 1u << 20; // smaller copies go the plain way
+constexpr size_t HOST_MIN = 64u << 10; // smaller copies go the plain way
+
+// Bytes of a slice of a copy of `total` bytes: downloads in smaller slices
+// below 64 MiB, so that the host's part overlaps the link's (us with 1 / 2 / 4
+// MiB: 2.1 MB of fields 87 / 104 / 106, 11.2 MB 381 / 416 / 473, 53 MB of
+// populations 1 560 / 1 411 / 1 736); uploads in whole ones, whose kernels
+// need the waves to hide the link's latency (53 MB 1 651 / 1 253 / 1 162).
+inline size_t host_slice(size_t total, bool down)
+{
+    return !down || total >= 64u << 20 ? HOST_SLICE : total >= 16u << 20 ? HOST_SLICE / 2 : HOST_SLICE / 4;
+}
+
+// Threads for a copy of `total` bytes: one (no thread is started) below 8 MiB.
+inline int host_workers(size_t total)
+{
+    return total < 8u << 20 ? 1 : (int)std::min<size_t>(HOST_WORKERS, 2 + (total >> 24));
+}
 
 struct HostPool {
     std::mutex mu;      // held by the copy that uses the slots
@@ -48,12 +66,13 @@ struct HostPool {
         }
         device = -1;
     }
-    // Slots and this device's events (called with mu held).
-    bool ready(int dev)
+    // The slots of `workers` threads and this device's events (called with mu
+    // held).
+    bool ready(int dev, int workers)
     {
-        for (char *&p : slot)
-            if (!p && hipHostMalloc((void **)&p, HOST_SLICE, hipHostMallocPortable) != hipSuccess) {
-                p = nullptr;
+        for (int k = 0; k < workers * HOST_DEPTH; k++)
+            if (!slot[k] && hipHostMalloc((void **)&slot[k], HOST_SLICE, hipHostMallocPortable) != hipSuccess) {
+                slot[k] = nullptr;
                 (void)hipGetLastError();
                 return false;
             }
@@ -197,10 +216,47 @@ hipError_t host_slices_in(HostPool &pool, int device, hipStream_t s, size_t n, i
     return err.load() != (int)hipSuccess ? (hipError_t)err.load() : e;
 }
 
-// Threads for a copy of `bytes`: one (no thread is started) below 8 MiB.
-inline int host_workers(size_t bytes)
+// Copy between device memory and a pinned slot, 16 bytes a lane and four in
+// flight; `tail` bytes (below 16) follow the n vectors.
+typedef uint32_t LinkVec __attribute__((ext_vector_type(4)));
+constexpr int LINK_BLOCK = 256, LINK_UNROLL = 4;
+// blocks of a copy, measured in 4 MiB pieces (GB/s with 8 / 32 / 128 / 512
+// blocks): down 48.3 / 53.3 / 54.7 / 54.9, up 54.7 / 54.5 / 49.1 / 41.4, where
+// more reads in flight than the link takes get in each other's way.  The copy
+// engine: 50.3 either way.
+constexpr size_t LINK_DOWN_BLOCKS = 256, LINK_UP_BLOCKS = 32;
+
+static __global__ void __launch_bounds__(LINK_BLOCK) k_link_copy(const LinkVec *__restrict__ src, LinkVec *__restrict__ dst,
+                                                                 size_t n, uint32_t tail)
 {
-    return (int)std::max<size_t>(1, std::min<size_t>(HOST_WORKERS, bytes / HOST_SLICE / 2));
+    constexpr size_t STRIDE = LINK_BLOCK * LINK_UNROLL;
+    for (size_t i = blockIdx.x * STRIDE + threadIdx.x; i < n; i += gridDim.x * STRIDE) {
+        LinkVec v[LINK_UNROLL];
+#pragma unroll
+        for (int k = 0; k < LINK_UNROLL; k++)
+            if (i + k * LINK_BLOCK < n)
+                v[k] = __builtin_nontemporal_load(src + i + k * LINK_BLOCK);
+#pragma unroll
+        for (int k = 0; k < LINK_UNROLL; k++)
+            if (i + k * LINK_BLOCK < n)
+                dst[i + k * LINK_BLOCK] = v[k];
+    }
+    if (blockIdx.x == 0 && threadIdx.x < tail)
+        ((char *)(dst + n))[threadIdx.x] = ((const char *)(src + n))[threadIdx.x];
+}
+
+// One slice between device memory and a pinned slot; device addresses that are
+// not on 16 bytes take the runtime's copy.
+inline hipError_t link_copy(void *dst, const void *src, size_t bytes, bool down, hipStream_t s)
+{
+    if (((uintptr_t)dst | (uintptr_t)src) % sizeof(LinkVec))
+        return hipMemcpyAsync(dst, src, bytes, down ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, s);
+    const size_t n = bytes / sizeof(LinkVec), per = LINK_BLOCK * LINK_UNROLL;
+    const unsigned grid =
+        (unsigned)std::max<size_t>(1, std::min<size_t>((n + per - 1) / per, down ? LINK_DOWN_BLOCKS : LINK_UP_BLOCKS));
+    hipLaunchKernelGGL(k_link_copy, dim3(grid), dim3(LINK_BLOCK), 0, s, (const LinkVec *)src, (LinkVec *)dst, n,
+                       (uint32_t)(bytes % sizeof(LinkVec)));
+    return hipGetLastError();
 }
 
 // One contiguous part of a copy; a null host pointer is skipped.
@@ -225,7 +281,8 @@ inline hipError_t host_copy(int device, hipStream_t s, const HostPart *parts, in
         if (e != hipSuccess)
             return e;
     }
-    if (total < HOST_MIN || !lock.try_lock() || !pool.ready(device)) {
+    const int workers = host_workers(total);
+    if (total < HOST_MIN || !lock.try_lock() || !pool.ready(device, workers)) {
         for (int p = 0; p < nparts; p++)
             if (parts[p].host) {
                 const hipError_t e =
@@ -236,9 +293,7 @@ inline hipError_t host_copy(int device, hipStream_t s, const HostPart *parts, in
             }
         return hipStreamSynchronize(s);
     }
-    // copies below two slices a worker in smaller ones, so that the host's
-    // part overlaps the link's
-    const size_t slice = total < 2 * HOST_SLICE ? HOST_SLICE / 4 : HOST_SLICE;
+    const size_t slice = host_slice(total, down);
     size_t n = 0;
     for (int p = 0; p < nparts; p++)
         n += parts[p].host ? (parts[p].bytes + slice - 1) / slice : 0;
@@ -257,11 +312,11 @@ inline hipError_t host_copy(int device, hipStream_t s, const HostPart *parts, in
     };
     if (down)
         return host_slices_out(
-            pool, device, s, n, host_workers(total),
+            pool, device, s, n, workers,
             [&](size_t k, int, char *pinned) {
                 char *host, *dev;
                 const size_t b = find(k, host, dev);
-                return hipMemcpyAsync(pinned, dev, b, hipMemcpyDeviceToHost, s);
+                return link_copy(pinned, dev, b, true, s);
             },
             [&](size_t k, const char *pinned) {
                 char *host, *dev;
@@ -269,7 +324,7 @@ inline hipError_t host_copy(int device, hipStream_t s, const HostPart *parts, in
                 memcpy(host, pinned, b);
             });
     return host_slices_in(
-        pool, device, s, n, host_workers(total),
+        pool, device, s, n, workers,
         [&](size_t k, char *pinned) {
             char *host, *dev;
             const size_t b = find(k, host, dev);
@@ -278,7 +333,7 @@ inline hipError_t host_copy(int device, hipStream_t s, const HostPart *parts, in
         [&](size_t k, int, const char *pinned) {
             char *host, *dev;
             const size_t b = find(k, host, dev);
-            return hipMemcpyAsync(dev, pinned, b, hipMemcpyHostToDevice, s);
+            return link_copy(dev, pinned, b, false, s);
         });
 }
 

@@ -86,7 +86,8 @@ constexpr uint32_t ERR_SLOTS = 64, ERR_STRIDE = 8;
 struct MacroArgs {
     Geom g;
     const void *L;
-    double *rho, *ux, *uy, *uz;
+    double *out[4];      // rho, ux, uy, uz of node n0 on (null: not wanted)
+    uint32_t n0, count;
     ForceSpec f;
     double rho_off;
     unsigned long long *errbits;

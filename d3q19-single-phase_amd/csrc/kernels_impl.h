@@ -771,7 +771,8 @@ __global__ void __launch_bounds__(BLOCK) k_step_run(StepArgs a)
     store_run_all<P>((S *)a.dst, a.g.S, n0, F, std::make_integer_sequence<int, 19>{});
 }
 
-// macrovar / rhoupdat / materialisation of the fields of lattice L.
+// macrovar / rhoupdat / materialisation of the fields of nodes [n0, n0 +
+// count) of lattice L.
 // WHAT 0: rho, ux, uy, uz = macrovar(F) with rho - rho_off.
 // WHAT 1: rho = sum F (rhoupdat); max |rho_new - rho_old| into errbits.
 template <int P, int WHAT>
@@ -779,9 +780,10 @@ __global__ void __launch_bounds__(BLOCK) k_macro(MacroArgs a)
 {
     using S = typename Prec<P>::S;
     using T = typename Prec<P>::T;
-    const uint32_t n = blockIdx.x * BLOCK + threadIdx.x;
+    const uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
     double err = 0.0;
-    if (n < a.g.N) {
+    if (i < a.count) {
+        const uint32_t n = a.n0 + i;
         const Nbr b = make_nbr(n, a.g);
         T f[19];
         pull_all<P>((const S *)a.L, a.g.S, b, f);
@@ -792,14 +794,16 @@ __global__ void __launch_bounds__(BLOCK) k_macro(MacroArgs a)
             node_coords(n, a.g, ix, iy, iz);
             double fx, fy, fz;
             node_force(a.f, a.g, ix, iy, iz, fx, fy, fz);
-            a.ux[n] = (double)(ux9 + (T)fx / T(2.));
-            a.uy[n] = (double)(uy9 + (T)fy / T(2.));
-            a.uz[n] = (double)(uz9 + (T)fz / T(2.));
-            a.rho[n] = (double)(rho9 - (T)a.rho_off);
+            const double v[4] = {(double)(rho9 - (T)a.rho_off), (double)(ux9 + (T)fx / T(2.)),
+                                 (double)(uy9 + (T)fy / T(2.)), (double)(uz9 + (T)fz / T(2.))};
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (a.out[k])
+                    a.out[k][i] = v[k];
         } else {
             const double rnew = (double)rho9;
-            err = fabs(rnew - a.rho[n]);
-            a.rho[n] = rnew;
+            err = fabs(rnew - a.out[0][i]);
+            a.out[0][i] = rnew;
         }
     }
     if constexpr (WHAT == 1) {
@@ -1549,7 +1553,7 @@ hipError_t Launch<P>::closure_eval(const StepArgs &a, uint64_t n_begin, uint64_t
 template <int P>
 hipError_t Launch<P>::macro(const MacroArgs &a, int what, hipStream_t s)
 {
-    const dim3 grid(nblocks<P>(a.g.N)), blk(BLOCK);
+    const dim3 grid(nblocks<P>(a.count)), blk(BLOCK);
     if (what == 0)
         hipLaunchKernelGGL((k_macro<P, 0>), grid, blk, 0, s, a);
     else

@@ -283,22 +283,30 @@ int ensure_fields(lbm_channel *h)
     return LBM_OK;
 }
 
+// macrovar's arguments for nodes [n0, n0 + count) of lattice `which`; the
+// caller sets the outputs.
+MacroArgs macro_args(const lbm_channel *h, int which, uint64_t n0, uint64_t count)
+{
+    MacroArgs a;
+    a.g = h->g;
+    a.L = h->lat[which];
+    a.f = h->fm;
+    a.rho_off = h->rho_off;
+    a.errbits = nullptr;
+    a.n0 = (uint32_t)n0;
+    a.count = (uint32_t)count;
+    return a;
+}
+
 // macrovar of lattice `which` (minus the pending rho offset) into the arrays.
 int compute_fields(lbm_channel *h, int which)
 {
     int rc = ensure_fields(h);
     if (rc)
         return rc;
-    MacroArgs a;
-    a.g = h->g;
-    a.L = h->lat[which];
-    a.rho = h->mac[0];
-    a.ux = h->mac[1];
-    a.uy = h->mac[2];
-    a.uz = h->mac[3];
-    a.f = h->fm;
-    a.rho_off = h->rho_off;
-    a.errbits = nullptr;
+    MacroArgs a = macro_args(h, which, 0, h->g.N);
+    for (int k = 0; k < 4; k++)
+        a.out[k] = h->mac[k];
     rc = dispatch_err(PREC_CALL(h, macro, a, 0, h->stream), "macrovar");
     if (rc || !h->part)
         return rc;
@@ -834,36 +842,55 @@ struct NodeSlices {
     size_t bytes(size_t k) const { return (size_t)nodes(k) * node_bytes; }
 };
 
-// Per-node values made on the device slice by slice (launch(first, nodes,
-// device slice)) into the host array out.
+// Per-node values made on the device slice by slice into nout host arrays of
+// node_bytes each (null ones are skipped): launch(first, nodes, dst, step)
+// writes those of array j to dst + j * step bytes, j counting the arrays that
+// are not null.  The kernels store straight into the pinned slots, unless
+// their stores are scattered (`staged`: through device slices).
 template <class Launch>
-int nodes_to_host(lbm_channel *h, void *out, size_t node_bytes, const char *what, Launch launch)
+int nodes_to_host(lbm_channel *h, void *const *out, int nout, size_t node_bytes, bool staged, const char *what,
+                  Launch launch)
 {
-    const int rc = ensure_stage(h);
-    if (rc)
-        return rc;
-    char *const host = (char *)out;
+    char *host[4];
+    int m = 0;
+    for (int j = 0; j < nout; j++)
+        if (out[j])
+            host[m++] = (char *)out[j];
     const hipStream_t s = h->stream;
+    const size_t total = h->g.N * node_bytes * m;
     HIP_TRY(hipStreamSynchronize(s));
     HostPool &pool = host_pool();
+    const int workers = host_workers(total);
     std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
     hipError_t e = hipSuccess;
-    if (h->g.N * node_bytes >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device)) {
-        const NodeSlices sl(h->g.N, node_bytes, HOST_SLICE);
+    const bool pooled = total >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device, workers);
+    if (staged || !pooled) {
+        const int rc = ensure_stage(h);
+        if (rc)
+            return rc;
+    }
+    if (pooled) {
+        const NodeSlices sl(h->g.N, node_bytes * m, host_slice(total, true));
+        const size_t step = sl.per * node_bytes;
         e = host_slices_out(
-            pool, h->cfg.device, s, sl.count(), host_workers(h->g.N * node_bytes),
+            pool, h->cfg.device, s, sl.count(), workers,
             [&](size_t k, int slot, char *pinned) {
-                char *dev = h->stage + slot * HOST_SLICE;
-                const hipError_t le = launch(sl.first(k), sl.nodes(k), dev);
-                return le != hipSuccess ? le : hipMemcpyAsync(pinned, dev, sl.bytes(k), hipMemcpyDeviceToHost, s);
+                char *dev = staged ? h->stage + slot * HOST_SLICE : pinned;
+                const hipError_t le = launch(sl.first(k), sl.nodes(k), dev, step);
+                return le != hipSuccess || !staged ? le : link_copy(pinned, dev, sl.bytes(k), true, s);
             },
-            [&](size_t k, const char *pinned) { memcpy(host + sl.first(k) * node_bytes, pinned, sl.bytes(k)); });
+            [&](size_t k, const char *pinned) {
+                for (int j = 0; j < m; j++)
+                    memcpy(host[j] + sl.first(k) * node_bytes, pinned + j * step, sl.nodes(k) * node_bytes);
+            });
     } else {
-        const NodeSlices sl(h->g.N, node_bytes, STAGE_BYTES);
+        const NodeSlices sl(h->g.N, node_bytes * m, STAGE_BYTES);
+        const size_t step = sl.per * node_bytes;
         for (size_t k = 0; k < sl.count() && e == hipSuccess; k++) {
-            e = launch(sl.first(k), sl.nodes(k), h->stage);
-            if (e == hipSuccess)
-                e = hipMemcpyAsync(host + sl.first(k) * node_bytes, h->stage, sl.bytes(k), hipMemcpyDeviceToHost, s);
+            e = launch(sl.first(k), sl.nodes(k), h->stage, step);
+            for (int j = 0; j < m && e == hipSuccess; j++)
+                e = hipMemcpyAsync(host[j] + sl.first(k) * node_bytes, h->stage + j * step, sl.nodes(k) * node_bytes,
+                                   hipMemcpyDeviceToHost, s);
             if (e == hipSuccess)
                 e = hipStreamSynchronize(s);
         }
@@ -873,30 +900,29 @@ int nodes_to_host(lbm_channel *h, void *out, size_t node_bytes, const char *what
     return LBM_OK;
 }
 
-// The host array `in` to the device slice by slice, launch consuming each.
+// The host array `in` to the device slice by slice, launch consuming each,
+// straight from the pinned slot.
 template <class Launch>
 int nodes_from_host(lbm_channel *h, const void *in, size_t node_bytes, const char *what, Launch launch)
 {
-    const int rc = ensure_stage(h);
-    if (rc)
-        return rc;
     const char *const host = (const char *)in;
     const hipStream_t s = h->stream;
+    const size_t total = h->g.N * node_bytes;
     HIP_TRY(hipStreamSynchronize(s));
     HostPool &pool = host_pool();
+    const int workers = host_workers(total);
     std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
     hipError_t e = hipSuccess;
-    if (h->g.N * node_bytes >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device)) {
-        const NodeSlices sl(h->g.N, node_bytes, HOST_SLICE);
+    if (total >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device, workers)) {
+        const NodeSlices sl(h->g.N, node_bytes, host_slice(total, false));
         e = host_slices_in(
-            pool, h->cfg.device, s, sl.count(), host_workers(h->g.N * node_bytes),
+            pool, h->cfg.device, s, sl.count(), workers,
             [&](size_t k, char *pinned) { memcpy(pinned, host + sl.first(k) * node_bytes, sl.bytes(k)); },
-            [&](size_t k, int slot, const char *pinned) {
-                char *dev = h->stage + slot * HOST_SLICE;
-                const hipError_t ce = hipMemcpyAsync(dev, pinned, sl.bytes(k), hipMemcpyHostToDevice, s);
-                return ce != hipSuccess ? ce : launch(sl.first(k), sl.nodes(k), dev);
-            });
+            [&](size_t k, int, const char *pinned) { return launch(sl.first(k), sl.nodes(k), (char *)pinned); });
     } else {
+        const int rc = ensure_stage(h);
+        if (rc)
+            return rc;
         const NodeSlices sl(h->g.N, node_bytes, STAGE_BYTES);
         for (size_t k = 0; k < sl.count() && e == hipSuccess; k++) {
             e = hipMemcpyAsync(h->stage, host + sl.first(k) * node_bytes, sl.bytes(k), hipMemcpyHostToDevice, s);
@@ -954,7 +980,9 @@ int lbm_download_f(lbm_channel *h, double *f)
     CHECK_H(h);
     if (!f)
         return fail(LBM_ERR_ARG, "lbm_download_f: null f");
-    return nodes_to_host(h, f, 19 * sizeof(double), "lbm_download_f", [h](uint64_t n0, uint64_t cnt, char *dev) {
+    void *const out[1] = {f};
+    return nodes_to_host(h, out, 1, 19 * sizeof(double), false, "lbm_download_f",
+                         [h](uint64_t n0, uint64_t cnt, char *dev, size_t) {
         CopyArgs a;
         a.g = h->g;
         a.L = h->lat[h->cur];
@@ -1196,13 +1224,25 @@ int lbm_macrovar(lbm_channel *h, double *rho, double *ux, double *uy, double *uz
     double *dst[4] = {rho, ux, uy, uz};
     if (!rho && !ux && !uy && !uz)
         return LBM_OK;
-    int rc = compute_fields(h, h->cur);
-    if (rc)
-        return rc;
-    HostPart parts[4];
-    for (int k = 0; k < 4; k++)
-        parts[k] = HostPart{dst[k], h->mac[k], h->g.N * sizeof(double)};
-    return copy_parts(h, parts, 4, true, "lbm_macrovar");
+    if (h->part) { // nodes inside particles are set in the arrays
+        int rc = compute_fields(h, h->cur);
+        if (rc)
+            return rc;
+        HostPart parts[4];
+        for (int k = 0; k < 4; k++)
+            parts[k] = HostPart{dst[k], h->mac[k], h->g.N * sizeof(double)};
+        return copy_parts(h, parts, 4, true, "lbm_macrovar");
+    }
+    void *const out[4] = {rho, ux, uy, uz};
+    return nodes_to_host(h, out, 4, sizeof(double), false, "lbm_macrovar",
+                         [h, &dst](uint64_t n0, uint64_t cnt, char *dev, size_t step) {
+                             MacroArgs a = macro_args(h, h->cur, n0, cnt);
+                             for (int k = 0; k < 4; k++) {
+                                 a.out[k] = dst[k] ? (double *)dev : nullptr;
+                                 dev += dst[k] ? step : 0;
+                             }
+                             return PREC_CALL(h, macro, a, 0, h->stream);
+                         });
 }
 
 // Pinned results of rhoupdat: an iteration of lbm_prerelax each.
@@ -1225,15 +1265,8 @@ int lbm_rhoupdat(lbm_channel *h, double *rhoerrmax)
     rc = ensure_errout(h);
     if (rc)
         return rc;
-    MacroArgs a;
-    a.g = h->g;
-    a.L = h->lat[h->cur];
-    a.rho = h->mac[0];
-    a.ux = h->mac[1];
-    a.uy = h->mac[2];
-    a.uz = h->mac[3];
-    a.f = h->fm;
-    a.rho_off = 0.0;
+    MacroArgs a = macro_args(h, h->cur, 0, h->g.N);
+    a.out[0] = h->mac[0];
     a.errbits = h->errbits;
     rc = dispatch_err(PREC_CALL(h, macro, a, 1, h->stream), "rhoupdat");
     if (rc)
@@ -2042,14 +2075,15 @@ static int download_post_range(lbm_channel *h, uint64_t n0, uint64_t count, doub
     HIP_TRY(hipStreamSynchronize(s));
     HostPool &pool = host_pool();
     std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
-    if (19 * count * h->elem >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device)) {
+    const int workers = host_workers(19 * count * sizeof(double));
+    if (19 * count * h->elem >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device, workers)) {
         const uint64_t per = HOST_SLICE / h->elem, m = (count + per - 1) / per; // slices of a population
         const hipError_t e = host_slices_out(
-            pool, h->cfg.device, s, 19 * m, host_workers(19 * count * sizeof(double)),
+            pool, h->cfg.device, s, 19 * m, workers,
             [&](size_t k, int, char *pinned) {
                 const uint64_t i = k / m, at = k % m * per;
-                return hipMemcpyAsync(pinned, L + (i * S + n0 + at) * h->elem,
-                                      std::min<uint64_t>(per, count - at) * h->elem, hipMemcpyDeviceToHost, s);
+                return link_copy(pinned, L + (i * S + n0 + at) * h->elem,
+                                 std::min<uint64_t>(per, count - at) * h->elem, true, s);
             },
             [&](size_t k, const char *pinned) {
                 const uint64_t i = k / m, at = k % m * per;
@@ -2449,7 +2483,9 @@ static int closure_eval(lbm_channel *h, float *out, int what, const char *name)
     a.inv_ystar = h->mlp_inv_ystar;
     a.yscale = h->mlp_yscale;
     const size_t node_bytes = (what == 0 ? MLP_IN : 1) * sizeof(float);
-    return nodes_to_host(h, out, node_bytes, name, [&](uint64_t n0, uint64_t cnt, char *dev) {
+    void *const arrays[1] = {out};
+    // the inputs' stores are 40 bytes apart from lane to lane
+    return nodes_to_host(h, arrays, 1, node_bytes, what == 0, name, [&](uint64_t n0, uint64_t cnt, char *dev, size_t) {
         return PREC_CALL(h, closure_eval, a, n0, cnt, (float *)dev, what, h->stream);
     });
 }
