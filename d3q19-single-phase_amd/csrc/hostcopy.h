@@ -5,9 +5,9 @@
 // GB/s down, 29 GB/s up here, 4 GB/s down into pages not touched yet).  Here
 // the array moves in slices: a kernel fills or drains one pinned slot over
 // the link while host threads copy others to or from the array, so the link's
-// rate is the bound: 50 GB/s down and 51 up, 45 and 41 when the copy engine
+// rate is the bound: 53 GB/s down and 54 up, 45 and 41 when the copy engine
 // moved the slices (kernels that make the values, macrovar and the checkpoint,
-// store into the slots themselves).  1.81 GB of fields: 40.9 -> 36.2 ms; 11.2
+// store into the slots themselves).  1.81 GB of fields: 40.9 -> 34.3 ms; 11.2
 // MB 480 -> 340 us.
 // Two threads keep up with the link; more share the page faults of a new array.
 //
@@ -49,16 +49,23 @@ inline int host_workers(size_t total)
     return total < 8u << 20 ? 1 : (int)std::min<size_t>(HOST_WORKERS, 2 + (total >> 24));
 }
 
+// Copies with at least this many threads (32 MiB) use two streams.
+constexpr int HOST_SIDE_WORKERS = 4;
+
 struct HostPool {
     std::mutex mu;      // held by the copy that uses the slots
     std::mutex life_mu; // users
     int users = 0;
-    int device = -1;    // device of the events
+    int device = -1;    // device of the events and the side stream
     char *slot[HOST_WORKERS * HOST_DEPTH] = {};
     hipEvent_t ev[HOST_WORKERS * HOST_DEPTH] = {};
+    hipStream_t side = nullptr; // of this device, created by the first large copy
 
     void drop_events()
     {
+        if (side)
+            (void)hipStreamDestroy(side);
+        side = nullptr;
         for (hipEvent_t &e : ev) {
             if (e)
                 (void)hipEventDestroy(e);
@@ -87,8 +94,19 @@ struct HostPool {
                 }
             device = dev;
         }
+        if (workers >= HOST_SIDE_WORKERS && !side &&
+            hipStreamCreateWithFlags(&side, hipStreamNonBlocking) != hipSuccess) {
+            side = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
         return true;
     }
+    // The stream of odd slices: the side stream for large copies, so that the
+    // link is not idle between the end of one slice's kernel and the start of
+    // the next (1.81 GB down 36.2 -> 34.3 ms, 1.08 GB up 20.9 -> 20.0 ms); 2 MB
+    // took 105 us with two streams, 90 with one.
+    hipStream_t other(hipStream_t s, int workers) const { return workers >= HOST_SIDE_WORKERS ? side : s; }
     void retain()
     {
         std::lock_guard<std::mutex> l(life_mu);
@@ -116,14 +134,15 @@ inline HostPool &host_pool()
     return *p;
 }
 
-// Slices 0 .. n-1 from the device: enqueue(k, slot, pinned) puts what fills
-// the pinned slot on stream s, consume(k, pinned) reads it on the host.
-// Called with the pool's lock held and its slots ready; returns the first
-// error.  Everything enqueued has finished when it returns.
+// Slices 0 .. n-1 from the device: enqueue(k, slot, pinned, stream) puts what
+// fills the pinned slot on the stream, consume(k, pinned) reads it on the host.
+// Called with the pool's lock held, its slots ready and stream s idle; returns
+// the first error.  Everything enqueued has finished when it returns.
 template <class Enqueue, class Consume>
 hipError_t host_slices_out(HostPool &pool, int device, hipStream_t s, size_t n, int workers, Enqueue enqueue,
                            Consume consume)
 {
+    const hipStream_t odd = pool.other(s, workers);
     std::atomic<size_t> next{0};
     std::atomic<int> err{(int)hipSuccess};
     auto work = [&](int w) {
@@ -136,9 +155,10 @@ hipError_t host_slices_out(HostPool &pool, int device, hipStream_t s, size_t n, 
                 if (k >= n)
                     break;
                 const int q = (first + count) % HOST_DEPTH, slot = w * HOST_DEPTH + q;
-                e = enqueue(k, slot, pool.slot[slot]);
+                const hipStream_t on = k % 2 ? odd : s;
+                e = enqueue(k, slot, pool.slot[slot], on);
                 if (e == hipSuccess)
-                    e = hipEventRecord(pool.ev[slot], s);
+                    e = hipEventRecord(pool.ev[slot], on);
                 if (e != hipSuccess)
                     break;
                 held[q] = k;
@@ -169,16 +189,17 @@ hipError_t host_slices_out(HostPool &pool, int device, hipStream_t s, size_t n, 
     for (int w = 1; w < HOST_WORKERS; w++)
         if (t[w].joinable())
             t[w].join();
-    const hipError_t e = hipStreamSynchronize(s);
-    return err.load() != (int)hipSuccess ? (hipError_t)err.load() : e;
+    const hipError_t e = hipStreamSynchronize(s), e2 = hipStreamSynchronize(odd);
+    return err.load() != (int)hipSuccess ? (hipError_t)err.load() : e != hipSuccess ? e : e2;
 }
 
 // Slices 0 .. n-1 to the device: produce(k, pinned) fills the pinned slot on
-// the host, enqueue(k, slot, pinned) puts what reads it on stream s.
+// the host, enqueue(k, slot, pinned, stream) puts what reads it on the stream.
 template <class Produce, class Enqueue>
 hipError_t host_slices_in(HostPool &pool, int device, hipStream_t s, size_t n, int workers, Produce produce,
                           Enqueue enqueue)
 {
+    const hipStream_t odd = pool.other(s, workers);
     std::atomic<size_t> next{0};
     std::atomic<int> err{(int)hipSuccess};
     auto work = [&](int w) {
@@ -193,9 +214,10 @@ hipError_t host_slices_in(HostPool &pool, int device, hipStream_t s, size_t n, i
             if (e != hipSuccess)
                 break;
             produce(k, pool.slot[slot]);
-            e = enqueue(k, slot, pool.slot[slot]);
+            const hipStream_t on = k % 2 ? odd : s;
+            e = enqueue(k, slot, pool.slot[slot], on);
             if (e == hipSuccess)
-                e = hipEventRecord(pool.ev[slot], s);
+                e = hipEventRecord(pool.ev[slot], on);
         }
         int ok = (int)hipSuccess;
         if (e != hipSuccess)
@@ -212,8 +234,8 @@ hipError_t host_slices_in(HostPool &pool, int device, hipStream_t s, size_t n, i
     for (int w = 1; w < HOST_WORKERS; w++)
         if (t[w].joinable())
             t[w].join();
-    const hipError_t e = hipStreamSynchronize(s);
-    return err.load() != (int)hipSuccess ? (hipError_t)err.load() : e;
+    const hipError_t e = hipStreamSynchronize(s), e2 = hipStreamSynchronize(odd);
+    return err.load() != (int)hipSuccess ? (hipError_t)err.load() : e != hipSuccess ? e : e2;
 }
 
 // Copy between device memory and a pinned slot, 16 bytes a lane and four in
@@ -313,10 +335,10 @@ inline hipError_t host_copy(int device, hipStream_t s, const HostPart *parts, in
     if (down)
         return host_slices_out(
             pool, device, s, n, workers,
-            [&](size_t k, int, char *pinned) {
+            [&](size_t k, int, char *pinned, hipStream_t on) {
                 char *host, *dev;
                 const size_t b = find(k, host, dev);
-                return link_copy(pinned, dev, b, true, s);
+                return link_copy(pinned, dev, b, true, on);
             },
             [&](size_t k, const char *pinned) {
                 char *host, *dev;
@@ -330,10 +352,10 @@ inline hipError_t host_copy(int device, hipStream_t s, const HostPart *parts, in
             const size_t b = find(k, host, dev);
             memcpy(pinned, host, b);
         },
-        [&](size_t k, int, const char *pinned) {
+        [&](size_t k, int, const char *pinned, hipStream_t on) {
             char *host, *dev;
             const size_t b = find(k, host, dev);
-            return link_copy(dev, pinned, b, false, s);
+            return link_copy(dev, pinned, b, false, on);
         });
 }
 

@@ -843,9 +843,9 @@ struct NodeSlices {
 };
 
 // Per-node values made on the device slice by slice into nout host arrays of
-// node_bytes each (null ones are skipped): launch(first, nodes, dst, step)
-// writes those of array j to dst + j * step bytes, j counting the arrays that
-// are not null.  The kernels store straight into the pinned slots, unless
+// node_bytes each (null ones are skipped): launch(first, nodes, dst, step,
+// stream) writes those of array j to dst + j * step bytes, j counting the
+// arrays that are not null.  The kernels store straight into the pinned slots, unless
 // their stores are scattered (`staged`: through device slices).
 template <class Launch>
 int nodes_to_host(lbm_channel *h, void *const *out, int nout, size_t node_bytes, bool staged, const char *what,
@@ -874,10 +874,10 @@ int nodes_to_host(lbm_channel *h, void *const *out, int nout, size_t node_bytes,
         const size_t step = sl.per * node_bytes;
         e = host_slices_out(
             pool, h->cfg.device, s, sl.count(), workers,
-            [&](size_t k, int slot, char *pinned) {
+            [&](size_t k, int slot, char *pinned, hipStream_t on) {
                 char *dev = staged ? h->stage + slot * HOST_SLICE : pinned;
-                const hipError_t le = launch(sl.first(k), sl.nodes(k), dev, step);
-                return le != hipSuccess || !staged ? le : link_copy(pinned, dev, sl.bytes(k), true, s);
+                const hipError_t le = launch(sl.first(k), sl.nodes(k), dev, step, on);
+                return le != hipSuccess || !staged ? le : link_copy(pinned, dev, sl.bytes(k), true, on);
             },
             [&](size_t k, const char *pinned) {
                 for (int j = 0; j < m; j++)
@@ -887,7 +887,7 @@ int nodes_to_host(lbm_channel *h, void *const *out, int nout, size_t node_bytes,
         const NodeSlices sl(h->g.N, node_bytes * m, STAGE_BYTES);
         const size_t step = sl.per * node_bytes;
         for (size_t k = 0; k < sl.count() && e == hipSuccess; k++) {
-            e = launch(sl.first(k), sl.nodes(k), h->stage, step);
+            e = launch(sl.first(k), sl.nodes(k), h->stage, step, s);
             for (int j = 0; j < m && e == hipSuccess; j++)
                 e = hipMemcpyAsync(host[j] + sl.first(k) * node_bytes, h->stage + j * step, sl.nodes(k) * node_bytes,
                                    hipMemcpyDeviceToHost, s);
@@ -918,7 +918,9 @@ int nodes_from_host(lbm_channel *h, const void *in, size_t node_bytes, const cha
         e = host_slices_in(
             pool, h->cfg.device, s, sl.count(), workers,
             [&](size_t k, char *pinned) { memcpy(pinned, host + sl.first(k) * node_bytes, sl.bytes(k)); },
-            [&](size_t k, int, const char *pinned) { return launch(sl.first(k), sl.nodes(k), (char *)pinned); });
+            [&](size_t k, int, const char *pinned, hipStream_t on) {
+                return launch(sl.first(k), sl.nodes(k), (char *)pinned, on);
+            });
     } else {
         const int rc = ensure_stage(h);
         if (rc)
@@ -927,7 +929,7 @@ int nodes_from_host(lbm_channel *h, const void *in, size_t node_bytes, const cha
         for (size_t k = 0; k < sl.count() && e == hipSuccess; k++) {
             e = hipMemcpyAsync(h->stage, host + sl.first(k) * node_bytes, sl.bytes(k), hipMemcpyHostToDevice, s);
             if (e == hipSuccess)
-                e = launch(sl.first(k), sl.nodes(k), h->stage);
+                e = launch(sl.first(k), sl.nodes(k), h->stage, s);
         }
         if (e == hipSuccess)
             e = hipStreamSynchronize(s);
@@ -960,14 +962,14 @@ int lbm_upload_f(lbm_channel *h, const double *f)
         if (rc)
             return rc;
     }
-    const int rc = nodes_from_host(h, f, 19 * sizeof(double), "lbm_upload_f", [h](uint64_t n0, uint64_t cnt, char *dev) {
+    const int rc = nodes_from_host(h, f, 19 * sizeof(double), "lbm_upload_f", [h](uint64_t n0, uint64_t cnt, char *dev, hipStream_t on) {
         CopyArgs a;
         a.g = h->g;
         a.L = h->lat[h->cur];
         a.aos = (double *)dev;
         a.n0 = n0;
         a.count = cnt;
-        return PREC_CALL(h, scatter, a, h->stream);
+        return PREC_CALL(h, scatter, a, on);
     });
     if (rc)
         return rc;
@@ -982,14 +984,14 @@ int lbm_download_f(lbm_channel *h, double *f)
         return fail(LBM_ERR_ARG, "lbm_download_f: null f");
     void *const out[1] = {f};
     return nodes_to_host(h, out, 1, 19 * sizeof(double), false, "lbm_download_f",
-                         [h](uint64_t n0, uint64_t cnt, char *dev, size_t) {
+                         [h](uint64_t n0, uint64_t cnt, char *dev, size_t, hipStream_t on) {
         CopyArgs a;
         a.g = h->g;
         a.L = h->lat[h->cur];
         a.aos = (double *)dev;
         a.n0 = n0;
         a.count = cnt;
-        return PREC_CALL(h, gather, a, h->stream);
+        return PREC_CALL(h, gather, a, on);
     });
 }
 
@@ -1235,13 +1237,13 @@ int lbm_macrovar(lbm_channel *h, double *rho, double *ux, double *uy, double *uz
     }
     void *const out[4] = {rho, ux, uy, uz};
     return nodes_to_host(h, out, 4, sizeof(double), false, "lbm_macrovar",
-                         [h, &dst](uint64_t n0, uint64_t cnt, char *dev, size_t step) {
+                         [h, &dst](uint64_t n0, uint64_t cnt, char *dev, size_t step, hipStream_t on) {
                              MacroArgs a = macro_args(h, h->cur, n0, cnt);
                              for (int k = 0; k < 4; k++) {
                                  a.out[k] = dst[k] ? (double *)dev : nullptr;
                                  dev += dst[k] ? step : 0;
                              }
-                             return PREC_CALL(h, macro, a, 0, h->stream);
+                             return PREC_CALL(h, macro, a, 0, on);
                          });
 }
 
@@ -2080,10 +2082,10 @@ static int download_post_range(lbm_channel *h, uint64_t n0, uint64_t count, doub
         const uint64_t per = HOST_SLICE / h->elem, m = (count + per - 1) / per; // slices of a population
         const hipError_t e = host_slices_out(
             pool, h->cfg.device, s, 19 * m, workers,
-            [&](size_t k, int, char *pinned) {
+            [&](size_t k, int, char *pinned, hipStream_t on) {
                 const uint64_t i = k / m, at = k % m * per;
                 return link_copy(pinned, L + (i * S + n0 + at) * h->elem,
-                                 std::min<uint64_t>(per, count - at) * h->elem, true, s);
+                                 std::min<uint64_t>(per, count - at) * h->elem, true, on);
             },
             [&](size_t k, const char *pinned) {
                 const uint64_t i = k / m, at = k % m * per;
@@ -2485,8 +2487,8 @@ static int closure_eval(lbm_channel *h, float *out, int what, const char *name)
     const size_t node_bytes = (what == 0 ? MLP_IN : 1) * sizeof(float);
     void *const arrays[1] = {out};
     // the inputs' stores are 40 bytes apart from lane to lane
-    return nodes_to_host(h, arrays, 1, node_bytes, what == 0, name, [&](uint64_t n0, uint64_t cnt, char *dev, size_t) {
-        return PREC_CALL(h, closure_eval, a, n0, cnt, (float *)dev, what, h->stream);
+    return nodes_to_host(h, arrays, 1, node_bytes, what == 0, name, [&](uint64_t n0, uint64_t cnt, char *dev, size_t, hipStream_t on) {
+        return PREC_CALL(h, closure_eval, a, n0, cnt, (float *)dev, what, on);
     });
 }
 
