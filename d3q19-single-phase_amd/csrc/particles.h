@@ -60,11 +60,12 @@ struct PartState {
     double *FHprev, *TQprev;       // the previous step's hydrodynamic force and torque (3*np)
     double *VWnew;                 // new velocities, then angular velocities, until committed (6*np)
     int *nsteps_done;              // 0 before the first move (Euler start)
-    int *solid;                    // N
+    int *solid;                    // N: the particle at a node, -1 fluid, -2 - p uncovered by p and not refilled
+    uint8_t *inside;               // N: solid >= 0, the flags the collision reads (part_inside)
     int *link_node;                // np*maxlink
     signed char *link_dir;         // np*maxlink
     double *link_q;                // np*maxlink
-    double *link_contrib;          // np*maxlink*6
+    double *link_contrib;          // np*6*maxlink
     int *link_count;               // np
     int *fill_node;                // np*maxfill
     int *fill_count;               // np
@@ -121,18 +122,26 @@ __host__ __device__ inline Box sphere_box(const PartGeom &pg, const double *X, i
 
 template <int P>
 struct PartLaunch {
-    static hipError_t ibb(const PartGeom &pg, const PartState &ps, void *L, hipStream_t s);
+    // next: after part_advance and refill_inside, which leave the link
+    // fractions and the settling of refilled nodes to the next bounce-back
+    static hipError_t ibb(const PartGeom &pg, const PartState &ps, void *L, bool next, hipStream_t s);
     static hipError_t refill(const PartGeom &pg, const PartState &ps, void *L, hipStream_t s);
-    // part_classify (not the first) and refill together
-    static hipError_t classify_refill(const PartGeom &pg, const PartState &ps, void *L, hipStream_t s);
+    // the refill without its settling, and part_inside
+    static hipError_t refill_inside(const PartGeom &pg, const PartState &ps, void *L, hipStream_t s);
 };
 
 hipError_t part_classify(const PartGeom &pg, const PartState &ps, int first, hipStream_t s);
+// ps.inside after part_classify
+hipError_t part_inside(const PartGeom &pg, const PartState &ps, hipStream_t s);
 // macrovar's solid branch: fields at nodes inside particles
 hipError_t part_solid_fields(const PartGeom &pg, const PartState &ps, double rho_off, double *rho, double *ux,
                              double *uy, double *uz, hipStream_t s);
 hipError_t part_sum(const PartGeom &pg, const PartState &ps, hipStream_t s);
 hipError_t part_move(const PartGeom &pg, const PartState &ps, hipStream_t s);
+// part_sum, part_move and part_classify (not the first) in fewer launches, but
+// for the link fractions; part_finish forms those and settles refilled nodes
+hipError_t part_advance(const PartGeom &pg, const PartState &ps, hipStream_t s);
+hipError_t part_finish(const PartGeom &pg, const PartState &ps, hipStream_t s);
 
 extern template struct PartLaunch<0>;
 extern template struct PartLaunch<1>;
