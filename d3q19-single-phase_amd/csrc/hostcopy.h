@@ -9,7 +9,6 @@
 // moved the slices (kernels that make the values, macrovar and the checkpoint,
 // store into the slots themselves).  1.81 GB of fields: 40.9 -> 34.3 ms; 11.2
 // MB 480 -> 340 us.
-// Two threads keep up with the link; more share the page faults of a new array.
 //
 // The pinned slots belong to the process, not to a handle: up to HOST_WORKERS
 // x HOST_DEPTH slots of HOST_SLICE bytes (48 MiB), each allocated by the first
@@ -43,14 +42,17 @@ inline size_t host_slice(size_t total, bool down)
     return !down || total >= 64u << 20 ? HOST_SLICE : total >= 16u << 20 ? HOST_SLICE / 2 : HOST_SLICE / 4;
 }
 
-// Threads for a copy of `total` bytes: one (no thread is started) below 8 MiB.
+// Threads for a copy of `total` bytes: one (no thread is started) below 8
+// MiB.  Two keep up with the link where the array's pages are there; more
+// share the faults of a new array (11.2 MB of fields into one 1 570 us with
+// two, 1 060 with four; 28 MB of viscosities 837 us with three, 780 with six).
 inline int host_workers(size_t total)
 {
-    return total < 8u << 20 ? 1 : (int)std::min<size_t>(HOST_WORKERS, 2 + (total >> 24));
+    return total < 8u << 20 ? 1 : (int)std::min<size_t>(HOST_WORKERS, 2 + (total >> 22));
 }
 
-// Copies with at least this many threads (32 MiB) use two streams.
-constexpr int HOST_SIDE_WORKERS = 4;
+// Copies with at least this many threads (16 MiB) use two streams.
+constexpr int HOST_SIDE_WORKERS = 6;
 
 struct HostPool {
     std::mutex mu;      // held by the copy that uses the slots
