@@ -37,15 +37,25 @@ constexpr int BLOCK = 256;
 template <int P, int MODE>
 constexpr int step_block() { return ((MODE & (8 | 128)) != 0 || P == 1) ? 256 : 512; }
 
+// The offset as a value of the basic block it is used in: widened in another
+// one (the closure stores in a branch of its own) it costs every access a
+// 64-bit vector addition.
+__device__ __forceinline__ uint32_t here(uint32_t off)
+{
+    __asm__ volatile("" : "+v"(off));
+    return off;
+}
+
 // Element `node` of a population row, addressed as the row base plus a 32-bit
 // byte offset when that cannot wrap: 2-byte storage, whose rows hold fewer than
-// 2^31 nodes (lbm_create's limit), i.e. fewer than 2^32 bytes.  A wave-uniform
-// row base then stays in scalar registers and the load or store takes the
-// lane's offset directly, with no 64-bit address arithmetic per population.
-template <int P>
+// 2^31 nodes (lbm_create's limit), i.e. fewer than 2^32 bytes, and W32 = 3.  A
+// wave-uniform row base then stays in scalar registers and the load or store
+// takes the lane's offset directly, with no 64-bit address arithmetic per
+// population.
+template <int P, int W32 = 0>
 __device__ __forceinline__ typename Prec<P>::S *elem(typename Prec<P>::S *row, uint32_t node)
 {
-    if constexpr (half_storage(P))
+    if constexpr (half_storage(P) || W32 == 3)
         return (typename Prec<P>::S *)((char *)row + node * (uint32_t)sizeof(typename Prec<P>::S));
     else
         return row + node;
@@ -71,16 +81,50 @@ __device__ __forceinline__ S load_pop(const S *p)
 // stride Geom::S here and in the functions below.  The bounce-back
 // choice is made with masks, not branches, so every load issues back to back.
 // Loads are plain (cached): the +-x shifted reads of neighbouring waves share
-// cache lines.  W32 = 1 (N <= w32_max_n(P)): a pull with c_x != 0 addresses
-// both of its rows, I and OPP[I], from the lower of the two with a 32-bit
-// byte offset (|OPP[I] - I| <= 3, so below 4N elements: 8N bytes in 2-byte
-// storage, 16N in FP32), and the lane selects between two 32-bit offsets
-// instead of two 64-bit row bases.  W32 = 2 (2-byte storage, N <= 2^30): only
-// the pulls whose rows are adjacent (|OPP[I] - I| = 1: I = 1, 2, 8, 9, 12,
-// 13; offsets below 2N elements, 4N bytes) take that form.
-constexpr uint64_t W32_MAX_N = 1ull << 29;
-constexpr uint64_t w32_max_n(int P) { return half_storage(P) ? W32_MAX_N : (P == 1 ? (1ull << 28) : 0); }
+// cache lines.  W32 = 1 (2-byte storage, N <= 2^29): a pull with c_x != 0
+// addresses both of its rows, I and OPP[I], from the lower of the two with a
+// 32-bit byte offset (|OPP[I] - I| <= 3, so below 4N elements, 8N bytes), and
+// the lane selects between two 32-bit offsets instead of two 64-bit row bases.
+// W32 = 2 (2-byte storage, N <= 2^30): only the pulls whose rows are adjacent
+// (|OPP[I] - I| = 1: I = 1, 2, 8, 9, 12, 13; offsets below 2N elements, 4N
+// bytes) take that form.  W32 = 3 (the closure and FP32, N <= w32_max_n(P)):
+// pull32.
+constexpr uint64_t w32_max_n(int P) { return half_storage(P) ? (1ull << 29) : (P == 1 ? (1ull << 28) : 0); }
 constexpr uint64_t W32_ADJ_MAX_N = 1ull << 30;
+
+// The same value with 32-bit byte offsets only; b in bytes (its n and offsets
+// times the size of a population).  The shift in x is part of the row's scalar
+// base, so the lane's offset of direction I is one of nine, for the nine (c_y,
+// c_z), and pulls with c_x != 0 reach both of their rows from one base as
+// above.  With stores that take the same offset (store_all) the closure has 46
+// of 889 vector instructions fewer, an FP32 step 95 of 497.  us per step:
+// closure on 96x384x192 in FP32 231.2 -> 224.3, in FP16 211.4 -> 204.9; FP32
+// 130^3 58.0 -> 56.7, 96x384x192 single steps 195.6 -> 193.7.  FP64, FP32
+// steps within the last-level cache and plain 2-byte steps, bound by memory,
+// measured no difference (45x101x77 in FP16 8.73 / 8.84).
+template <int P, int I, int NT>
+__device__ __forceinline__ typename Prec<P>::T pull32(const typename Prec<P>::S *__restrict__ L, uint64_t N, const Nbr &b)
+{
+    using S = typename Prec<P>::S;
+    constexpr uint32_t SZ = sizeof(S);
+    constexpr int O = OPP[I];
+    const uint32_t at = src_yz<I>(b);
+    if constexpr (CX[I] == 0) {
+        uint64_t row = (uint64_t)I * N;
+        return Prec<P>::template to_T<I>(load_pop<NT>((const S *)((const char *)(L + row) + at)));
+    } else {
+        static_assert(Prec<P>::template scale_class<I>() == Prec<P>::template scale_class<O>());
+        // the lower of the two rows, I with its shift in x, and the way to the
+        // other one; wave-uniform (N is the kernel argument Geom::S) and
+        // opaque, so that they stay in scalar registers
+        uint64_t row = I < O ? (uint64_t)I * N - CX[I] : (uint64_t)O * N;
+        uint32_t d = ((uint32_t)(I < O ? O - I : I - O) * (uint32_t)N + (uint32_t)(I < O ? CX[I] : -CX[I])) * SZ;
+        __asm__("" : "+s"(row));
+        __asm__("" : "+s"(d));
+        const uint32_t off = I < O ? (walled<I>(b) ? b.n + d : at) : (walled<I>(b) ? b.n : at + d);
+        return Prec<P>::template to_T<I>(load_pop<NT>((const S *)((const char *)(L + row) + off)));
+    }
+}
 
 template <int P, int I, int W32 = 0, int NT = 0>
 __device__ __forceinline__ typename Prec<P>::T pull(const typename Prec<P>::S *__restrict__ L, uint64_t N,
@@ -98,7 +142,7 @@ __device__ __forceinline__ typename Prec<P>::T pull(const typename Prec<P>::S *_
             return Prec<P>::template to_T<I>(
                 load_pop<NT>(L + ((w ? (uint64_t)OPP[I] * N : (uint64_t)I * N) + node)));
         } else if constexpr (W32 == 1 || (W32 == 2 && (OPP[I] - I == 1 || I - OPP[I] == 1))) {
-            static_assert(half_storage(P) || P == 1, "32-bit pull offsets are for FP32 and 2-byte storage");
+            static_assert(half_storage(P), "rows within 2^32 bytes of 2-byte storage");
             constexpr int M = I < OPP[I] ? I : OPP[I];
             uint64_t row_m = (uint64_t)M * N;
             uint32_t d_i = (uint32_t)(I - M) * (uint32_t)N, d_o = (uint32_t)(OPP[I] - M) * (uint32_t)N;
@@ -133,7 +177,13 @@ template <int P, int W32, int NT, int... Is>
 __device__ __forceinline__ void pull_all_impl(const typename Prec<P>::S *__restrict__ L, uint64_t N, const Nbr &b,
                                               typename Prec<P>::T (&f)[19], std::integer_sequence<int, Is...>)
 {
-    ((f[Is] = pull<P, Is, W32, NT>(L, N, b)), ...);
+    if constexpr (W32 == 3) {
+        constexpr uint32_t SZ = sizeof(typename Prec<P>::S);
+        const Nbr c = {b.n * SZ, b.ym * SZ, b.yp * SZ, b.zm * SZ, b.zp * SZ, b.wlo, b.whi};
+        ((f[Is] = pull32<P, Is, NT>(L, N, c)), ...);
+    } else {
+        ((f[Is] = pull<P, Is, W32, NT>(L, N, b)), ...);
+    }
 }
 
 template <int P, int W32 = 0, int NT = 0>
@@ -143,25 +193,35 @@ __device__ __forceinline__ void pull_all(const typename Prec<P>::S *__restrict__
     pull_all_impl<P, W32, NT>(L, N, b, f, std::make_integer_sequence<int, 19>{});
 }
 
-template <int P, int... Is>
+// Row I of a lattice that is stored to, kept in scalar registers with W32 = 3.
+template <int P, int I, int W32>
+__device__ __forceinline__ typename Prec<P>::S *store_row(typename Prec<P>::S *L, uint64_t N)
+{
+    uint64_t row = (uint64_t)I * N;
+    if constexpr (W32 == 3)
+        __asm__("" : "+s"(row));
+    return L + row;
+}
+
+template <int P, int W32, int... Is>
 __device__ __forceinline__ void store_all_impl(typename Prec<P>::S *__restrict__ L, uint64_t N, uint32_t n,
                                                const typename Prec<P>::T (&f)[19], std::integer_sequence<int, Is...>)
 {
-    ((Prec<P>::template st<Is>(elem<P>(L + (uint64_t)Is * N, n), f[Is])), ...);
+    ((Prec<P>::template st<Is>(elem<P, W32>(store_row<P, Is, W32>(L, N), n), f[Is])), ...);
 }
 
-template <int P>
+template <int P, int W32>
 __device__ __forceinline__ void store_all(typename Prec<P>::S *__restrict__ L, uint64_t N, uint32_t n,
                                           const typename Prec<P>::T (&f)[19])
 {
-    store_all_impl<P>(L, N, n, f, std::make_integer_sequence<int, 19>{});
+    store_all_impl<P, W32>(L, N, n, f, std::make_integer_sequence<int, 19>{});
 }
 
-template <int P, int... Is>
+template <int P, int W32, int... Is>
 __device__ __forceinline__ void store_all_cached(typename Prec<P>::S *__restrict__ L, uint64_t N, uint32_t n,
                                                  const typename Prec<P>::T (&f)[19], std::integer_sequence<int, Is...>)
 {
-    ((*elem<P>(L + (uint64_t)Is * N, n) = Prec<P>::template to_S<Is>(f[Is])), ...);
+    ((*elem<P, W32>(store_row<P, Is, W32>(L, N), n) = Prec<P>::template to_S<Is>(f[Is])), ...);
 }
 
 // Scatter the streamed value F_I(x) back to the post-collision slot it came
@@ -306,10 +366,10 @@ __device__ __forceinline__ void block_err_max(double err, uint32_t nb, unsigned 
 // fields were formed with another force than the collision's (the force was
 // changed after the last macrovar): a.fc is the collision's force, a.fm the
 // fields'.
-// MODE + 32: 2-byte storage with N <= W32_MAX_N (and the FP32 closure with
-// N <= 2^28): the pulls with c_x != 0 take 32-bit offsets (pull<P, I, 1>);
-// the same loads, fewer instructions.  MODE + 64: 2-byte storage with
-// N <= 2^30: the pulls between adjacent rows only (pull<P, I, 2>).
+// MODE + 32: N <= w32_max_n(P): 32-bit offsets (pull<P, I, 1> in 2-byte storage,
+// pull32 with the closure and in FP32), the same accesses with fewer
+// instructions.  MODE + 64: 2-byte storage with N <= 2^30: the pulls between
+// adjacent rows only (pull<P, I, 2>).
 // MODE + 128: cached instead of non-temporal stores; MODE + 256:
 // non-temporal loads (step_policy).
 // MODE 2 + 512: an iteration of the pre-relaxation, rhoupdat and the step in
@@ -343,7 +403,8 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
     // the 19 loads issue first; the closure's weights are staged while they
     // are in flight
     T f[19];
-    pull_all<P, (MODE & 32) != 0 ? 1 : ((MODE & 64) != 0 ? 2 : 0), (MODE & 256) != 0>(src, a.g.S, b, f);
+    constexpr int W32 = (MODE & 32) != 0 ? (WAVE || P == 1 ? 3 : 1) : ((MODE & 64) != 0 ? 2 : 0);
+    pull_all<P, W32, (MODE & 256) != 0>(src, a.g.S, b, f);
     __shared__ __attribute__((aligned(16))) _Float16 wl[WAVE ? MLP_LDS : 8];
     if constexpr (WAVE) {
         mlp_stage(a.mlp, wl, threadIdx.x, a.nb);
@@ -437,10 +498,11 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
     }
     if constexpr (RHO)
         a.rho_out[n] = rnew;
+    const uint32_t at = W32 == 3 ? here(n) : n;
     if constexpr ((MODE & 128) != 0)
-        store_all_cached<P>(dst, a.g.S, n, f, std::make_integer_sequence<int, 19>{});
+        store_all_cached<P, W32>(dst, a.g.S, at, f, std::make_integer_sequence<int, 19>{});
     else
-        store_all<P>(dst, a.g.S, n, f);
+        store_all<P, W32>(dst, a.g.S, at, f);
 }
 
 template <int P, int MODE>
@@ -1416,38 +1478,40 @@ hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
     const StepPolicy policy = step_policy<P>(a);
 #define STEP_CASE(MODE) \
     case (MODE) & 31: return launch(k_step<P, MODE>, step_block<P, MODE>())
+    // 32-bit offsets in FP32 unless the cache holds both lattices (a lattice
+    // that it holds is far below w32_max_n)
+    constexpr int W = P == 1 ? 32 : 0;
 #define POLICY_CASE(MODE)                                                                      \
     case (MODE) & 31:                                                                          \
         if constexpr (!half_storage(P)) {                                                      \
             if (policy == POLICY_FILL)                                                         \
-                return launch(k_step<P, (MODE) + 384>, step_block<P, 128>());                  \
+                return launch(k_step<P, (MODE) + W + 384>, step_block<P, 128>());              \
         }                                                                                      \
         return policy == POLICY_CACHED ? launch(k_step<P, (MODE) + 128>, step_block<P, 128>()) \
+               : w32                   ? launch(k_step<P, (MODE) + W>, step_block<P, MODE>())  \
                                        : launch(k_step<P, MODE>, step_block<P, MODE>())
 #define CLOSURE_CASE(MODE) \
     case (MODE) & 31: return launch_closure(k_step_closure<P, MODE>)
+    const bool w32 = a.w32 == 1 && a.g.S <= w32_max_n(P);
     if (mode == 2 && a.errbits) {
         return policy == POLICY_CACHED ? launch(k_step<P, 642>, step_block<P, 128>())
-               : policy == POLICY_FILL && !half_storage(P) ? launch(k_step<P, 898>, step_block<P, 128>())
+               : policy == POLICY_FILL && !half_storage(P) ? launch(k_step<P, 898 + W>, step_block<P, 128>())
+               : w32                                       ? launch(k_step<P, 514 + W>, step_block<P, 514>())
                                                            : launch(k_step<P, 514>, step_block<P, 514>());
     }
-    if constexpr (half_storage(P) || P == 1) {
-        // 32-bit pull offsets where the lattice allows them: the main loop's
-        // modes in 2-byte storage (FP16 1.8-2.5 % faster, FP16C 2.7-2.9 %, on
-        // the 192x768x384 channel; FP32's memory-bound step measured no
-        // change), and the closure modes, which are issue-bound, in FP32 and
-        // 2-byte storage
-        if (a.w32 == 1 && a.g.S <= w32_max_n(P)) {
-            if constexpr (half_storage(P)) {
-                switch (mode) {
-                    POLICY_CASE(32);
-                    POLICY_CASE(33);
-                    POLICY_CASE(36);
-                    POLICY_CASE(48);
-                default:
-                    break;
-                }
+    if constexpr (half_storage(P)) {
+        if (w32)
+            switch (mode) {
+                POLICY_CASE(32);
+                POLICY_CASE(33);
+                POLICY_CASE(36);
+                POLICY_CASE(48);
+            default:
+                break;
             }
+    }
+    if constexpr (P != 0) {
+        if (w32)
             switch (mode) {
                 CLOSURE_CASE(40);
                 CLOSURE_CASE(44);
@@ -1455,7 +1519,6 @@ hipError_t Launch<P>::step(const StepArgs &args, int mode, hipStream_t s)
             default:
                 break;
             }
-        }
     }
     if constexpr (half_storage(P)) {
         // above 2^29 nodes (the 2048x1024x512 channel), the pulls between

@@ -619,9 +619,10 @@ int lbm_create(const lbm_config *cfg, lbm_channel **out)
         // the 192x768x384 channel: 64.6 % vs 69.2 % of HBM in FP64)
         const char *k = getenv("LBM_STEP_KERNEL");
         h->runs = (k && strcmp(k, "runs") == 0) ? 1 : 0;
-        // LBM_STEP_W32=0: 2-byte storage and the FP32 closure address their
-        // walled pulls from two 64-bit row bases even where 32-bit offsets
-        // would do; LBM_STEP_W32=adjacent: 2-byte storage takes 32-bit
+        // LBM_STEP_W32=0: 2-byte storage, the FP32 closure and FP32 steps of
+        // lattices beyond the last-level cache address their pulls with
+        // 64-bit arithmetic even where 32-bit offsets would do;
+        // LBM_STEP_W32=adjacent: 2-byte storage takes 32-bit
         // offsets between adjacent rows only, the form lattices above 2^29
         // nodes use (the same values; for comparing the forms)
         const char *w = getenv("LBM_STEP_W32");
