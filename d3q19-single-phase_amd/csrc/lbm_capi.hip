@@ -859,7 +859,8 @@ int nodes_to_host(lbm_channel *h, void *const *out, int nout, size_t node_bytes,
             host[m++] = (char *)out[j];
     const hipStream_t s = h->stream;
     const size_t total = h->g.N * node_bytes * m;
-    HIP_TRY(hipStreamSynchronize(s));
+    if (total >= HOST_MIN)
+        HIP_TRY(hipStreamSynchronize(s));
     HostPool &pool = host_pool();
     const int workers = host_workers(total);
     std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
@@ -909,7 +910,8 @@ int nodes_from_host(lbm_channel *h, const void *in, size_t node_bytes, const cha
     const char *const host = (const char *)in;
     const hipStream_t s = h->stream;
     const size_t total = h->g.N * node_bytes;
-    HIP_TRY(hipStreamSynchronize(s));
+    if (total >= HOST_MIN)
+        HIP_TRY(hipStreamSynchronize(s));
     HostPool &pool = host_pool();
     const int workers = host_workers(total);
     std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
@@ -2795,14 +2797,32 @@ int lbm_trainer_predict(lbm_trainer *t, long long first, long long count, float 
     CHECK_T(t);
     if (!out || first < 0 || count < 1 || first + count > t->count)
         return fail(LBM_ERR_ARG, "lbm_trainer_predict: bad range or null output");
-    float *d = nullptr;
-    HIP_TRY(hipMalloc((void **)&d, (size_t)count * sizeof(float)));
-    hipError_t e = mlp_predict(t->w, t->feat, (uint32_t)first, (uint32_t)count, d, t->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(out, d, (size_t)count * sizeof(float), hipMemcpyDeviceToHost, t->stream);
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(t->stream);
-    (void)hipFree(d);
+    // as nodes_to_host: the kernel stores into the pinned slots
+    const size_t total = (size_t)count * sizeof(float);
+    const int workers = host_workers(total);
+    hipError_t e = total >= HOST_MIN ? hipStreamSynchronize(t->stream) : hipSuccess;
+    HostPool &pool = host_pool();
+    std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
+    if (e == hipSuccess && total >= HOST_MIN && lock.owns_lock() && pool.ready(t->device, workers)) {
+        const size_t per = host_slice(total, true) / sizeof(float), n = ((size_t)count + per - 1) / per;
+        auto here = [&](size_t k) { return std::min<size_t>(per, (size_t)count - k * per); };
+        e = host_slices_out(
+            pool, t->device, t->stream, n, workers,
+            [&](size_t k, int, char *pinned, hipStream_t on) {
+                return mlp_predict(t->w, t->feat, (uint32_t)(first + k * per), (uint32_t)here(k), (float *)pinned, on);
+            },
+            [&](size_t k, const char *pinned) { memcpy(out + k * per, pinned, here(k) * sizeof(float)); });
+    } else if (e == hipSuccess) {
+        float *d = nullptr;
+        e = hipMalloc((void **)&d, total);
+        if (e == hipSuccess)
+            e = mlp_predict(t->w, t->feat, (uint32_t)first, (uint32_t)count, d, t->stream);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(out, d, total, hipMemcpyDeviceToHost, t->stream);
+        if (e == hipSuccess)
+            e = hipStreamSynchronize(t->stream);
+        (void)hipFree(d);
+    }
     if (e != hipSuccess)
         return fail(LBM_ERR_HIP, "lbm_trainer_predict: %s", hipGetErrorString(e));
     return LBM_OK;

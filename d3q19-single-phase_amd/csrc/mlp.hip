@@ -151,11 +151,11 @@ __global__ void __launch_bounds__(256) k_features(FeatArgs a)
 // Bound: 53 matrix instructions of 64 cycles and 16 of 32 (the gradient of W1,
 // whose ten columns and b1 fill a 16-wide product) a group of 32 samples, with
 // 32 tanh and the LDS traffic between them; the samples (44 B each) stay in
-// cache.  An iteration of 65 536 samples takes 15.2 us, 287 us with one lane
+// cache.  An iteration of 65 536 samples takes 14.4 us, 287 us with one lane
 // per sample on the vector ALUs (48 us) and one thread per parameter adding 1
 // 024 partials (231 us).
 constexpr int GROUP = 32;
-constexpr int MLP_WAVES = 4;             // waves per block
+constexpr int MLP_WAVES = 4;             // waves per block of the prediction
 constexpr int TS = 36;                   // LDS stride of a sample's 32 values
 constexpr int TX = 12;                   // LDS stride of a sample's inputs
 constexpr int MLP_OUT = MLP_NPARAM + 1;  // gradient and loss
@@ -223,17 +223,19 @@ __device__ __forceinline__ void wave_lds_order()
 // Gradient of mean((softplus(o) + m - y)^2) over samples [first, first+count):
 // wave v of the grid takes groups v, v + waves, ... of 32 samples; the block
 // adds its waves in order and writes partial[block * MLP_OUT + i] (i =
-// NPARAM: loss).  253 VGPRs and 78 KiB of LDS: two blocks per CU.
-__global__ void __launch_bounds__(64 * MLP_WAVES, 2)
+// NPARAM: loss).  253 VGPRs and 19.5 KiB of LDS a wave: W = 4 or 8 waves, one
+// block per CU (mlp_shape).
+template <int W>
+__global__ void __launch_bounds__(64 * W, 2)
 k_mlp_grad(const float *__restrict__ w, const float *__restrict__ feat, const float *__restrict__ target,
            uint32_t first, uint32_t count, float *__restrict__ partial)
 {
-    __shared__ __attribute__((aligned(16))) float lds[MLP_WAVES][GROUP * (4 * TS + TX)];
+    __shared__ __attribute__((aligned(16))) float lds[W][GROUP * (4 * TS + TX)];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, j = lane & 31, h = lane >> 5;
     float *const th1 = lds[wv], *const tg2 = th1 + GROUP * TS, *const tg1 = tg2 + GROUP * TS,
                  *const th3 = tg1 + GROUP * TS, *const tx = th3 + GROUP * TS;
     const float inv_count = 1.0f / (float)count;
-    const uint32_t groups = (count + GROUP - 1) / GROUP, waves = gridDim.x * MLP_WAVES;
+    const uint32_t groups = (count + GROUP - 1) / GROUP, waves = gridDim.x * W;
     // the lane's sample of group g: half its inputs and the target, loaded one
     // group ahead (the first with the weights)
     auto sample = [&](uint32_t g, float (&x)[5], float &y) {
@@ -245,7 +247,7 @@ k_mlp_grad(const float *__restrict__ w, const float *__restrict__ feat, const fl
         y = valid ? target[(uint64_t)first + s] : 0.0f;
     };
     float xn[5], yn;
-    sample(blockIdx.x * MLP_WAVES + wv, xn, yn);
+    sample(blockIdx.x * W + wv, xn, yn);
     MlpRegs n;
     n.load(w, j, h);
     float a2t[16]; // columns of W2: the transposed product of the back-propagation
@@ -259,7 +261,7 @@ k_mlp_grad(const float *__restrict__ w, const float *__restrict__ feat, const fl
     for (int r = 0; r < 16; r++)
         dw2[r] = 0.0f;
     float db2 = 0.0f, dw3 = 0.0f, db3 = 0.0f, loss = 0.0f;
-    for (uint32_t g = blockIdx.x * MLP_WAVES + wv; g < groups; g += waves) {
+    for (uint32_t g = blockIdx.x * W + wv; g < groups; g += waves) {
         const bool valid = g * GROUP + j < count;
         float x[5];
 #pragma unroll
@@ -354,10 +356,10 @@ k_mlp_grad(const float *__restrict__ w, const float *__restrict__ feat, const fl
         out[MLP_NPARAM] = loss;
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < MLP_OUT; i += 64 * MLP_WAVES) {
+    for (int i = threadIdx.x; i < MLP_OUT; i += 64 * W) {
         float v = lds[0][i];
 #pragma unroll
-        for (int k = 1; k < MLP_WAVES; k++)
+        for (int k = 1; k < W; k++)
             v += lds[k][i];
         partial[(uint64_t)blockIdx.x * MLP_OUT + i] = v;
     }
@@ -377,10 +379,18 @@ k_mlp_sum_adam(const float *__restrict__ partial, uint32_t rows, float *__restri
     const int p = threadIdx.x % SUM_PARAMS, q = threadIdx.x / SUM_PARAMS;
     const int i = blockIdx.x * SUM_PARAMS + p;
     float g = 0.0f;
+    // the step's own operands load with the partials
+    const bool step = adam && q == 0 && i < MLP_NPARAM;
+    const float m0 = step ? m[i] : 0.0f, v0 = step ? v[i] : 0.0f, w0 = step ? w[i] : 0.0f;
     if (i < MLP_OUT) {
-#pragma unroll 8
-        for (uint32_t b = q; b < rows; b += SUM_ROWS)
-            g += partial[(uint64_t)b * MLP_OUT + i];
+        // MLP_GRAD_BLOCKS rows at most: a thread's loads are all in flight at once
+        float t[MLP_GRAD_BLOCKS / SUM_ROWS];
+#pragma unroll
+        for (uint32_t b = 0; b < MLP_GRAD_BLOCKS / SUM_ROWS; b++)
+            t[b] = q + b * SUM_ROWS < rows ? partial[(uint64_t)(q + b * SUM_ROWS) * MLP_OUT + i] : 0.0f;
+#pragma unroll
+        for (uint32_t b = 0; b < MLP_GRAD_BLOCKS / SUM_ROWS; b++)
+            g += t[b];
     }
     sums[q][p] = g;
     __syncthreads();
@@ -390,13 +400,13 @@ k_mlp_sum_adam(const float *__restrict__ partial, uint32_t rows, float *__restri
     for (int k = 1; k < SUM_ROWS; k++)
         g += sums[k][p];
     grad[i] = g;
-    if (adam && i < MLP_NPARAM) {
+    if (step) {
         const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-        const float mi = b1 * m[i] + (1.0f - b1) * g;
-        const float vi = b2 * v[i] + (1.0f - b2) * g * g;
+        const float mi = b1 * m0 + (1.0f - b1) * g;
+        const float vi = b2 * v0 + (1.0f - b2) * g * g;
         m[i] = mi;
         v[i] = vi;
-        w[i] = w[i] - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
+        w[i] = w0 - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
     }
 }
 
@@ -488,30 +498,38 @@ hipError_t mlp_plane_targets(uint32_t lx, uint32_t ly, uint32_t lz, const float 
     return hipGetLastError();
 }
 
-// Blocks for `count` samples: a wave for every group of 32 up to a block per
-// CU, beyond that several groups to a wave.  From eight groups a wave on, two
-// blocks per CU: their matrix and vector instructions overlap, which then
-// outweighs loading the weights and writing the partials twice (us an
-// iteration, one / two blocks: 65 536 samples 15.2 / 16.4, 131 072 22.5 / 23.3,
-// 262 144 36.8 / 35.5, 524 288 65.8 / 59.6).
-static uint32_t mlp_blocks(uint32_t count)
+// Blocks and waves per block of a gradient over `count` samples: a wave for
+// every group of 32 up to a block of four waves per CU, beyond that blocks of
+// eight, whose two waves per SIMD overlap matrix and vector instructions while
+// the CU still writes one partial gradient; more than 65 536 samples take
+// several groups a wave.  us an iteration with blocks of four waves, two per
+// CU from 262 144 samples on / with these: 32 800 samples 14.0 / 13.5, 65 536
+// 14.8 / 14.4, 131 072 22.2 / 21.3, 262 144 35.3 / 33.4, 524 288 59.2 / 57.6;
+// 9.2 us of each are the two launches with their chains of loads.
+struct MlpShape {
+    uint32_t blocks, waves;
+};
+static MlpShape mlp_shape(uint32_t count)
 {
     const uint32_t groups = (count + GROUP - 1) / GROUP;
-    const uint32_t most = groups >= 8 * MLP_WAVES * (MLP_GRAD_BLOCKS / 2) ? MLP_GRAD_BLOCKS : MLP_GRAD_BLOCKS / 2;
-    return std::min<uint32_t>((groups + MLP_WAVES - 1) / MLP_WAVES, most);
+    const uint32_t waves = groups <= 4 * MLP_GRAD_BLOCKS ? 4 : 8;
+    return MlpShape{std::min<uint32_t>((groups + waves - 1) / waves, MLP_GRAD_BLOCKS), waves};
 }
 
 hipError_t mlp_grad(const float *w, const float *feat, const float *target, uint32_t first, uint32_t count,
                     float *partial, float *grad, float *wmut, float *m, float *v, int step, float lr, int adam,
                     hipStream_t s)
 {
-    const uint32_t nb = mlp_blocks(count);
+    const MlpShape sh = mlp_shape(count);
     // Adam's bias corrections, in double on the host
     const float c1 = (float)(1.0 / (1.0 - std::pow((double)0.9f, step)));
     const float c2 = (float)(1.0 / (1.0 - std::pow((double)0.999f, step)));
-    hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(64 * MLP_WAVES), 0, s, w, feat, target, first, count, partial);
+    if (sh.waves == 4)
+        hipLaunchKernelGGL(k_mlp_grad<4>, dim3(sh.blocks), dim3(64 * 4), 0, s, w, feat, target, first, count, partial);
+    else
+        hipLaunchKernelGGL(k_mlp_grad<8>, dim3(sh.blocks), dim3(64 * 8), 0, s, w, feat, target, first, count, partial);
     hipLaunchKernelGGL(k_mlp_sum_adam, dim3((MLP_OUT + SUM_PARAMS - 1) / SUM_PARAMS), dim3(SUM_PARAMS * SUM_ROWS), 0, s,
-                       partial, nb, grad, wmut, m, v, c1, c2, lr, adam);
+                       partial, sh.blocks, grad, wmut, m, v, c1, c2, lr, adam);
     return hipGetLastError();
 }
 
@@ -525,7 +543,10 @@ hipError_t mlp_fill_plane_targets(float *target, uint64_t first, uint64_t count,
 
 hipError_t mlp_predict(const float *w, const float *feat, uint32_t first, uint32_t count, float *out, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_mlp_predict, dim3(mlp_blocks(count)), dim3(64 * MLP_WAVES), 0, s, w, feat, first, count, out);
+    // a wave for every group up to two blocks of four per CU
+    const uint32_t groups = (count + GROUP - 1) / GROUP;
+    const uint32_t nb = std::min<uint32_t>((groups + MLP_WAVES - 1) / MLP_WAVES, 512);
+    hipLaunchKernelGGL(k_mlp_predict, dim3(nb), dim3(64 * MLP_WAVES), 0, s, w, feat, first, count, out);
     return hipGetLastError();
 }
 

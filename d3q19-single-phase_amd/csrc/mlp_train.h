@@ -43,7 +43,7 @@ struct MlpLaunch {
 
 // Most blocks of a gradient pass: `partial` holds a gradient and a loss
 // (MLP_NPARAM + 1 floats) for each.
-constexpr uint32_t MLP_GRAD_BLOCKS = 512;
+constexpr uint32_t MLP_GRAD_BLOCKS = 256; // a block per CU
 
 hipError_t mlp_features(const FeatArgs &a, hipStream_t s);
 hipError_t mlp_grad(const float *w, const float *feat, const float *target, uint32_t first, uint32_t count,
