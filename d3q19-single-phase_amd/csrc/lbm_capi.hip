@@ -136,6 +136,7 @@ struct lbm_trainer {
 };
 
 // Particle set on the device (see particles.h).
+constexpr size_t PART_STATE = 24; // doubles a particle in the block that ps.X starts
 struct Part {
     PartGeom pg;
     PartState ps;
@@ -2201,16 +2202,19 @@ int lbm_particles_create(lbm_channel *h, const lbm_particle_config *pc, const do
         if (rc == LBM_OK)
             rc = part_alloc(pt, p, bytes);
     };
-    A((void **)&ps.X, 6 * np * sizeof(double)); // X, then the previous positions
-    A((void **)&ps.V, 3 * np * sizeof(double));
-    A((void **)&ps.W, 3 * np * sizeof(double));
+    // what lbm_particles_get reads in one piece: X, the previous positions, V,
+    // W, FH, TQ, FC, FL and the overflow word
+    A((void **)&ps.X, (PART_STATE * np + 1) * sizeof(double));
+    ps.V = ps.X + 6 * np;
+    ps.W = ps.V + 3 * np;
+    ps.FH = ps.W + 3 * np;
+    ps.TQ = ps.FH + 3 * np;
+    ps.FC = ps.TQ + 3 * np;
+    ps.FL = ps.FC + 3 * np;
+    ps.overflow = (int *)(ps.FL + 3 * np);
     A((void **)&ps.TH, 3 * np * sizeof(double));
     A((void **)&ps.Aprev, 3 * np * sizeof(double));
     A((void **)&ps.ALprev, 3 * np * sizeof(double));
-    A((void **)&ps.FH, 3 * np * sizeof(double));
-    A((void **)&ps.TQ, 3 * np * sizeof(double));
-    A((void **)&ps.FC, 3 * np * sizeof(double));
-    A((void **)&ps.FL, 3 * np * sizeof(double));
     A((void **)&ps.FHprev, 3 * np * sizeof(double));
     A((void **)&ps.TQprev, 3 * np * sizeof(double));
     A((void **)&ps.VWnew, 6 * np * sizeof(double));
@@ -2224,7 +2228,6 @@ int lbm_particles_create(lbm_channel *h, const lbm_particle_config *pc, const do
     A((void **)&ps.link_count, np * sizeof(int));
     A((void **)&ps.fill_node, nf * sizeof(int));
     A((void **)&ps.fill_count, np * sizeof(int));
-    A((void **)&ps.overflow, sizeof(int));
     if (rc) {
         for (void *p : pt->allocs)
             (void)hipFree(p);
@@ -2266,11 +2269,8 @@ int lbm_particles_create(lbm_channel *h, const lbm_particle_config *pc, const do
             return fail(LBM_ERR_STATE, "%s: no particles on this handle", __func__);     \
     } while (0)
 
-static int check_overflow(lbm_channel *h, const char *what)
+static int overflow_error(const lbm_channel *h, int ovf, const char *what)
 {
-    int ovf = 0;
-    HIP_TRY(hipMemcpyAsync(&ovf, h->part->ps.overflow, sizeof(int), hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
     if (ovf & 2)
         return fail(LBM_ERR_STATE, "%s: a particle's position or velocity became non-finite (the run diverged)",
                     what);
@@ -2278,6 +2278,14 @@ static int check_overflow(lbm_channel *h, const char *what)
         return fail(LBM_ERR_STATE, "%s: a per-particle link or refill list overflowed (maxlink %d, maxfill %d)",
                     what, h->part->pg.maxlink, h->part->pg.maxfill);
     return LBM_OK;
+}
+
+static int check_overflow(lbm_channel *h, const char *what)
+{
+    int ovf = 0;
+    HIP_TRY(hipMemcpyAsync(&ovf, h->part->ps.overflow, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    return overflow_error(h, ovf, what);
 }
 
 int lbm_beads_links(lbm_channel *h)
@@ -2322,6 +2330,9 @@ int lbm_beads_move(lbm_channel *h)
     return dispatch_err(part_move(pt->pg, pt->ps, h->stream), "beads_move");
 }
 
+// Lattices above this size run the particle work beside the collision.
+constexpr uint64_t PART_ASIDE_BYTES = 260000000ull;
+
 int lbm_run_particles(lbm_channel *h, int istep0, int nsteps)
 {
     CHECK_P(h);
@@ -2335,9 +2346,14 @@ int lbm_run_particles(lbm_channel *h, int istep0, int nsteps)
     // settles the refilled nodes.  Streams of the default priority.  us per
     // step, with the classification between the steps / beside the collision:
     // 250 spheres on 96x384x192, FP64 492 / 462, FP32 293 / 280; 2 000 on
-    // 192x768x384, 3 715 / 3 655 and 2 150 / 2 075; 20 on 64x100x90 in FP64
-    // 101 / 93.
-    if (!h->pstream) {
+    // 192x768x384, 3 715 / 3 655 and 2 150 / 2 075.
+    // A short collision hides little and the streams' events cost 20 us, so
+    // small lattices use one stream and larger blocks (two / one: 3 spheres on
+    // 32x64x32, FP64 77 / 48, FP32 77 / 46; 20 on 64x100x90, 93 / 73 and 86 /
+    // 60; 40 on 64x192x96, FP64 of 179 MB 112 / 102, FP32 of 90 MB 99 / 74; FP32
+    // of 140 MB 116 / 95, of 239 MB 149 / 140; FP64 of 280 MB 152 / 156).
+    const bool aside = 19 * h->g.S * h->elem > PART_ASIDE_BYTES;
+    if (aside && !h->pstream) {
         HIP_TRY(hipStreamCreateWithFlags(&h->pstream, hipStreamNonBlocking));
         for (hipEvent_t &e : h->pev)
             HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -2368,19 +2384,23 @@ int lbm_run_particles(lbm_channel *h, int istep0, int nsteps)
             if (rc)
                 return rc;
         }
-        HIP_TRY(hipEventRecord(h->pev[0], h->stream));
-        HIP_TRY(hipStreamWaitEvent(h->pstream, h->pev[0], 0));
+        if (aside) {
+            HIP_TRY(hipEventRecord(h->pev[0], h->stream));
+            HIP_TRY(hipStreamWaitEvent(h->pstream, h->pev[0], 0));
+        }
         pt->pg.fx = h->fc.fx; // beads_move's body force (pressure_force)
         pt->pg.fy = h->fc.fy;
         pt->pg.fz = h->fc.fz;
-        rc = dispatch_err(part_advance(pt->pg, pt->ps, h->pstream), "beads_move and beads_links");
+        rc = dispatch_err(part_advance(pt->pg, pt->ps, aside, aside ? h->pstream : h->stream), "beads_move and beads_links");
         // the join point; on every return below the main stream waits for it
         // first, so no later call races the side stream's writes
-        HIP_TRY(hipEventRecord(h->pev[1], h->pstream));
+        if (aside)
+            HIP_TRY(hipEventRecord(h->pev[1], h->pstream));
         if (!rc)
             rc = launch_step(h);
         if (rc) {
-            (void)hipStreamWaitEvent(h->stream, h->pev[1], 0);
+            if (aside)
+                (void)hipStreamWaitEvent(h->stream, h->pev[1], 0);
             return rc;
         }
         fields_from_cur(h); // macrovar
@@ -2388,7 +2408,8 @@ int lbm_run_particles(lbm_channel *h, int istep0, int nsteps)
         const long long istep = (long long)istep0 + s + 1;
         if (nave > 0 && istep % nave == 0)
             h->ave_pending = true;
-        HIP_TRY(hipStreamWaitEvent(h->stream, h->pev[1], 0));
+        if (aside)
+            HIP_TRY(hipStreamWaitEvent(h->stream, h->pev[1], 0));
         void *lat = h->lat[h->cur];
         e = h->prec == LBM_FP64   ? PartLaunch<0>::refill_inside(pt->pg, pt->ps, lat, h->stream)
             : h->prec == LBM_FP32 ? PartLaunch<1>::refill_inside(pt->pg, pt->ps, lat, h->stream)
@@ -2410,15 +2431,20 @@ int lbm_particles_get(lbm_channel *h, double *pos, double *vel, double *omg, dou
                       double *contact, double *lub)
 {
     CHECK_P(h);
-    const PartState &ps = h->part->ps;
-    const size_t b = 3 * (size_t)h->part->pg.np * sizeof(double);
-    const double *src[7] = {ps.X, ps.V, ps.W, ps.FH, ps.TQ, ps.FC, ps.FL};
+    // one copy (seven small ones and the check's took 127 us)
+    const size_t n = 3 * (size_t)h->part->pg.np;
+    std::vector<double> all(PART_STATE / 3 * n + 1);
+    const HostPart part = {all.data(), h->part->ps.X, all.size() * sizeof(double)};
+    const int rc = copy_parts(h, &part, 1, true, "lbm_particles_get");
+    if (rc)
+        return rc;
     double *dst[7] = {pos, vel, omg, force, torque, contact, lub};
     for (int k = 0; k < 7; k++)
         if (dst[k])
-            HIP_TRY(hipMemcpyAsync(dst[k], src[k], b, hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    return check_overflow(h, "lbm_particles_get");
+            memcpy(dst[k], all.data() + (k == 0 ? 0 : k + 1) * n, n * sizeof(double));
+    int ovf;
+    memcpy(&ovf, &all.back(), sizeof(ovf));
+    return overflow_error(h, ovf, "lbm_particles_get");
 }
 
 int lbm_particles_links(lbm_channel *h, int *maxlink, int *counts, int *node, int *dir, double *q)

@@ -139,8 +139,9 @@ hipError_t part_solid_fields(const PartGeom &pg, const PartState &ps, double rho
 hipError_t part_sum(const PartGeom &pg, const PartState &ps, hipStream_t s);
 hipError_t part_move(const PartGeom &pg, const PartState &ps, hipStream_t s);
 // part_sum, part_move and part_classify (not the first) in fewer launches, but
-// for the link fractions; part_finish forms those and settles refilled nodes
-hipError_t part_advance(const PartGeom &pg, const PartState &ps, hipStream_t s);
+// for the link fractions; part_finish forms those and settles refilled nodes.
+// aside: in blocks that find room beside the collision
+hipError_t part_advance(const PartGeom &pg, const PartState &ps, bool aside, hipStream_t s);
 hipError_t part_finish(const PartGeom &pg, const PartState &ps, hipStream_t s);
 
 extern template struct PartLaunch<0>;

@@ -11,12 +11,14 @@ namespace {
 
 constexpr int PBLOCK = 256;
 // Threads of the kernels that walk a particle's box, one block per particle,
-// and the nodes a thread takes per pass: a box of 13^3-14^3 nodes (R = 5)
-// takes six passes, each a round trip to memory and a scan.  The main loop
-// runs them beside the collision, whose blocks of 256 threads leave room for
-// 256 when one of them ends; 512 threads waited for the collision's end (250
-// spheres on 96x384x192: link search 207 us, 114 with 256; 18 us alone).
-constexpr int BOXBLOCK = 256, BOXNODES = 2;
+// and the nodes a thread takes per pass: a box of 13^3-15^3 nodes (R = 5)
+// takes six or seven passes with 256 threads, each a scan of the block.  The
+// main loop runs them beside the collision of large lattices, whose blocks of
+// 256 threads leave room for 256 when one of them ends; 512 threads waited for
+// the collision's end (250 spheres on 96x384x192: link search 207 us, 114 with
+// 256).  With nothing beside them, BOXALONE threads: link search of 20 spheres
+// 20.7 us with 256, 11.1 with 1 024, commit and uncovering 9.9 / 6.0 us.
+constexpr int BOXBLOCK = 256, BOXALONE = 1024, BOXNODES = 2;
 constexpr int IBB_BLOCKS = 4; // blocks per particle for the cut links (~1000-2000 each at R = 5)
 
 // Waves of the kernels that run beside the collision issue ahead of its waves:
@@ -122,11 +124,12 @@ __device__ inline int block_scan(int v, int &total)
 // Block-wide exclusive scan of BOXNODES counts per thread: the counts of every
 // thread's first node come before those of the second.  Two counts of at most
 // 18 share an int.
-static_assert(BOXNODES == 2 && BOXBLOCK * 18 < 32768, "two 16-bit sums in an int");
+static_assert(BOXNODES == 2 && BOXALONE * 18 < 32768, "two 16-bit sums in an int");
+template <int NT>
 __device__ inline void box_scan(const int (&v)[BOXNODES], int (&off)[BOXNODES], int &total)
 {
     int t;
-    const int o = block_scan<BOXBLOCK>(v[0] | v[1] << 16, t);
+    const int o = block_scan<NT>(v[0] | v[1] << 16, t);
     const int t0 = t & 0xffff;
     off[0] = o & 0xffff;
     off[1] = t0 + (o >> 16);
@@ -143,6 +146,7 @@ constexpr int STAGE_FLAGS = 16384; // boxes with more nodes (R above about 10) r
 
 // Phase 1: nodes of particle p's previous box still marked p but no longer
 // inside become -2-p and join p's refill list (canonical box order).
+template <int NT>
 __device__ inline void uncover_of(const PartGeom &pg, const PartState &ps, int p, const double *Xold, const double *X)
 {
     const BoxNodes box(sphere_box(pg, Xold, 0));
@@ -150,27 +154,27 @@ __device__ inline void uncover_of(const PartGeom &pg, const PartState &ps, int p
     const bool staged = box.total <= STAGE_FLAGS;
     if (staged) {
 #pragma unroll 4
-        for (int e = threadIdx.x; e < box.total; e += BOXBLOCK) {
+        for (int e = threadIdx.x; e < box.total; e += NT) {
             int ix, iy, iz;
             mine[e] = ps.solid[box.at(e, pg.g, ix, iy, iz)] == p;
         }
     } // each thread reads back what it wrote
     int base = 0;
-    for (int c0 = 0; c0 < box.total; c0 += BOXBLOCK * BOXNODES) {
+    for (int c0 = 0; c0 < box.total; c0 += NT * BOXNODES) {
         int flag[BOXNODES] = {0, 0}, off[BOXNODES], tot;
         uint32_t n[BOXNODES];
         bool in[BOXNODES];
 #pragma unroll
         for (int h = 0; h < BOXNODES; h++) {
-            const int e = c0 + h * BOXBLOCK + threadIdx.x;
+            const int e = c0 + h * NT + threadIdx.x;
             int ix, iy, iz;
             n[h] = box.at(e < box.total ? e : 0, pg.g, ix, iy, iz);
             in[h] = e >= box.total || inside(pg, ix, iy, iz, X);
         }
 #pragma unroll
         for (int h = 0; h < BOXNODES; h++)
-            flag[h] = !in[h] && (staged ? mine[c0 + h * BOXBLOCK + threadIdx.x] != 0 : ps.solid[n[h]] == p);
-        box_scan(flag, off, tot);
+            flag[h] = !in[h] && (staged ? mine[c0 + h * NT + threadIdx.x] != 0 : ps.solid[n[h]] == p);
+        box_scan<NT>(flag, off, tot);
 #pragma unroll
         for (int h = 0; h < BOXNODES; h++)
             if (flag[h]) {
@@ -186,9 +190,9 @@ __device__ inline void uncover_of(const PartGeom &pg, const PartState &ps, int p
         ps.fill_count[p] = base < pg.maxfill ? base : pg.maxfill;
 }
 
-__global__ void __launch_bounds__(BOXBLOCK) k_p_uncover(PartGeom pg, PartState ps, const double *Xold)
+__global__ void __launch_bounds__(BOXALONE) k_p_uncover(PartGeom pg, PartState ps, const double *Xold)
 {
-    uncover_of(pg, ps, blockIdx.x, Xold + 3 * blockIdx.x, ps.X + 3 * blockIdx.x);
+    uncover_of<BOXALONE>(pg, ps, blockIdx.x, Xold + 3 * blockIdx.x, ps.X + 3 * blockIdx.x);
 }
 
 // Commits particle p's move (swaps new positions in, the previous ones are
@@ -214,12 +218,13 @@ __device__ inline void commit_of(const PartGeom &pg, const PartState &ps, double
 }
 
 // The main loop's commit and phase 1.
-__global__ void __launch_bounds__(BOXBLOCK) k_p_commit_uncover(PartGeom pg, PartState ps, double *Xold)
+template <int NT>
+__global__ void __launch_bounds__(NT) k_p_commit_uncover(PartGeom pg, PartState ps, double *Xold)
 {
     ahead_of_collision();
     double X[3], Xo[3];
     commit_of(pg, ps, Xold, blockIdx.x, X, Xo);
-    uncover_of(pg, ps, blockIdx.x, Xo, X);
+    uncover_of<NT>(pg, ps, blockIdx.x, Xo, X);
 }
 
 // Phase 2: claim the nodes inside particle p (smallest id wins an overlap).
@@ -243,7 +248,8 @@ __global__ void __launch_bounds__(BOXBLOCK) k_p_mark(PartGeom pg, PartState ps)
 // inside p.  Canonical order: box node (z, y, x), then direction 1..18.
 // A link is at most sqrt(2) long: nodes farther than R + 1.5 from the centre
 // cannot reach the sphere.
-__global__ void __launch_bounds__(BOXBLOCK) k_p_links(PartGeom pg, PartState ps)
+template <int NT>
+__global__ void __launch_bounds__(NT) k_p_links(PartGeom pg, PartState ps)
 {
     ahead_of_collision();
     const int p = blockIdx.x;
@@ -257,7 +263,7 @@ __global__ void __launch_bounds__(BOXBLOCK) k_p_links(PartGeom pg, PartState ps)
     if (staged) {
         const double isx = 1.0 / (double)sx, isxy = 1.0 / (double)(sx * sy);
 #pragma unroll 4
-        for (int e = threadIdx.x; e < sall; e += BOXBLOCK) {
+        for (int e = threadIdx.x; e < sall; e += NT) {
             const int kz = (int)(((double)e + 0.5) * isxy), r = e - kz * (sx * sy);
             const int ky = (int)(((double)r + 0.5) * isx);
             const int jx = box.b.x0 + (r - ky * sx) - 1;
@@ -270,11 +276,11 @@ __global__ void __launch_bounds__(BOXBLOCK) k_p_links(PartGeom pg, PartState ps)
     }
     __syncthreads();
     int base = 0;
-    for (int c0 = 0; c0 < box.total; c0 += BOXBLOCK * BOXNODES) {
+    for (int c0 = 0; c0 < box.total; c0 += NT * BOXNODES) {
         uint32_t mask[BOXNODES], n[BOXNODES];
 #pragma unroll
         for (int h = 0; h < BOXNODES; h++) {
-            const int e = c0 + h * BOXBLOCK + threadIdx.x;
+            const int e = c0 + h * NT + threadIdx.x;
             int ix = 0, iy = 0, iz = 0;
             mask[h] = 0;
             n[h] = 0;
@@ -326,7 +332,7 @@ __global__ void __launch_bounds__(BOXBLOCK) k_p_links(PartGeom pg, PartState ps)
 #pragma unroll
         for (int h = 0; h < BOXNODES; h++)
             cnt[h] = __builtin_popcount(mask[h]);
-        box_scan(cnt, off, tot);
+        box_scan<NT>(cnt, off, tot);
 #pragma unroll
         for (int h = 0; h < BOXNODES; h++) {
             int k = base + off[h];
@@ -922,10 +928,13 @@ static void launch_settle(const PartGeom &pg, const PartState &ps, hipStream_t s
     hipLaunchKernelGGL(k_p_settle, dim3(pg.np), dim3(64), 0, s, pg, ps);
 }
 
-static void launch_mark_links(const PartGeom &pg, const PartState &ps, hipStream_t s)
+static void launch_mark_links(const PartGeom &pg, const PartState &ps, bool aside, hipStream_t s)
 {
     hipLaunchKernelGGL(k_p_mark, dim3(pg.np), dim3(BOXBLOCK), 0, s, pg, ps);
-    hipLaunchKernelGGL(k_p_links, dim3(pg.np), dim3(BOXBLOCK), 0, s, pg, ps);
+    if (aside)
+        hipLaunchKernelGGL(k_p_links<BOXBLOCK>, dim3(pg.np), dim3(BOXBLOCK), 0, s, pg, ps);
+    else
+        hipLaunchKernelGGL(k_p_links<BOXALONE>, dim3(pg.np), dim3(BOXALONE), 0, s, pg, ps);
 }
 
 static void launch_fractions(const PartGeom &pg, const PartState &ps, hipStream_t s)
@@ -937,18 +946,21 @@ hipError_t part_classify(const PartGeom &pg, const PartState &ps, int first, hip
 {
     // ps.Aprev is not touched; Xold lives after X in the state (see lbm_capi)
     if (!first)
-        hipLaunchKernelGGL(k_p_uncover, dim3(pg.np), dim3(BOXBLOCK), 0, s, pg, ps, ps.X + 3 * (size_t)pg.np);
-    launch_mark_links(pg, ps, s);
+        hipLaunchKernelGGL(k_p_uncover, dim3(pg.np), dim3(BOXALONE), 0, s, pg, ps, ps.X + 3 * (size_t)pg.np);
+    launch_mark_links(pg, ps, false, s);
     launch_fractions(pg, ps, s);
     return hipGetLastError();
 }
 
-hipError_t part_advance(const PartGeom &pg, const PartState &ps, hipStream_t s)
+hipError_t part_advance(const PartGeom &pg, const PartState &ps, bool aside, hipStream_t s)
 {
     double *Xold = ps.X + 3 * (size_t)pg.np;
     hipLaunchKernelGGL(k_p_sum_move, dim3(pg.np), dim3(4 * SUMW), 0, s, pg, ps, Xold);
-    hipLaunchKernelGGL(k_p_commit_uncover, dim3(pg.np), dim3(BOXBLOCK), 0, s, pg, ps, Xold);
-    launch_mark_links(pg, ps, s);
+    if (aside)
+        hipLaunchKernelGGL(k_p_commit_uncover<BOXBLOCK>, dim3(pg.np), dim3(BOXBLOCK), 0, s, pg, ps, Xold);
+    else
+        hipLaunchKernelGGL(k_p_commit_uncover<BOXALONE>, dim3(pg.np), dim3(BOXALONE), 0, s, pg, ps, Xold);
+    launch_mark_links(pg, ps, aside, s);
     return hipGetLastError();
 }
 
