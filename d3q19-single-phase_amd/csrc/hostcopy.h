@@ -269,11 +269,11 @@ static __global__ void __launch_bounds__(LINK_BLOCK) k_link_copy(const LinkVec *
         ((char *)(dst + n))[threadIdx.x] = ((const char *)(src + n))[threadIdx.x];
 }
 
-// One slice between device memory and a pinned slot; device addresses that are
-// not on 16 bytes take the runtime's copy.
+// One slice between device memory and a pinned slot; addresses that are not on
+// 16 bytes take the runtime's copy, unless the tail's bytes are all there is.
 inline hipError_t link_copy(void *dst, const void *src, size_t bytes, bool down, hipStream_t s)
 {
-    if (((uintptr_t)dst | (uintptr_t)src) % sizeof(LinkVec))
+    if (bytes >= sizeof(LinkVec) && ((uintptr_t)dst | (uintptr_t)src) % sizeof(LinkVec))
         return hipMemcpyAsync(dst, src, bytes, down ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, s);
     const size_t n = bytes / sizeof(LinkVec), per = LINK_BLOCK * LINK_UNROLL;
     const unsigned grid =

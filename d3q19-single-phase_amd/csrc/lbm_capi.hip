@@ -94,6 +94,7 @@ struct lbm_channel {
     double *red_out;    // 2 doubles + NPLANE*lx doubles of final sums
     unsigned long long *errbits; // ERR_SLOTS maxima of rhoupdat, zero between calls; behind them the stop word of lbm_prerelax
     unsigned long long *errout;  // their maxima, PRE_ITERS words of pinned host memory (allocated on first use)
+    double *small;      // NPLANE*lx doubles (64 at least) of pinned memory for results the host reads (ensure_small)
     double *stat_acc;   // NPLANE*lx running sums
     long long stat_n;
     double *fstat_acc;  // NPLANE*(lx/2) running sums of the box-filtered fields (allocated on first use)
@@ -130,6 +131,7 @@ struct lbm_trainer {
     float *feat, *target;   // capacity x 10, capacity
     float *w, *m, *v;       // LBM_MLP_TOTAL parameters, Adam moments
     float *partial, *grad;  // per-block partial gradients, summed gradient (+ loss)
+    float *small;           // MLP_TOTAL floats of pinned memory for results the host reads
     uint32_t max_waves;
     int step;
     int target_mode; // LBM_TARGET_LOCAL or LBM_TARGET_PLANE for lbm_trainer_add_filtered
@@ -419,6 +421,33 @@ int launch_step(lbm_channel *h, bool fused = false, const unsigned long long *st
     return LBM_OK;
 }
 
+// Pinned memory that reductions store their results into: a copy to ordinary
+// memory takes 8-10 us longer.
+size_t small_bytes(const lbm_channel *h) { return std::max<size_t>(NPLANE * (size_t)h->g.lx, 64) * sizeof(double); }
+
+int ensure_small(lbm_channel *h)
+{
+    if (!h->small) {
+        const hipError_t e = hipHostMalloc((void **)&h->small, small_bytes(h), hipHostMallocDefault);
+        if (e != hipSuccess) {
+            h->small = nullptr;
+            return fail(LBM_ERR_NOMEM, "hipHostMalloc of the result buffer failed: %s", hipGetErrorString(e));
+        }
+    }
+    return LBM_OK;
+}
+
+// `bytes` of device memory, at most the buffer's size, into h->small.
+int read_small(lbm_channel *h, const void *src, size_t bytes)
+{
+    const int rc = ensure_small(h);
+    if (rc)
+        return rc;
+    HIP_TRY(link_copy(h->small, src, bytes, true, h->stream));
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    return LBM_OK;
+}
+
 const int *solid_of(const lbm_channel *h) { return h->part ? h->part->ps.solid : nullptr; }
 
 // Sum of rho over fluid nodes (SRC 0: field array, SRC 1: macrovar of the
@@ -436,19 +465,20 @@ int reduce_rho(lbm_channel *h, int src, double *sum, double *count)
     if (rc)
         return rc;
     // partials: sums in [0, grid), counts in [grid, 2*grid)
-    hipLaunchKernelGGL(k_sum_ordered, dim3(2), dim3(256), 0, h->stream, (const double *)h->partials, grid, h->red_out);
+    rc = ensure_small(h);
+    if (rc)
+        return rc;
+    hipLaunchKernelGGL(k_sum_ordered, dim3(2), dim3(256), 0, h->stream, (const double *)h->partials, grid, h->small);
     HIP_TRY(hipGetLastError());
-    double out[2];
-    HIP_TRY(hipMemcpyAsync(out, h->red_out, 2 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
-    *sum = out[0];
-    *count = out[1];
+    *sum = h->small[0];
+    *count = h->small[1];
     return LBM_OK;
 }
 
-// Plane sums of the current fields into red_out[0 .. 11*lx) (and the running
+// Plane sums of the current fields into out[0 .. 12*lx) (and the running
 // accumulator when acc is set).
-int plane_sums(lbm_channel *h, bool acc)
+int plane_sums(lbm_channel *h, double *out, bool acc)
 {
     PlaneArgs a;
     a.g = h->g;
@@ -469,7 +499,7 @@ int plane_sums(lbm_channel *h, bool acc)
         return rc;
     const uint32_t width = NPLANE * h->g.lx;
     hipLaunchKernelGGL(k_sum_columns, dim3((width + SUM_COLS - 1) / SUM_COLS), dim3(SUM_COLS * SUM_ROWS), 0, h->stream, a.partials, chunks, width,
-                       h->red_out + 2, acc ? h->stat_acc : (double *)nullptr);
+                       out, acc ? h->stat_acc : (double *)nullptr);
     HIP_TRY(hipGetLastError());
     return LBM_OK;
 }
@@ -748,6 +778,8 @@ int lbm_destroy(lbm_channel *h)
         (void)hipFree(h->errbits);
     if (h->errout)
         (void)hipHostFree(h->errout);
+    if (h->small)
+        (void)hipHostFree(h->small);
     if (h->stage)
         (void)hipFree(h->stage);
     if (h->part) {
@@ -1574,10 +1606,13 @@ int lbm_mass_sum(lbm_channel *h, double *mass)
     int rc = dispatch_err(PREC_CALL(h, mass_partials, a, grid, h->stream), "mass reduction");
     if (rc)
         return rc;
-    hipLaunchKernelGGL(k_sum_ordered, dim3(1), dim3(256), 0, h->stream, (const double *)h->partials, grid, h->red_out);
+    rc = ensure_small(h);
+    if (rc)
+        return rc;
+    hipLaunchKernelGGL(k_sum_ordered, dim3(1), dim3(256), 0, h->stream, (const double *)h->partials, grid, h->small);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(mass, h->red_out, sizeof(double), hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
+    *mass = h->small[0];
     return LBM_OK;
 }
 
@@ -1622,13 +1657,13 @@ int lbm_statistc2(lbm_channel *h, double ustar, double ystar, double *out)
     CHECK_H(h);
     if (!out)
         return fail(LBM_ERR_ARG, "lbm_statistc2: null output");
-    int rc = plane_sums(h, false);
+    int rc = ensure_small(h);
+    if (!rc)
+        rc = plane_sums(h, h->small, false);
     if (rc)
         return rc;
-    std::vector<double> s(NPLANE * (size_t)h->g.lx);
-    HIP_TRY(hipMemcpyAsync(s.data(), h->red_out + 2, s.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
-    stat_columns(h->g.lx, (double)h->g.ly * (double)h->g.lz, s.data(), 1.0, ustar, ystar, out);
+    stat_columns(h->g.lx, (double)h->g.ly * (double)h->g.lz, h->small, 1.0, ustar, ystar, out);
     return LBM_OK;
 }
 
@@ -1757,12 +1792,13 @@ int lbm_diag(lbm_channel *h, double ustar, double *out)
     int rc = dispatch_err(PREC_CALL(h, diag_partials, a, h->ms == ARRAYS ? 0 : 1, grid, h->stream), "diag");
     if (rc)
         return rc;
-    hipLaunchKernelGGL(k_diag_final, dim3(1), dim3(64 * 10), 0, h->stream, (const double *)h->partials, grid,
-                       h->red_out + 2);
+    rc = ensure_small(h);
+    if (rc)
+        return rc;
+    hipLaunchKernelGGL(k_diag_final, dim3(1), dim3(64 * 10), 0, h->stream, (const double *)h->partials, grid, h->small);
     HIP_TRY(hipGetLastError());
-    double t[DIAG_Q];
-    HIP_TRY(hipMemcpyAsync(t, h->red_out + 2, sizeof(t), hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
+    const double *t = h->small;
     // saveload.f90:1627-1640, in its order
     const double rn = t[6];
     double um = t[0] / rn, vm = t[1] / rn, wm = t[2] / rn;
@@ -1847,13 +1883,15 @@ int lbm_dissipation(lbm_channel *h, double tau, double ystar, double *out)
                           "dissipation");
     if (rc)
         return rc;
+    rc = ensure_small(h);
+    if (rc)
+        return rc;
     const uint32_t width = NDISS * h->g.lx;
-    hipLaunchKernelGGL(k_sum_columns, dim3((width + SUM_COLS - 1) / SUM_COLS), dim3(SUM_COLS * SUM_ROWS), 0, h->stream, a.partials, chunks, width,
-                       h->red_out + 2, (double *)nullptr);
+    hipLaunchKernelGGL(k_sum_columns, dim3((width + SUM_COLS - 1) / SUM_COLS), dim3(SUM_COLS * SUM_ROWS), 0, h->stream,
+                       a.partials, chunks, width, h->small, (double *)nullptr);
     HIP_TRY(hipGetLastError());
-    std::vector<double> t(width);
-    HIP_TRY(hipMemcpyAsync(t.data(), h->red_out + 2, width * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
+    const double *t = h->small;
     const int lx = h->g.lx;
     for (int i = 1; i <= lx; i++) { // saveload.f90:4857-4875
         const double nf = t[4 * (size_t)lx + i - 1];
@@ -1872,7 +1910,7 @@ int lbm_dissipation(lbm_channel *h, double tau, double ystar, double *out)
 int lbm_stats_accumulate(lbm_channel *h)
 {
     CHECK_H(h);
-    int rc = plane_sums(h, true);
+    int rc = plane_sums(h, h->red_out + 2, true);
     if (rc)
         return rc;
     h->stat_n++;
@@ -1888,10 +1926,10 @@ int lbm_stats_read(lbm_channel *h, double ustar, double ystar, double *out, long
         *nsamples = h->stat_n;
     if (h->stat_n == 0)
         return fail(LBM_ERR_STATE, "lbm_stats_read: no samples accumulated");
-    std::vector<double> s(NPLANE * (size_t)h->g.lx);
-    HIP_TRY(hipMemcpyAsync(s.data(), h->stat_acc, s.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    stat_columns(h->g.lx, (double)h->g.ly * (double)h->g.lz, s.data(), (double)h->stat_n, ustar, ystar, out);
+    const int rc = read_small(h, h->stat_acc, NPLANE * (size_t)h->g.lx * sizeof(double));
+    if (rc)
+        return rc;
+    stat_columns(h->g.lx, (double)h->g.ly * (double)h->g.lz, h->small, (double)h->stat_n, ustar, ystar, out);
     return LBM_OK;
 }
 
@@ -1929,11 +1967,10 @@ int lbm_stats_read_filtered(lbm_channel *h, double ustar, double ystar, double *
     if (h->fstat_n == 0)
         return fail(LBM_ERR_STATE, "lbm_stats_read_filtered: no samples accumulated");
     const uint32_t lxc = h->g.lx / 2;
-    std::vector<double> s(NPLANE * (size_t)lxc);
-    HIP_TRY(hipMemcpyAsync(s.data(), h->fstat_acc, s.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    stat_columns(lxc, (double)(h->g.ly / 2) * (double)(h->g.lz / 2), s.data(), (double)h->fstat_n, ustar, ystar,
-                 out);
+    const int rc = read_small(h, h->fstat_acc, NPLANE * (size_t)lxc * sizeof(double));
+    if (rc)
+        return rc;
+    stat_columns(lxc, (double)(h->g.ly / 2) * (double)(h->g.lz / 2), h->small, (double)h->fstat_n, ustar, ystar, out);
     return LBM_OK;
 }
 
@@ -2282,9 +2319,10 @@ static int overflow_error(const lbm_channel *h, int ovf, const char *what)
 
 static int check_overflow(lbm_channel *h, const char *what)
 {
-    int ovf = 0;
-    HIP_TRY(hipMemcpyAsync(&ovf, h->part->ps.overflow, sizeof(int), hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    int rc = read_small(h, h->part->ps.overflow, sizeof(int)), ovf = 0;
+    if (rc)
+        return rc;
+    memcpy(&ovf, h->small, sizeof(ovf));
     return overflow_error(h, ovf, what);
 }
 
@@ -2432,18 +2470,27 @@ int lbm_particles_get(lbm_channel *h, double *pos, double *vel, double *omg, dou
 {
     CHECK_P(h);
     // one copy (seven small ones and the check's took 127 us)
-    const size_t n = 3 * (size_t)h->part->pg.np;
-    std::vector<double> all(PART_STATE / 3 * n + 1);
-    const HostPart part = {all.data(), h->part->ps.X, all.size() * sizeof(double)};
-    const int rc = copy_parts(h, &part, 1, true, "lbm_particles_get");
+    const size_t n = 3 * (size_t)h->part->pg.np, bytes = (PART_STATE / 3 * n + 1) * sizeof(double);
+    std::vector<double> large;
+    const double *all = nullptr;
+    int rc;
+    if (bytes <= small_bytes(h)) {
+        rc = read_small(h, h->part->ps.X, bytes);
+        all = h->small;
+    } else {
+        large.resize(bytes / sizeof(double));
+        const HostPart part = {large.data(), h->part->ps.X, bytes};
+        rc = copy_parts(h, &part, 1, true, "lbm_particles_get");
+        all = large.data();
+    }
     if (rc)
         return rc;
     double *dst[7] = {pos, vel, omg, force, torque, contact, lub};
     for (int k = 0; k < 7; k++)
         if (dst[k])
-            memcpy(dst[k], all.data() + (k == 0 ? 0 : k + 1) * n, n * sizeof(double));
+            memcpy(dst[k], all + (k == 0 ? 0 : k + 1) * n, n * sizeof(double));
     int ovf;
-    memcpy(&ovf, &all.back(), sizeof(ovf));
+    memcpy(&ovf, all + PART_STATE / 3 * n, sizeof(ovf));
     return overflow_error(h, ovf, "lbm_particles_get");
 }
 
@@ -2587,7 +2634,8 @@ int lbm_trainer_create(int device, long long capacity, const float *params, lbm_
         hipMalloc((void **)&t->m, MLP_NPARAM * sizeof(float)) != hipSuccess ||
         hipMalloc((void **)&t->v, MLP_NPARAM * sizeof(float)) != hipSuccess ||
         hipMalloc((void **)&t->partial, (size_t)MLP_GRAD_BLOCKS * (MLP_NPARAM + 1) * sizeof(float)) != hipSuccess ||
-        hipMalloc((void **)&t->grad, (MLP_NPARAM + 1) * sizeof(float)) != hipSuccess)
+        hipMalloc((void **)&t->grad, (MLP_NPARAM + 1) * sizeof(float)) != hipSuccess ||
+        hipHostMalloc((void **)&t->small, MLP_TOTAL * sizeof(float), hipHostMallocDefault) != hipSuccess)
         return cleanup(fail(LBM_ERR_NOMEM, "lbm_trainer_create: device allocation failed"));
     if (hipMemcpyAsync(t->w, params, MLP_TOTAL * sizeof(float), hipMemcpyHostToDevice, t->stream) != hipSuccess ||
         hipMemsetAsync(t->m, 0, MLP_NPARAM * sizeof(float), t->stream) != hipSuccess ||
@@ -2609,6 +2657,8 @@ int lbm_trainer_destroy(lbm_trainer *t)
                     (void *)t->grad})
         if (p)
             (void)hipFree(p);
+    if (t->small)
+        (void)hipHostFree(t->small);
     if (t->stream)
         (void)hipStreamDestroy(t->stream);
     host_pool().release();
@@ -2779,13 +2829,12 @@ int lbm_trainer_grad(lbm_trainer *t, long long first, long long count, float *gr
         return rc;
     HIP_TRY(mlp_grad(t->w, t->feat, t->target, (uint32_t)first, (uint32_t)count, t->partial, t->grad, t->w, t->m,
                      t->v, 1, 0.0f, 0, t->stream));
-    std::vector<float> g(MLP_NPARAM + 1);
-    HIP_TRY(hipMemcpyAsync(g.data(), t->grad, g.size() * sizeof(float), hipMemcpyDeviceToHost, t->stream));
+    HIP_TRY(link_copy(t->small, t->grad, (MLP_NPARAM + 1) * sizeof(float), true, t->stream));
     HIP_TRY(hipStreamSynchronize(t->stream));
     if (grad)
-        memcpy(grad, g.data(), MLP_NPARAM * sizeof(float));
+        memcpy(grad, t->small, MLP_NPARAM * sizeof(float));
     if (loss)
-        *loss = g[MLP_NPARAM];
+        *loss = t->small[MLP_NPARAM];
     return LBM_OK;
 }
 
@@ -2810,11 +2859,10 @@ int lbm_trainer_train(lbm_trainer *t, long long first, long long count, int iter
                          t->w, t->m, t->v, t->step, lr, 1, t->stream));
         pos += batch;
     }
-    float g[MLP_NPARAM + 1];
-    HIP_TRY(hipMemcpyAsync(g, t->grad, sizeof(g), hipMemcpyDeviceToHost, t->stream));
+    HIP_TRY(link_copy(t->small, t->grad + MLP_NPARAM, sizeof(float), true, t->stream));
     HIP_TRY(hipStreamSynchronize(t->stream));
     if (loss)
-        *loss = g[MLP_NPARAM];
+        *loss = t->small[0];
     return LBM_OK;
 }
 
@@ -2859,8 +2907,9 @@ int lbm_trainer_params(lbm_trainer *t, float *params)
     CHECK_T(t);
     if (!params)
         return fail(LBM_ERR_ARG, "lbm_trainer_params: null output");
-    HIP_TRY(hipMemcpyAsync(params, t->w, MLP_TOTAL * sizeof(float), hipMemcpyDeviceToHost, t->stream));
+    HIP_TRY(link_copy(t->small, t->w, MLP_TOTAL * sizeof(float), true, t->stream));
     HIP_TRY(hipStreamSynchronize(t->stream));
+    memcpy(params, t->small, MLP_TOTAL * sizeof(float));
     return LBM_OK;
 }
 
