@@ -42,13 +42,15 @@ inline size_t host_slice(size_t total, bool down)
     return !down || total >= 64u << 20 ? HOST_SLICE : total >= 16u << 20 ? HOST_SLICE / 2 : HOST_SLICE / 4;
 }
 
-// Threads for a copy of `total` bytes: one (no thread is started) below 8
-// MiB.  Two keep up with the link where the array's pages are there; more
-// share the faults of a new array (11.2 MB of fields into one 1 570 us with
-// two, 1 060 with four; 28 MB of viscosities 837 us with three, 780 with six).
-inline int host_workers(size_t total)
+// Threads for a copy of `total` bytes: one (no thread is started) for downloads
+// below 8 MiB and uploads below 24 MiB.  Two keep up with the link where the
+// array's pages are there, as an upload's are (11.5 MB of samples 0.46 ms with
+// one, 0.52 with four); more share the faults of a new array (11.2 MB of fields
+// into one 1 570 us with two, 1 060 with four; 28 MB of viscosities 837 us with
+// three, 780 with six).
+inline int host_workers(size_t total, bool down)
 {
-    return total < 8u << 20 ? 1 : (int)std::min<size_t>(HOST_WORKERS, 2 + (total >> 22));
+    return total < (down ? 8u : 24u) << 20 ? 1 : (int)std::min<size_t>(HOST_WORKERS, 2 + (total >> 22));
 }
 
 // Copies with at least this many threads (16 MiB) use two streams.
@@ -305,7 +307,7 @@ inline hipError_t host_copy(int device, hipStream_t s, const HostPart *parts, in
         if (e != hipSuccess)
             return e;
     }
-    const int workers = host_workers(total);
+    const int workers = host_workers(total, down);
     if (total < HOST_MIN || !lock.try_lock() || !pool.ready(device, workers)) {
         for (int p = 0; p < nparts; p++)
             if (parts[p].host) {

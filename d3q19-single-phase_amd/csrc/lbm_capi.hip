@@ -895,7 +895,7 @@ int nodes_to_host(lbm_channel *h, void *const *out, int nout, size_t node_bytes,
     if (total >= HOST_MIN)
         HIP_TRY(hipStreamSynchronize(s));
     HostPool &pool = host_pool();
-    const int workers = host_workers(total);
+    const int workers = host_workers(total, true);
     std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
     hipError_t e = hipSuccess;
     const bool pooled = total >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device, workers);
@@ -946,7 +946,7 @@ int nodes_from_host(lbm_channel *h, const void *in, size_t node_bytes, const cha
     if (total >= HOST_MIN)
         HIP_TRY(hipStreamSynchronize(s));
     HostPool &pool = host_pool();
-    const int workers = host_workers(total);
+    const int workers = host_workers(total, false);
     std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
     hipError_t e = hipSuccess;
     if (total >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device, workers)) {
@@ -2118,7 +2118,7 @@ static int download_post_range(lbm_channel *h, uint64_t n0, uint64_t count, doub
     HIP_TRY(hipStreamSynchronize(s));
     HostPool &pool = host_pool();
     std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
-    const int workers = host_workers(19 * count * sizeof(double));
+    const int workers = host_workers(19 * count * sizeof(double), true);
     if (19 * count * h->elem >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device, workers)) {
         const uint64_t per = HOST_SLICE / h->elem, m = (count + per - 1) / per; // slices of a population
         const hipError_t e = host_slices_out(
@@ -2873,7 +2873,7 @@ int lbm_trainer_predict(lbm_trainer *t, long long first, long long count, float 
         return fail(LBM_ERR_ARG, "lbm_trainer_predict: bad range or null output");
     // as nodes_to_host: the kernel stores into the pinned slots
     const size_t total = (size_t)count * sizeof(float);
-    const int workers = host_workers(total);
+    const int workers = host_workers(total, true);
     hipError_t e = total >= HOST_MIN ? hipStreamSynchronize(t->stream) : hipSuccess;
     HostPool &pool = host_pool();
     std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
