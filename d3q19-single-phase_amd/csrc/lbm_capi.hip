@@ -93,7 +93,7 @@ struct lbm_channel {
     double *partials;   // 2*RED_BLOCKS doubles, then PLANE_CHUNKS*NPLANE*lx doubles
     double *red_out;    // 2 doubles + NPLANE*lx doubles of final sums
     unsigned long long *errbits; // ERR_SLOTS maxima of rhoupdat, zero between calls; behind them the stop word of lbm_prerelax
-    unsigned long long *errout;  // their maxima, PRE_ITERS words of pinned host memory (allocated on first use)
+    unsigned long long *errout;  // their maxima, pinned (allocated on first use): PRE_ITERS words of lbm_prerelax, one of rhoupdat
     double *small;      // NPLANE*lx doubles (64 at least) of pinned memory for results the host reads (ensure_small)
     double *stat_acc;   // NPLANE*lx running sums
     long long stat_n;
@@ -1283,13 +1283,16 @@ int lbm_macrovar(lbm_channel *h, double *rho, double *ux, double *uy, double *uz
                          });
 }
 
-// Pinned results of rhoupdat: an iteration of lbm_prerelax each.
+// Pinned results of rhoupdat: a word for each iteration of lbm_prerelax, whose
+// loop prepares and reads them without waiting for the stream, and behind them
+// one of lbm_rhoupdat's own, whose kernel may still be queued by then when the
+// caller did not ask for the maximum.
 constexpr int PRE_ITERS = 64;
 
 static int ensure_errout(lbm_channel *h)
 {
     if (!h->errout)
-        HIP_TRY(hipHostMalloc((void **)&h->errout, PRE_ITERS * sizeof(unsigned long long), hipHostMallocDefault));
+        HIP_TRY(hipHostMalloc((void **)&h->errout, (PRE_ITERS + 1) * sizeof(unsigned long long), hipHostMallocDefault));
     return LBM_OK;
 }
 
@@ -1312,13 +1315,14 @@ int lbm_rhoupdat(lbm_channel *h, double *rhoerrmax)
     // the device writes the result where the host reads it: the loop waits for
     // this value every iteration (a copy to ordinary memory and the clearing
     // of the slots before the kernel took 12 us longer)
-    hipLaunchKernelGGL(k_err_final, dim3(1), dim3(ERR_SLOTS), 0, h->stream, h->errbits, h->errout,
+    unsigned long long *const out = h->errout + PRE_ITERS;
+    hipLaunchKernelGGL(k_err_final, dim3(1), dim3(ERR_SLOTS), 0, h->stream, h->errbits, out,
                        (unsigned long long *)nullptr, 0.0, 0);
     HIP_TRY(hipGetLastError());
     h->fresh = false;
     if (rhoerrmax) {
         HIP_TRY(hipStreamSynchronize(h->stream));
-        memcpy(rhoerrmax, h->errout, sizeof(double));
+        memcpy(rhoerrmax, out, sizeof(double));
     }
     return LBM_OK;
 }
