@@ -1338,6 +1338,8 @@ constexpr int PRE_AHEAD = 4;
 static int prerelax_fused(lbm_channel *h, double rhoepsl, int niter, int *done, double *rhoerrmax)
 {
     constexpr unsigned long long PENDING = ~0ull; // no fabs() has these bits
+    constexpr unsigned long long UNKNOWN = 0x7ff8ull << 48; // a NaN
+    *done = 0;
     int rc = ensure_errout(h);
     if (rc)
         return rc;
@@ -1353,12 +1355,15 @@ static int prerelax_fused(lbm_channel *h, double rhoepsl, int niter, int *done, 
             rc = launch_step(h, true, sent ? stop : nullptr);
             if (rc)
                 break;
-            hipLaunchKernelGGL(k_err_final, dim3(1), dim3(ERR_SLOTS), 0, h->stream, h->errbits, h->errout + sent, stop,
-                               rhoepsl, sent == 0);
-            rc = dispatch_err(hipGetLastError(), "prerelax");
-            if (rc)
-                break;
             sent++;
+            hipLaunchKernelGGL(k_err_final, dim3(1), dim3(ERR_SLOTS), 0, h->stream, h->errbits, h->errout + sent - 1,
+                               stop, rhoepsl, sent == 1);
+            rc = dispatch_err(hipGetLastError(), "prerelax");
+            if (rc) { // a step without its maximum
+                out[sent - 1] = UNKNOWN;
+                (void)hipMemsetAsync(h->errbits, 0, ERR_SLOTS * ERR_STRIDE * sizeof(unsigned long long), h->stream);
+                break;
+            }
             continue;
         }
         unsigned long long u;
@@ -1381,9 +1386,17 @@ static int prerelax_fused(lbm_channel *h, double rhoepsl, int niter, int *done, 
         seen++;
     }
     // what ran after the end had no effect; its results are written before the
-    // next call's
-    if (sent > seen && !rc)
-        rc = dispatch_err(hipStreamSynchronize(h->stream), "prerelax");
+    // next call's.  After an error the iterations in flight still take effect.
+    if (sent > seen) {
+        const hipError_t e = hipStreamSynchronize(h->stream);
+        if (!rc)
+            rc = dispatch_err(e, "prerelax");
+        for (; !end && seen < sent && out[seen] != PENDING; seen++) {
+            const unsigned long long u = out[seen];
+            memcpy(&rhoerrmax[seen], &u, sizeof(u));
+            end = rhoerrmax[seen] <= rhoepsl;
+        }
+    }
     h->cur = cur0 ^ (seen & 1);
     *done = seen;
     return rc;
@@ -1400,7 +1413,7 @@ int lbm_prerelax(lbm_channel *h, double rhoepsl, int niter, int *done, double *r
         return rc;
     const bool fused = !h->part && !h->mlp && !h->fc.tab;
     while (*done < niter) {
-        int n = 1;
+        int n = 0;
         double *err = rhoerrmax + *done;
         if (fused) {
             rc = prerelax_fused(h, rhoepsl, std::min(niter - *done, PRE_ITERS), &n, err);
@@ -1408,10 +1421,11 @@ int lbm_prerelax(lbm_channel *h, double rhoepsl, int niter, int *done, double *r
             rc = lbm_rhoupdat(h, err);
             if (!rc)
                 rc = launch_step(h);
+            n = rc ? 0 : 1;
         }
+        *done += n;
         if (rc)
             return rc;
-        *done += n;
         if (err[n - 1] <= rhoepsl)
             break;
     }

@@ -167,7 +167,8 @@ int lbm_rhoupdat(lbm_channel *h, double *rhoerrmax);
 /* Up to niter iterations of the pre-relaxation loop, Channel-Flow/main.f90:70-90
  * (rhoupdat, collision_MRT), ending after the first whose max |rho_new - rho_old|
  * is at most rhoepsl.  *done receives their number, rhoerrmax[0 .. *done-1]
- * their maxima (niter values of room). */
+ * their maxima (niter values of room); after an error, those of the iterations
+ * that took effect before it. */
 int lbm_prerelax(lbm_channel *h, double rhoepsl, int niter, int *done, double *rhoerrmax);
 
 /* avedensity, Channel-Flow/collision.f90:487-513: subtracts the mean density

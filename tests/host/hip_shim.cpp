@@ -1,0 +1,44 @@
+// Runtime calls that fail on request or are counted, for tests of error paths
+// and fallbacks: loaded with RTLD_GLOBAL before liblbm.so, its definitions are
+// the ones liblbm.so binds to.  Nothing here reaches the GPU by itself.
+#include <dlfcn.h>
+#include <stddef.h>
+
+extern "C" {
+
+int shim_fail_host_malloc = 0;      // hipHostMalloc: out of memory
+int shim_fail_query = 0;             // hipStreamQuery: the next so many calls fail
+unsigned long long shim_malloc_bytes = 0; // bytes asked of hipMalloc so far
+
+static void *real(const char *name)
+{
+    static void *lib = dlopen("libamdhip64.so.7", RTLD_NOW | RTLD_LOCAL);
+    return lib ? dlsym(lib, name) : nullptr;
+}
+
+int hipHostMalloc(void **p, size_t bytes, unsigned flags)
+{
+    if (shim_fail_host_malloc)
+        return 2; // hipErrorOutOfMemory
+    static auto f = (int (*)(void **, size_t, unsigned))real("hipHostMalloc");
+    return f(p, bytes, flags);
+}
+
+int hipStreamQuery(void *stream)
+{
+    if (shim_fail_query > 0) {
+        shim_fail_query--;
+        return 999; // hipErrorUnknown
+    }
+    static auto f = (int (*)(void *))real("hipStreamQuery");
+    return f(stream);
+}
+
+int hipMalloc(void **p, size_t bytes)
+{
+    shim_malloc_bytes += bytes;
+    static auto f = (int (*)(void **, size_t))real("hipMalloc");
+    return f(p, bytes);
+}
+
+} // extern "C"
