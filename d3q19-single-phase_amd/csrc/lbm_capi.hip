@@ -94,7 +94,8 @@ struct lbm_channel {
     double *red_out;    // 2 doubles + NPLANE*lx doubles of final sums
     unsigned long long *errbits; // ERR_SLOTS maxima of rhoupdat, zero between calls; behind them the stop word of lbm_prerelax
     unsigned long long *errout;  // their maxima, pinned (allocated on first use): PRE_ITERS words of lbm_prerelax, one of rhoupdat
-    double *small;      // NPLANE*lx doubles (64 at least) of pinned memory for results the host reads (ensure_small)
+    double *small;      // NPLANE*lx doubles (64 at least) for results the host reads (ensure_small)
+    bool small_pinned;  // the device can store into it
     double *stat_acc;   // NPLANE*lx running sums
     long long stat_n;
     double *fstat_acc;  // NPLANE*(lx/2) running sums of the box-filtered fields (allocated on first use)
@@ -131,7 +132,8 @@ struct lbm_trainer {
     float *feat, *target;   // capacity x 10, capacity
     float *w, *m, *v;       // LBM_MLP_TOTAL parameters, Adam moments
     float *partial, *grad;  // per-block partial gradients, summed gradient (+ loss)
-    float *small;           // MLP_TOTAL floats of pinned memory for results the host reads
+    float *small;           // MLP_TOTAL floats for results the host reads
+    bool small_pinned;      // the device can store into it
     uint32_t max_waves;
     int step;
     int target_mode; // LBM_TARGET_LOCAL or LBM_TARGET_PLANE for lbm_trainer_add_filtered
@@ -421,19 +423,56 @@ int launch_step(lbm_channel *h, bool fused = false, const unsigned long long *st
     return LBM_OK;
 }
 
-// Pinned memory that reductions store their results into: a copy to ordinary
-// memory takes 8-10 us longer.
+// Memory for small results the host reads: pinned, or ordinary where no pinned
+// memory is to be had.
+void *small_alloc(size_t bytes, bool *pinned)
+{
+    void *p = nullptr;
+    *pinned = hipHostMalloc(&p, bytes, hipHostMallocDefault) == hipSuccess;
+    if (*pinned)
+        return p;
+    (void)hipGetLastError();
+    return malloc(bytes);
+}
+
+void small_free(void *p, bool pinned)
+{
+    if (pinned)
+        (void)hipHostFree(p);
+    else
+        free(p);
+}
+
+hipError_t small_copy(void *small, bool pinned, const void *src, size_t bytes, hipStream_t s)
+{
+    const hipError_t e = pinned ? link_copy(small, src, bytes, true, s)
+                                : hipMemcpyAsync(small, src, bytes, hipMemcpyDeviceToHost, s);
+    return e != hipSuccess ? e : hipStreamSynchronize(s);
+}
+
 size_t small_bytes(const lbm_channel *h) { return std::max<size_t>(NPLANE * (size_t)h->g.lx, 64) * sizeof(double); }
 
 int ensure_small(lbm_channel *h)
 {
     if (!h->small) {
-        const hipError_t e = hipHostMalloc((void **)&h->small, small_bytes(h), hipHostMallocDefault);
-        if (e != hipSuccess) {
-            h->small = nullptr;
-            return fail(LBM_ERR_NOMEM, "hipHostMalloc of the result buffer failed: %s", hipGetErrorString(e));
-        }
+        h->small = (double *)small_alloc(small_bytes(h), &h->small_pinned);
+        if (!h->small)
+            return fail(LBM_ERR_NOMEM, "allocation of the result buffer failed");
     }
+    return LBM_OK;
+}
+
+// Where a reduction stores what the host reads next (at most NPLANE * lx
+// doubles, after ensure_small): straight to the pinned buffer, since a copy to
+// ordinary memory takes 8-10 us longer, or to device memory without one.
+double *results_at(const lbm_channel *h) { return h->small_pinned ? h->small : h->red_out + 2; }
+
+// The n doubles stored there, in h->small.
+int results(lbm_channel *h, size_t n)
+{
+    if (!h->small_pinned)
+        HIP_TRY(hipMemcpyAsync(h->small, h->red_out + 2, n * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    HIP_TRY(hipStreamSynchronize(h->stream));
     return LBM_OK;
 }
 
@@ -443,8 +482,7 @@ int read_small(lbm_channel *h, const void *src, size_t bytes)
     const int rc = ensure_small(h);
     if (rc)
         return rc;
-    HIP_TRY(link_copy(h->small, src, bytes, true, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    HIP_TRY(small_copy(h->small, h->small_pinned, src, bytes, h->stream));
     return LBM_OK;
 }
 
@@ -468,9 +506,12 @@ int reduce_rho(lbm_channel *h, int src, double *sum, double *count)
     rc = ensure_small(h);
     if (rc)
         return rc;
-    hipLaunchKernelGGL(k_sum_ordered, dim3(2), dim3(256), 0, h->stream, (const double *)h->partials, grid, h->small);
+    hipLaunchKernelGGL(k_sum_ordered, dim3(2), dim3(256), 0, h->stream, (const double *)h->partials, grid,
+                       results_at(h));
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    rc = results(h, 2);
+    if (rc)
+        return rc;
     *sum = h->small[0];
     *count = h->small[1];
     return LBM_OK;
@@ -778,8 +819,7 @@ int lbm_destroy(lbm_channel *h)
         (void)hipFree(h->errbits);
     if (h->errout)
         (void)hipHostFree(h->errout);
-    if (h->small)
-        (void)hipHostFree(h->small);
+    small_free(h->small, h->small_pinned);
     if (h->stage)
         (void)hipFree(h->stage);
     if (h->part) {
@@ -1289,11 +1329,17 @@ int lbm_macrovar(lbm_channel *h, double *rho, double *ux, double *uy, double *uz
 // caller did not ask for the maximum.
 constexpr int PRE_ITERS = 64;
 
-static int ensure_errout(lbm_channel *h)
+// False without pinned memory: rhoupdat then takes its maximum from device
+// memory, and lbm_prerelax makes the calls one by one.
+static bool ensure_errout(lbm_channel *h)
 {
-    if (!h->errout)
-        HIP_TRY(hipHostMalloc((void **)&h->errout, (PRE_ITERS + 1) * sizeof(unsigned long long), hipHostMallocDefault));
-    return LBM_OK;
+    if (!h->errout &&
+        hipHostMalloc((void **)&h->errout, (PRE_ITERS + 1) * sizeof(unsigned long long), hipHostMallocDefault) !=
+            hipSuccess) {
+        (void)hipGetLastError();
+        h->errout = nullptr;
+    }
+    return h->errout != nullptr;
 }
 
 int lbm_rhoupdat(lbm_channel *h, double *rhoerrmax)
@@ -1303,9 +1349,7 @@ int lbm_rhoupdat(lbm_channel *h, double *rhoerrmax)
     int rc = materialize(h);
     if (rc)
         return rc;
-    rc = ensure_errout(h);
-    if (rc)
-        return rc;
+    const bool pinned = ensure_errout(h);
     MacroArgs a = macro_args(h, h->cur, 0, h->g.N);
     a.out[0] = h->mac[0];
     a.errbits = h->errbits;
@@ -1315,14 +1359,17 @@ int lbm_rhoupdat(lbm_channel *h, double *rhoerrmax)
     // the device writes the result where the host reads it: the loop waits for
     // this value every iteration (a copy to ordinary memory and the clearing
     // of the slots before the kernel took 12 us longer)
-    unsigned long long *const out = h->errout + PRE_ITERS;
+    unsigned long long *const out = pinned ? h->errout + PRE_ITERS : (unsigned long long *)h->red_out;
     hipLaunchKernelGGL(k_err_final, dim3(1), dim3(ERR_SLOTS), 0, h->stream, h->errbits, out,
                        (unsigned long long *)nullptr, 0.0, 0);
     HIP_TRY(hipGetLastError());
     h->fresh = false;
     if (rhoerrmax) {
+        if (!pinned)
+            HIP_TRY(hipMemcpyAsync(rhoerrmax, out, sizeof(double), hipMemcpyDeviceToHost, h->stream));
         HIP_TRY(hipStreamSynchronize(h->stream));
-        memcpy(rhoerrmax, out, sizeof(double));
+        if (pinned)
+            memcpy(rhoerrmax, out, sizeof(double));
     }
     return LBM_OK;
 }
@@ -1339,10 +1386,7 @@ static int prerelax_fused(lbm_channel *h, double rhoepsl, int niter, int *done, 
 {
     constexpr unsigned long long PENDING = ~0ull; // no fabs() has these bits
     constexpr unsigned long long UNKNOWN = 0x7ff8ull << 48; // a NaN
-    *done = 0;
-    int rc = ensure_errout(h);
-    if (rc)
-        return rc;
+    int rc = LBM_OK;
     unsigned long long *stop = h->errbits + ERR_SLOTS * ERR_STRIDE;
     volatile unsigned long long *out = h->errout;
     for (int k = 0; k < niter; k++)
@@ -1411,7 +1455,7 @@ int lbm_prerelax(lbm_channel *h, double rhoepsl, int niter, int *done, double *r
     int rc = materialize(h);
     if (rc)
         return rc;
-    const bool fused = !h->part && !h->mlp && !h->fc.tab;
+    const bool fused = !h->part && !h->mlp && !h->fc.tab && ensure_errout(h);
     while (*done < niter) {
         int n = 0;
         double *err = rhoerrmax + *done;
@@ -1627,9 +1671,12 @@ int lbm_mass_sum(lbm_channel *h, double *mass)
     rc = ensure_small(h);
     if (rc)
         return rc;
-    hipLaunchKernelGGL(k_sum_ordered, dim3(1), dim3(256), 0, h->stream, (const double *)h->partials, grid, h->small);
+    hipLaunchKernelGGL(k_sum_ordered, dim3(1), dim3(256), 0, h->stream, (const double *)h->partials, grid,
+                       results_at(h));
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    rc = results(h, 1);
+    if (rc)
+        return rc;
     *mass = h->small[0];
     return LBM_OK;
 }
@@ -1677,10 +1724,11 @@ int lbm_statistc2(lbm_channel *h, double ustar, double ystar, double *out)
         return fail(LBM_ERR_ARG, "lbm_statistc2: null output");
     int rc = ensure_small(h);
     if (!rc)
-        rc = plane_sums(h, h->small, false);
+        rc = plane_sums(h, results_at(h), false);
+    if (!rc)
+        rc = results(h, NPLANE * (size_t)h->g.lx);
     if (rc)
         return rc;
-    HIP_TRY(hipStreamSynchronize(h->stream));
     stat_columns(h->g.lx, (double)h->g.ly * (double)h->g.lz, h->small, 1.0, ustar, ystar, out);
     return LBM_OK;
 }
@@ -1813,9 +1861,12 @@ int lbm_diag(lbm_channel *h, double ustar, double *out)
     rc = ensure_small(h);
     if (rc)
         return rc;
-    hipLaunchKernelGGL(k_diag_final, dim3(1), dim3(64 * 10), 0, h->stream, (const double *)h->partials, grid, h->small);
+    hipLaunchKernelGGL(k_diag_final, dim3(1), dim3(64 * 10), 0, h->stream, (const double *)h->partials, grid,
+                       results_at(h));
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    rc = results(h, DIAG_Q);
+    if (rc)
+        return rc;
     const double *t = h->small;
     // saveload.f90:1627-1640, in its order
     const double rn = t[6];
@@ -1906,9 +1957,11 @@ int lbm_dissipation(lbm_channel *h, double tau, double ystar, double *out)
         return rc;
     const uint32_t width = NDISS * h->g.lx;
     hipLaunchKernelGGL(k_sum_columns, dim3((width + SUM_COLS - 1) / SUM_COLS), dim3(SUM_COLS * SUM_ROWS), 0, h->stream,
-                       a.partials, chunks, width, h->small, (double *)nullptr);
+                       a.partials, chunks, width, results_at(h), (double *)nullptr);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    rc = results(h, width);
+    if (rc)
+        return rc;
     const double *t = h->small;
     const int lx = h->g.lx;
     for (int i = 1; i <= lx; i++) { // saveload.f90:4857-4875
@@ -2652,9 +2705,11 @@ int lbm_trainer_create(int device, long long capacity, const float *params, lbm_
         hipMalloc((void **)&t->m, MLP_NPARAM * sizeof(float)) != hipSuccess ||
         hipMalloc((void **)&t->v, MLP_NPARAM * sizeof(float)) != hipSuccess ||
         hipMalloc((void **)&t->partial, (size_t)MLP_GRAD_BLOCKS * (MLP_NPARAM + 1) * sizeof(float)) != hipSuccess ||
-        hipMalloc((void **)&t->grad, (MLP_NPARAM + 1) * sizeof(float)) != hipSuccess ||
-        hipHostMalloc((void **)&t->small, MLP_TOTAL * sizeof(float), hipHostMallocDefault) != hipSuccess)
+        hipMalloc((void **)&t->grad, (MLP_NPARAM + 1) * sizeof(float)) != hipSuccess)
         return cleanup(fail(LBM_ERR_NOMEM, "lbm_trainer_create: device allocation failed"));
+    t->small = (float *)small_alloc(MLP_TOTAL * sizeof(float), &t->small_pinned);
+    if (!t->small)
+        return cleanup(fail(LBM_ERR_NOMEM, "lbm_trainer_create: allocation of the result buffer failed"));
     if (hipMemcpyAsync(t->w, params, MLP_TOTAL * sizeof(float), hipMemcpyHostToDevice, t->stream) != hipSuccess ||
         hipMemsetAsync(t->m, 0, MLP_NPARAM * sizeof(float), t->stream) != hipSuccess ||
         hipMemsetAsync(t->v, 0, MLP_NPARAM * sizeof(float), t->stream) != hipSuccess ||
@@ -2675,8 +2730,7 @@ int lbm_trainer_destroy(lbm_trainer *t)
                     (void *)t->grad})
         if (p)
             (void)hipFree(p);
-    if (t->small)
-        (void)hipHostFree(t->small);
+    small_free(t->small, t->small_pinned);
     if (t->stream)
         (void)hipStreamDestroy(t->stream);
     host_pool().release();
@@ -2847,8 +2901,7 @@ int lbm_trainer_grad(lbm_trainer *t, long long first, long long count, float *gr
         return rc;
     HIP_TRY(mlp_grad(t->w, t->feat, t->target, (uint32_t)first, (uint32_t)count, t->partial, t->grad, t->w, t->m,
                      t->v, 1, 0.0f, 0, t->stream));
-    HIP_TRY(link_copy(t->small, t->grad, (MLP_NPARAM + 1) * sizeof(float), true, t->stream));
-    HIP_TRY(hipStreamSynchronize(t->stream));
+    HIP_TRY(small_copy(t->small, t->small_pinned, t->grad, (MLP_NPARAM + 1) * sizeof(float), t->stream));
     if (grad)
         memcpy(grad, t->small, MLP_NPARAM * sizeof(float));
     if (loss)
@@ -2877,8 +2930,7 @@ int lbm_trainer_train(lbm_trainer *t, long long first, long long count, int iter
                          t->w, t->m, t->v, t->step, lr, 1, t->stream));
         pos += batch;
     }
-    HIP_TRY(link_copy(t->small, t->grad + MLP_NPARAM, sizeof(float), true, t->stream));
-    HIP_TRY(hipStreamSynchronize(t->stream));
+    HIP_TRY(small_copy(t->small, t->small_pinned, t->grad + MLP_NPARAM, sizeof(float), t->stream));
     if (loss)
         *loss = t->small[0];
     return LBM_OK;
@@ -2925,8 +2977,7 @@ int lbm_trainer_params(lbm_trainer *t, float *params)
     CHECK_T(t);
     if (!params)
         return fail(LBM_ERR_ARG, "lbm_trainer_params: null output");
-    HIP_TRY(link_copy(t->small, t->w, MLP_TOTAL * sizeof(float), true, t->stream));
-    HIP_TRY(hipStreamSynchronize(t->stream));
+    HIP_TRY(small_copy(t->small, t->small_pinned, t->w, MLP_TOTAL * sizeof(float), t->stream));
     memcpy(params, t->small, MLP_TOTAL * sizeof(float));
     return LBM_OK;
 }
