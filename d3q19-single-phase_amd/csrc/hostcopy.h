@@ -14,7 +14,10 @@
 // x HOST_DEPTH slots of HOST_SLICE bytes (48 MiB), each allocated by the first
 // copy that needs it and freed with the last handle (retain / release).  One
 // copy uses them at a time; a copy that finds them taken by another thread, or
-// cannot allocate them, goes the plain way.
+// cannot allocate them, goes the plain way.  So does one whose array the runtime
+// knows (runtime_array): it moves a pinned array at the link's rate by itself
+// (us through the slots / by the runtime: 11.2 MB of fields 329 / 256, 10 MB of
+// populations down 318 / 205, up 256 / 204).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -285,6 +288,20 @@ inline hipError_t link_copy(void *dst, const void *src, size_t bytes, bool down,
     return hipGetLastError();
 }
 
+// What the runtime knows the caller's array as: pinned (hipMemoryTypeHost),
+// managed, a device's, or nothing (hipMemoryTypeUnregistered).  Only the
+// runtime's own copies serve all of those.
+inline hipMemoryType array_type(const void *p)
+{
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return hipMemoryTypeUnregistered;
+    }
+    return a.type;
+}
+inline bool runtime_array(const void *p) { return array_type(p) != hipMemoryTypeUnregistered; }
+
 // One contiguous part of a copy; a null host pointer is skipped.
 struct HostPart {
     void *host;
@@ -297,18 +314,22 @@ struct HostPart {
 inline hipError_t host_copy(int device, hipStream_t s, const HostPart *parts, int nparts, bool down)
 {
     size_t total = 0;
+    bool known = false;
     for (int p = 0; p < nparts; p++)
         total += parts[p].host ? parts[p].bytes : 0;
+    for (int p = 0; p < nparts && total >= HOST_MIN; p++)
+        known = known || (parts[p].host && runtime_array(parts[p].host));
+    const bool sliced = total >= HOST_MIN && !known;
     HostPool &pool = host_pool();
     std::unique_lock<std::mutex> lock(pool.mu, std::defer_lock);
-    if (total >= HOST_MIN) {
+    if (sliced) {
         // what the stream still computes is waited for before the slots are taken
         const hipError_t e = hipStreamSynchronize(s);
         if (e != hipSuccess)
             return e;
     }
     const int workers = host_workers(total, down);
-    if (total < HOST_MIN || !lock.try_lock() || !pool.ready(device, workers)) {
+    if (!sliced || !lock.try_lock() || !pool.ready(device, workers)) {
         for (int p = 0; p < nparts; p++)
             if (parts[p].host) {
                 const hipError_t e =

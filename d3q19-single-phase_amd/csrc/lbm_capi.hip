@@ -927,18 +927,28 @@ int nodes_to_host(lbm_channel *h, void *const *out, int nout, size_t node_bytes,
 {
     char *host[4];
     int m = 0;
+    bool known = false;
     for (int j = 0; j < nout; j++)
         if (out[j])
             host[m++] = (char *)out[j];
     const hipStream_t s = h->stream;
     const size_t total = h->g.N * node_bytes * m;
-    if (total >= HOST_MIN)
+    // the runtime takes several pinned arrays one after another, 8 us each: up
+    // to 1 MiB for each after the first the slots are faster (us through the
+    // slots / by the runtime, 0.8 MB of fields 45 / 60, 2.1 MB 83 / 88, 5.2 MB
+    // 205 / 151)
+    for (int j = 0; j < m && total >= HOST_MIN; j++) {
+        const hipMemoryType t = array_type(host[j]);
+        known = known || (t == hipMemoryTypeHost ? total >= (size_t)(m - 1) << 20 : t != hipMemoryTypeUnregistered);
+    }
+    const bool sliced = total >= HOST_MIN && !known;
+    if (sliced)
         HIP_TRY(hipStreamSynchronize(s));
     HostPool &pool = host_pool();
     const int workers = host_workers(total, true);
-    std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
+    std::unique_lock<std::mutex> lock(pool.mu, std::defer_lock);
     hipError_t e = hipSuccess;
-    const bool pooled = total >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device, workers);
+    const bool pooled = sliced && lock.try_lock() && pool.ready(h->cfg.device, workers);
     if (staged || !pooled) {
         const int rc = ensure_stage(h);
         if (rc)
@@ -983,13 +993,14 @@ int nodes_from_host(lbm_channel *h, const void *in, size_t node_bytes, const cha
     const char *const host = (const char *)in;
     const hipStream_t s = h->stream;
     const size_t total = h->g.N * node_bytes;
-    if (total >= HOST_MIN)
+    const bool sliced = total >= HOST_MIN && !runtime_array(host);
+    if (sliced)
         HIP_TRY(hipStreamSynchronize(s));
     HostPool &pool = host_pool();
     const int workers = host_workers(total, false);
-    std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
+    std::unique_lock<std::mutex> lock(pool.mu, std::defer_lock);
     hipError_t e = hipSuccess;
-    if (total >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device, workers)) {
+    if (sliced && lock.try_lock() && pool.ready(h->cfg.device, workers)) {
         const NodeSlices sl(h->g.N, node_bytes, host_slice(total, false));
         e = host_slices_in(
             pool, h->cfg.device, s, sl.count(), workers,
@@ -2188,9 +2199,10 @@ static int download_post_range(lbm_channel *h, uint64_t n0, uint64_t count, doub
     const hipStream_t s = h->stream;
     HIP_TRY(hipStreamSynchronize(s));
     HostPool &pool = host_pool();
-    std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
+    std::unique_lock<std::mutex> lock(pool.mu, std::defer_lock);
     const int workers = host_workers(19 * count * sizeof(double), true);
-    if (19 * count * h->elem >= HOST_MIN && lock.owns_lock() && pool.ready(h->cfg.device, workers)) {
+    const bool sliced = 19 * count * h->elem >= HOST_MIN && !runtime_array(out);
+    if (sliced && lock.try_lock() && pool.ready(h->cfg.device, workers)) {
         const uint64_t per = HOST_SLICE / h->elem, m = (count + per - 1) / per; // slices of a population
         const hipError_t e = host_slices_out(
             pool, h->cfg.device, s, 19 * m, workers,
@@ -2205,6 +2217,13 @@ static int download_post_range(lbm_channel *h, uint64_t n0, uint64_t count, doub
             });
         if (e != hipSuccess)
             return fail(LBM_ERR_HIP, "lattice download: %s", hipGetErrorString(e));
+        return LBM_OK;
+    }
+    if (h->prec == LBM_FP64) { // nothing to widen
+        for (int i = 0; i < 19; i++)
+            HIP_TRY(hipMemcpyAsync(out + (size_t)i * count, L + ((size_t)i * S + n0) * sizeof(double),
+                                   count * sizeof(double), hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
         return LBM_OK;
     }
     std::vector<unsigned char> buf(count * h->elem);
@@ -2944,10 +2963,11 @@ int lbm_trainer_predict(lbm_trainer *t, long long first, long long count, float 
     // as nodes_to_host: the kernel stores into the pinned slots
     const size_t total = (size_t)count * sizeof(float);
     const int workers = host_workers(total, true);
-    hipError_t e = total >= HOST_MIN ? hipStreamSynchronize(t->stream) : hipSuccess;
+    const bool sliced = total >= HOST_MIN && !runtime_array(out);
+    hipError_t e = sliced ? hipStreamSynchronize(t->stream) : hipSuccess;
     HostPool &pool = host_pool();
-    std::unique_lock<std::mutex> lock(pool.mu, std::try_to_lock);
-    if (e == hipSuccess && total >= HOST_MIN && lock.owns_lock() && pool.ready(t->device, workers)) {
+    std::unique_lock<std::mutex> lock(pool.mu, std::defer_lock);
+    if (e == hipSuccess && sliced && lock.try_lock() && pool.ready(t->device, workers)) {
         const size_t per = host_slice(total, true) / sizeof(float), n = ((size_t)count + per - 1) / per;
         auto here = [&](size_t k) { return std::min<size_t>(per, (size_t)count - k * per); };
         e = host_slices_out(

@@ -7,6 +7,7 @@
 extern "C" {
 
 int shim_fail_host_malloc = 0;      // hipHostMalloc: out of memory
+int shim_host_mallocs = 0;           // hipHostMalloc calls for 4 MiB and more so far
 int shim_fail_query = 0;             // hipStreamQuery: the next so many calls fail
 unsigned long long shim_malloc_bytes = 0; // bytes asked of hipMalloc so far
 
@@ -20,6 +21,8 @@ int hipHostMalloc(void **p, size_t bytes, unsigned flags)
 {
     if (shim_fail_host_malloc)
         return 2; // hipErrorOutOfMemory
+    if (bytes >= 4u << 20)
+        shim_host_mallocs++;
     static auto f = (int (*)(void **, size_t, unsigned))real("hipHostMalloc");
     return f(p, bytes, flags);
 }
