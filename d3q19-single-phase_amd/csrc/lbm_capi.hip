@@ -1385,7 +1385,12 @@ int lbm_rhoupdat(lbm_channel *h, double *rhoerrmax)
     return LBM_OK;
 }
 
-// Iterations ahead of the last one whose result the host has seen.
+// Iterations ahead of the last one whose result the host has seen.  The first of
+// a call runs alone (`hold`): from initpop's populations it often is the last, as
+// the equilibrium's own density changes by nothing, and the three iterations
+// after it would read the lattice for nothing (96x384x192, us of a loop of one
+// iteration: FP64 1 122, 461 alone, 844 with the calls one by one; FP32 709 / 269
+// / 621).  Two iterations with three in vain are still faster than two by calls.
 constexpr int PRE_AHEAD = 4;
 
 // The iterations run ahead of the host's test: it reads each maximum from
@@ -1393,7 +1398,7 @@ constexpr int PRE_AHEAD = 4;
 // and do nothing.  us per iteration, calls one by one / this loop: FP64
 // 16x32x32 21.6 / 7.9, 64x192x96 108 / 69, 96x384x192 655 / 444; FP32 20.4 /
 // 6.8, 64 / 41, 364 / 254.
-static int prerelax_fused(lbm_channel *h, double rhoepsl, int niter, int *done, double *rhoerrmax)
+static int prerelax_fused(lbm_channel *h, double rhoepsl, int niter, bool hold, int *done, double *rhoerrmax)
 {
     constexpr unsigned long long PENDING = ~0ull; // no fabs() has these bits
     constexpr unsigned long long UNKNOWN = 0x7ff8ull << 48; // a NaN
@@ -1406,7 +1411,7 @@ static int prerelax_fused(lbm_channel *h, double rhoepsl, int niter, int *done, 
     const int cur0 = h->cur;
     bool end = false;
     while (seen < niter && !end) {
-        if (sent < niter && sent - seen < PRE_AHEAD) {
+        if (sent < niter && sent - seen < (hold && seen == 0 ? 1 : PRE_AHEAD)) {
             rc = launch_step(h, true, sent ? stop : nullptr);
             if (rc)
                 break;
@@ -1471,7 +1476,7 @@ int lbm_prerelax(lbm_channel *h, double rhoepsl, int niter, int *done, double *r
         int n = 0;
         double *err = rhoerrmax + *done;
         if (fused) {
-            rc = prerelax_fused(h, rhoepsl, std::min(niter - *done, PRE_ITERS), &n, err);
+            rc = prerelax_fused(h, rhoepsl, std::min(niter - *done, PRE_ITERS), *done == 0, &n, err);
         } else {
             rc = lbm_rhoupdat(h, err);
             if (!rc)

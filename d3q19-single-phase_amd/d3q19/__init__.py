@@ -353,7 +353,7 @@ class Channel:
     def prerelax(self, rhoepsl=1.0e-5, maxiter=15000):
         """Pre-relaxation loop of Channel-Flow/main.f90:70-90 (u held fixed).
         Returns (iterations, last max|drho|)."""
-        istep, errs, done = 0, np.empty(64), ctypes.c_int()
+        istep, errs, done = 0, np.empty(256), ctypes.c_int()
         while True:
             n = int(min(errs.size, max(1, maxiter + 2 - istep)))
             _call("lbm_prerelax", self._h, rhoepsl, n, ctypes.byref(done), _ptr(errs))

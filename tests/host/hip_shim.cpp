@@ -8,7 +8,9 @@ extern "C" {
 
 int shim_fail_host_malloc = 0;      // hipHostMalloc: out of memory
 int shim_host_mallocs = 0;           // hipHostMalloc calls for 4 MiB and more so far
-int shim_fail_query = 0;             // hipStreamQuery: the next so many calls fail
+int shim_launches = 0;               // kernels launched so far
+int shim_fail_query = 0;             // hipStreamQuery: so many calls fail ...
+int shim_fail_query_from = 0;        // ... once so many kernels have been launched
 unsigned long long shim_malloc_bytes = 0; // bytes asked of hipMalloc so far
 
 static void *real(const char *name)
@@ -29,7 +31,7 @@ int hipHostMalloc(void **p, size_t bytes, unsigned flags)
 
 int hipStreamQuery(void *stream)
 {
-    if (shim_fail_query > 0) {
+    if (shim_fail_query > 0 && shim_launches >= shim_fail_query_from) {
         shim_fail_query--;
         return 999; // hipErrorUnknown
     }
@@ -42,6 +44,17 @@ int hipMalloc(void **p, size_t bytes)
     shim_malloc_bytes += bytes;
     static auto f = (int (*)(void **, size_t))real("hipMalloc");
     return f(p, bytes);
+}
+
+struct Dim3 {
+    unsigned x, y, z;
+};
+
+int hipLaunchKernel(const void *kernel, Dim3 grid, Dim3 block, void **args, size_t lds, void *stream)
+{
+    shim_launches++;
+    static auto f = (int (*)(const void *, Dim3, Dim3, void **, size_t, void *))real("hipLaunchKernel");
+    return f(kernel, grid, block, args, lds, stream);
 }
 
 } // extern "C"
