@@ -353,11 +353,26 @@ int materialize(lbm_channel *h)
     return LBM_OK;
 }
 
+// Whether the handle's next step is refused, before anything of it is launched.
+int step_check(const lbm_channel *h)
+{
+    const bool arrays = h->ms != FROM_CUR; // the previous lattice's fields go to the arrays first
+    if (h->part && (h->fc.tab || (!arrays && !same_force(h->fm, h->fc))))
+        return fail(LBM_ERR_STATE, "collision: particles need a uniform force that macrovar has seen "
+                                   "(FORCINGP is not combined with particles)");
+    if (h->mlp && (arrays || h->rho_off != 0.0)) // the closure runs with fused fields only
+        return fail(LBM_ERR_STATE, "collision: the learned closure needs fields from macrovar");
+    return LBM_OK;
+}
+
 // One step of the handle.  fused: an iteration of the pre-relaxation, whose
 // fields are in the arrays and whose force is uniform, without particles or
 // closure; it has no effect once *stop is not 0.
 int launch_step(lbm_channel *h, bool fused = false, const unsigned long long *stop = nullptr)
 {
+    const int refused = step_check(h);
+    if (refused)
+        return refused;
     StepArgs a;
     a.g = h->g;
     a.src = h->lat[h->cur];
@@ -392,12 +407,8 @@ int launch_step(lbm_channel *h, bool fused = false, const unsigned long long *st
     a.fm = h->fm;
     // a force that varies over the nodes, or fused fields formed with a force
     // other than the collision's
-    if (h->fc.tab || (h->ms != ARRAYS && !same_force(h->fm, h->fc))) {
-        if (h->part)
-            return fail(LBM_ERR_STATE, "collision: particles need a uniform force that macrovar has seen "
-                                       "(FORCINGP is not combined with particles)");
+    if (h->fc.tab || (h->ms != ARRAYS && !same_force(h->fm, h->fc)))
         mode |= 16;
-    }
     a.mlp = h->mlp;
     a.inv_ystar = h->mlp_inv_ystar;
     a.yscale = h->mlp_yscale;
@@ -407,11 +418,8 @@ int launch_step(lbm_channel *h, bool fused = false, const unsigned long long *st
     a.rho_out = h->mac[0];
     a.errbits = fused ? h->errbits : nullptr;
     a.stop = stop;
-    if (h->mlp) {
-        if (mode & 3) // the closure runs with fused fields only
-            return fail(LBM_ERR_STATE, "collision: the learned closure needs fields from macrovar");
+    if (h->mlp)
         mode |= 8;
-    }
     int rc = dispatch_err(PREC_CALL(h, step, a, mode, h->stream), "collision");
     if (rc)
         return rc;
@@ -2493,6 +2501,11 @@ int lbm_run_particles(lbm_channel *h, int istep0, int nsteps)
     }
     Part *pt = h->part;
     const int nave = pt->pg.nave;
+    // a step that the collision refuses moves nothing (later ones of the call
+    // follow their own macrovar and are not refused)
+    const int refused = nsteps > 0 ? step_check(h) : LBM_OK;
+    if (refused)
+        return refused;
     for (int s = 0; s < nsteps; s++) {
         // beads_collision: the bounce-back here, its sums below
         hipError_t e = h->prec == LBM_FP64   ? PartLaunch<0>::ibb(pt->pg, pt->ps, h->lat[h->cur], s > 0, h->stream)
