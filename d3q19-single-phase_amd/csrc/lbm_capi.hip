@@ -145,6 +145,7 @@ struct Part {
     PartGeom pg;
     PartState ps;
     std::vector<void *> allocs;
+    std::vector<double> host; // what lbm_particles_get reads, where it does not fit lbm_channel::small
 };
 
 namespace {
@@ -2305,6 +2306,8 @@ int lbm_particles_create(lbm_channel *h, const lbm_particle_config *pc, const do
                         p, X[0], X[1], X[2]);
     }
     Part *pt = new Part();
+    if ((PART_STATE * (size_t)pc->npart + 1) * sizeof(double) > small_bytes(h))
+        pt->host.resize(PART_STATE * (size_t)pc->npart + 1);
     PartGeom &pg = pt->pg;
     PartState &ps = pt->ps;
     memset(&pg, 0, sizeof(pg));
@@ -2579,17 +2582,15 @@ int lbm_particles_get(lbm_channel *h, double *pos, double *vel, double *omg, dou
     CHECK_P(h);
     // one copy (seven small ones and the check's took 127 us)
     const size_t n = 3 * (size_t)h->part->pg.np, bytes = (PART_STATE / 3 * n + 1) * sizeof(double);
-    std::vector<double> large;
     const double *all = nullptr;
     int rc;
     if (bytes <= small_bytes(h)) {
         rc = read_small(h, h->part->ps.X, bytes);
         all = h->small;
     } else {
-        large.resize(bytes / sizeof(double));
-        const HostPart part = {large.data(), h->part->ps.X, bytes};
+        const HostPart part = {h->part->host.data(), h->part->ps.X, bytes};
         rc = copy_parts(h, &part, 1, true, "lbm_particles_get");
-        all = large.data();
+        all = h->part->host.data();
     }
     if (rc)
         return rc;

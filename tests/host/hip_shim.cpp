@@ -3,6 +3,9 @@
 // the ones liblbm.so binds to.  Nothing here reaches the GPU by itself.
 #include <dlfcn.h>
 #include <stddef.h>
+#include <stdlib.h>
+
+#include <new>
 
 extern "C" {
 
@@ -11,6 +14,7 @@ int shim_host_mallocs = 0;           // hipHostMalloc calls for 4 MiB and more s
 int shim_launches = 0;               // kernels launched so far
 int shim_fail_query = 0;             // hipStreamQuery: so many calls fail ...
 int shim_fail_query_from = 0;        // ... once so many kernels have been launched
+unsigned long long shim_fail_new = 0; // operator new of exactly so many bytes throws
 unsigned long long shim_malloc_bytes = 0; // bytes asked of hipMalloc so far
 
 static void *real(const char *name)
@@ -58,3 +62,14 @@ int hipLaunchKernel(const void *kernel, Dim3 grid, Dim3 block, void **args, size
 }
 
 } // extern "C"
+
+void *operator new(size_t bytes)
+{
+    void *p = shim_fail_new && bytes == shim_fail_new ? nullptr : malloc(bytes ? bytes : 1);
+    if (!p)
+        throw std::bad_alloc();
+    return p;
+}
+
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
