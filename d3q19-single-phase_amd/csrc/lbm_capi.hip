@@ -59,6 +59,7 @@ enum MacroState { FROM_CUR = 0, FROM_PREV = 1, ARRAYS = 2 };
 constexpr uint32_t RED_BLOCKS = 2048;   // partial sums per reduction
 constexpr uint32_t DIAG_BLOCKS = 1024;  // partials per quantity of diag
 constexpr uint32_t PLANE_CHUNKS = 512;  // row chunks for plane sums
+constexpr size_t ERR_BYTES = (ERR_SLOTS * ERR_STRIDE + 1) * sizeof(unsigned long long); // lbm_channel::errbits
 constexpr size_t STAGE_BYTES = HOST_WORKERS * HOST_DEPTH * HOST_SLICE; // device side of the copy slices
 
 // Scratch of lbm_mass_sum_noalloc: the per-block partial sums of the mass
@@ -784,7 +785,7 @@ int lbm_create(const lbm_config *cfg, lbm_channel **out)
     if (hipMalloc((void **)&h->partials, part * sizeof(double)) != hipSuccess ||
         hipMalloc((void **)&h->red_out, (2 + NPLANE * (size_t)c.lx) * sizeof(double)) != hipSuccess ||
         hipMalloc((void **)&h->stat_acc, NPLANE * (size_t)c.lx * sizeof(double)) != hipSuccess ||
-        hipMalloc((void **)&h->errbits, (ERR_SLOTS * ERR_STRIDE + 1) * sizeof(unsigned long long)) != hipSuccess)
+        hipMalloc((void **)&h->errbits, ERR_BYTES) != hipSuccess)
         return cleanup(fail(LBM_ERR_NOMEM, "hipMalloc of reduction scratch failed"));
     e = hipMemsetAsync(h->stat_acc, 0, NPLANE * (size_t)c.lx * sizeof(double), h->stream);
     if (e == hipSuccess)
@@ -2158,7 +2159,7 @@ int lbm_device_bytes(lbm_channel *h, size_t *bytes)
         b += STAGE_BYTES;
     if (h->bring)
         b += (block_ring_elems(h->g, h->baxis, h->bK, h->bW) + block_head_elems(h->g, h->baxis, h->bW)) * h->elem;
-    b += (2 * RED_BLOCKS + (size_t)PLANE_CHUNKS * NPLANE * h->g.lx + 2 + 2 * NPLANE * (size_t)h->g.lx) * sizeof(double) + 8;
+    b += (2 * RED_BLOCKS + (size_t)PLANE_CHUNKS * NPLANE * h->g.lx + 2 + 2 * NPLANE * (size_t)h->g.lx) * sizeof(double) + ERR_BYTES;
     *bytes = b;
     return LBM_OK;
 }
