@@ -2174,6 +2174,15 @@ int lbm_block_info(lbm_channel *h, int *axis, int *slabs)
     return LBM_OK;
 }
 
+int lbm_block_pairs(lbm_channel *h, int *pairs)
+{
+    CHECK_H(h);
+    if (!pairs)
+        return fail(LBM_ERR_ARG, "lbm_block_pairs: null output");
+    *pairs = h->bK > 0 && !h->bskip;
+    return LBM_OK;
+}
+
 int lbm_block_rows(lbm_channel *h, int *rows)
 {
     CHECK_H(h);

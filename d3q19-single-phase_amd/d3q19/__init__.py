@@ -90,6 +90,7 @@ _SIGS = {
     "lbm_device_bytes": [_H, ctypes.POINTER(ctypes.c_size_t)],
     "lbm_block_info": [_H, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)],
     "lbm_block_rows": [_H, ctypes.POINTER(ctypes.c_int)],
+    "lbm_block_pairs": [_H, ctypes.POINTER(ctypes.c_int)],
     "lbm_download_post": [_H, _D],
     "lbm_download_post_range": [_H, ctypes.c_longlong, ctypes.c_longlong, _D],
     "lbm_particles_create": [_H, _D, _D, _D, _D],
@@ -441,10 +442,16 @@ class Channel:
         return v.value
 
     def block_info(self):
-        """The blocked sweep run() uses for pairs of steps: (axis 'z'|'y', slabs per chunk; 0 = off)."""
+        """The blocked sweep chosen for pairs of steps: (axis 'z'|'y', slabs per chunk; 0 = none)."""
         a, k = ctypes.c_int(), ctypes.c_int()
         _call("lbm_block_info", self._h, ctypes.byref(a), ctypes.byref(k))
         return chr(a.value), k.value
+
+    def block_pairs(self):
+        """Whether pairs of steps run as that sweep (small lattices run single steps)."""
+        v = ctypes.c_int()
+        _call("lbm_block_pairs", self._h, ctypes.byref(v))
+        return bool(v.value)
 
     def block_rows(self):
         """Rows per window of the blocked sweep's slabs (0: whole slabs)."""

@@ -187,7 +187,7 @@ int lbm_avedensity(lbm_channel *h, double *rhomean);
  * and lbm_block_rows report the choice.  Lattices of at most 300 MB, and those whose
  * slabs are so small that a chunk holds less than 90 MB, run their steps one
  * by one, which measures faster there, unless one of the sweep's variables is
- * set. */
+ * set; lbm_block_pairs tells which it is. */
 int lbm_run(lbm_channel *h, int nsteps);
 
 /* Sum of all populations in FP64 (mass monitor; the sum is invariant under
@@ -265,11 +265,18 @@ int lbm_time_steps(lbm_channel *h, int nsteps, double *avg_ms, double *total_ms)
 /* Device bytes held by the handle (lattices, fields, scratch). */
 int lbm_device_bytes(lbm_channel *h, size_t *bytes);
 
-/* The two-step blocked sweep lbm_run uses for pairs of steps, as lbm_create
- * chose it: *axis = 'z' (slabs of lx*ly nodes) or 'y' (lx*lz), *slabs = slabs
- * per chunk (0: single steps only).  Either pointer may be null.  No
- * reference counterpart (measurement and tests). */
+/* The two-step blocked sweep for pairs of steps, as lbm_create chose it: *axis
+ * = 'z' (slabs of lx*ly nodes) or 'y' (lx*lz), *slabs = slabs per chunk (0: no
+ * sweep).  Small lattices have one but run single steps (lbm_block_pairs).
+ * Either pointer may be null.  No reference counterpart (measurement and
+ * tests). */
 int lbm_block_info(lbm_channel *h, int *axis, int *slabs);
+
+/* *pairs = 1 where lbm_run, lbm_run_forcingp and the main loop's calls one by
+ * one run pairs of steps as that sweep, 0 where as single steps: without a
+ * sweep, and on lattices too small for it to pay (see lbm_run).  No reference
+ * counterpart (measurement and tests). */
+int lbm_block_pairs(lbm_channel *h, int *pairs);
 
 /* Rows per window of that sweep's slabs: 0 when it sweeps whole slabs.  A
  * lattice whose slabs are too large for a chunk of four in the ring (the
