@@ -105,7 +105,8 @@ struct lbm_channel {
     hipEvent_t ev[2];
     struct Part *part;  // rigid particles (nullptr without)
     hipStream_t pstream; // lbm_run_particles: the force sums and beads_move beside the collision
-    hipEvent_t pev[2];   // its fork (after the bounce-back) and join (before beads_links)
+    hipEvent_t pev[2];   // its fork (after the bounce-back) and join (before the refill)
+    int pstreams;        // streams of lbm_run_particles: 1, 2 or by the lattice's size (0)
     float *mlp;         // learned closure parameters on the device (nullptr: plain MRT)
     float mlp_inv_ystar, mlp_yscale;
     int runs;           // step kernel: 1 = vector runs where the shape allows, 0 = one node per thread
@@ -760,6 +761,14 @@ int lbm_create(const lbm_config *cfg, lbm_channel **out)
             return fail(LBM_ERR_ARG, "lbm_create: invalid value of LBM_DEFER (0 or 1)");
         }
         h->defer = (kd && strcmp(kd, "0") == 0) ? 0 : 1;
+        // LBM_PART_STREAMS=1|2: lbm_run_particles on so many streams (default:
+        // by the lattice's size)
+        const char *kp = getenv("LBM_PART_STREAMS");
+        if (kp && strcmp(kp, "1") != 0 && strcmp(kp, "2") != 0) {
+            (void)lbm_destroy(h);
+            return fail(LBM_ERR_ARG, "lbm_create: invalid value of LBM_PART_STREAMS (1 or 2)");
+        }
+        h->pstreams = kp ? kp[0] - '0' : 0;
     }
     fields_from_cur(h);
     h->fresh = true;
@@ -2506,7 +2515,7 @@ int lbm_run_particles(lbm_channel *h, int istep0, int nsteps)
     // 32x64x32, FP64 77 / 48, FP32 77 / 46; 20 on 64x100x90, 93 / 73 and 86 /
     // 60; 40 on 64x192x96, FP64 of 179 MB 112 / 102, FP32 of 90 MB 99 / 74; FP32
     // of 140 MB 116 / 95, of 239 MB 149 / 140; FP64 of 280 MB 152 / 156).
-    const bool aside = 19 * h->g.S * h->elem > PART_ASIDE_BYTES;
+    const bool aside = h->pstreams ? h->pstreams == 2 : 19 * h->g.S * h->elem > PART_ASIDE_BYTES;
     if (aside && !h->pstream) {
         HIP_TRY(hipStreamCreateWithFlags(&h->pstream, hipStreamNonBlocking));
         for (hipEvent_t &e : h->pev)
