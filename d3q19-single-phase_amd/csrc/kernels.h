@@ -204,7 +204,7 @@ __host__ __device__ inline PlaneRef plane_write_head(const PlaneStore &st, uint3
 // waves (slabp = slab rounded up to a multiple of 64), so every wave lies in
 // one slab and the slab's buffers and offsets are the same for all its lanes.
 // Thread t works on node t % slabt - slab_shift(res, s) of the launch's slab t /
-// slabt.  When whole z slabs of lx * ly nodes do not fill cache lines, res is
+// slabt (block_thread_slab, block_thread_node).  When whole z slabs of lx * ly nodes do not fill cache lines, res is
 // that count modulo 64 and slabt leaves room for the shift: a wave's nodes
 // then start on a line of the lattice, and of the ring, whose slots hold each
 // slab at the same shift.  Without it every wave stored two partial lines a
@@ -253,6 +253,15 @@ __host__ __device__ inline uint32_t block_plane(const BlockArgs &a, uint32_t sl)
     if (s >= (int32_t)a.ns)
         s -= (int32_t)a.ns;
     return (uint32_t)s;
+}
+
+// The launch's slab that thread t works on (the same for all lanes of a wave),
+// and its node of it, slab sb of the lattice: beyond a.slab, also below the
+// slab's shift, where the difference wraps, the thread has none.
+__host__ __device__ inline uint32_t block_thread_slab(const BlockArgs &a, uint32_t t) { return fdiv(t, a.dslabt); }
+__host__ __device__ inline uint32_t block_thread_node(const BlockArgs &a, uint32_t t, uint32_t sl, uint32_t sb)
+{
+    return t - sl * a.slabt - slab_shift(a.res, sb);
 }
 
 // The source slabs of slab s: index c + 1 holds slab s - c, for the sweep-axis

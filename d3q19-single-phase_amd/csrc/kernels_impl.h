@@ -578,11 +578,11 @@ __global__ void __launch_bounds__((plane_block<P, NT>())) k_step_planes(BlockArg
     const uint32_t t = blockIdx.x * plane_block<P, NT>() + threadIdx.x;
     // the wave's slab, uniform across its lanes (slabs are padded to whole
     // waves), so the slab buffers and offsets below stay in scalar registers
-    const uint32_t sl = __builtin_amdgcn_readfirstlane(fdiv(t, a.dslabt));
+    const uint32_t sl = __builtin_amdgcn_readfirstlane(block_thread_slab(a, t));
     if (sl >= a.count)
         return;
     const uint32_t sb = block_plane(a, sl);
-    const uint32_t w = t - sl * a.slabt - slab_shift(a.res, sb); // wraps below the shift
+    const uint32_t w = block_thread_node(a, t, sl, sb);
     if (w >= a.slab)
         return;
     const BlockRow br = block_row(a, w);
