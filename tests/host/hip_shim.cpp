@@ -12,6 +12,8 @@ extern "C" {
 int shim_fail_host_malloc = 0;      // hipHostMalloc: out of memory
 int shim_host_mallocs = 0;           // hipHostMalloc calls for 4 MiB and more so far
 int shim_launches = 0;               // kernels launched so far
+int shim_copies = 0;                 // hipMemcpyAsync calls so far
+int shim_streams = 0;                // streams created so far
 int shim_fail_query = 0;             // hipStreamQuery: so many calls fail ...
 int shim_fail_query_from = 0;        // ... once so many kernels have been launched
 unsigned long long shim_fail_new = 0; // operator new of exactly so many bytes throws
@@ -48,6 +50,20 @@ int hipMalloc(void **p, size_t bytes)
     shim_malloc_bytes += bytes;
     static auto f = (int (*)(void **, size_t))real("hipMalloc");
     return f(p, bytes);
+}
+
+int hipMemcpyAsync(void *dst, const void *src, size_t bytes, int kind, void *stream)
+{
+    shim_copies++;
+    static auto f = (int (*)(void *, const void *, size_t, int, void *))real("hipMemcpyAsync");
+    return f(dst, src, bytes, kind, stream);
+}
+
+int hipStreamCreateWithFlags(void **stream, unsigned flags)
+{
+    shim_streams++;
+    static auto f = (int (*)(void **, unsigned))real("hipStreamCreateWithFlags");
+    return f(stream, flags);
 }
 
 struct Dim3 {
