@@ -45,6 +45,12 @@ inline size_t host_slice(size_t total, bool down)
     return !down || total >= 64u << 20 ? HOST_SLICE : total >= 16u << 20 ? HOST_SLICE / 2 : HOST_SLICE / 4;
 }
 
+// Uploads below this size take three threads, which are as fast as six there
+// (33 MB in four arrays 908 us with three, 917-954 with six, 82 MB 1 893 / 1 865,
+// 184 MB 3 884 / 3 727) and need half of the slots, whose allocation the first
+// copy pays for.
+constexpr size_t HOST_UP_ALL = 96u << 20;
+
 // Threads for a copy of `total` bytes: one (no thread is started) for downloads
 // below 8 MiB and uploads below 24 MiB.  Two keep up with the link where the
 // array's pages are there, as an upload's are (11.5 MB of samples 0.46 ms with
@@ -53,8 +59,19 @@ inline size_t host_slice(size_t total, bool down)
 // three, 780 with six).
 inline int host_workers(size_t total, bool down)
 {
-    return total < (down ? 8u : 24u) << 20 ? 1 : (int)std::min<size_t>(HOST_WORKERS, 2 + (total >> 22));
+    if (total < (down ? 8u : 24u) << 20)
+        return 1;
+    const size_t most = down || total >= HOST_UP_ALL ? HOST_WORKERS : 3;
+    return (int)std::min<size_t>(most, 2 + (total >> 22));
 }
+
+// Whole arrays from the host that go the plain way although they are large
+// enough: one thread fills the slots no faster than the runtime its own pinned
+// buffers from 2 MiB on, and several do from 26 MiB on (us from arrays not seen
+// before, runtime / slots: 0.5 MB 31 / 35, 2.1 MB in four 102 / 103, 2.9 MB 114 /
+// 136, 4.4 MB 153 / 183, 17.6 MB in four 607 / 905, 24.6 MB in four 867 / 1 091,
+// 29 MB 1 080 / 866, 33 MB in four 1 207 / 954, 41 MB 1 571 / 1 147).
+constexpr size_t HOST_UP_PLAIN = 2u << 20, HOST_UP_MANY = 26u << 20;
 
 // Copies with at least this many threads (16 MiB) use two streams.
 constexpr int HOST_SIDE_WORKERS = 6;
@@ -196,7 +213,7 @@ hipError_t host_slices_out(HostPool &pool, int device, hipStream_t s, size_t n, 
     for (int w = 1; w < HOST_WORKERS; w++)
         if (t[w].joinable())
             t[w].join();
-    const hipError_t e = hipStreamSynchronize(s), e2 = hipStreamSynchronize(odd);
+    const hipError_t e = hipStreamSynchronize(s), e2 = odd == s ? e : hipStreamSynchronize(odd);
     return err.load() != (int)hipSuccess ? (hipError_t)err.load() : e != hipSuccess ? e : e2;
 }
 
@@ -223,7 +240,8 @@ hipError_t host_slices_in(HostPool &pool, int device, hipStream_t s, size_t n, i
             produce(k, pool.slot[slot]);
             const hipStream_t on = k % 2 ? odd : s;
             e = enqueue(k, slot, pool.slot[slot], on);
-            if (e == hipSuccess)
+            // the only worker's last slices are not waited for one by one
+            if (e == hipSuccess && (workers > 1 || k + HOST_DEPTH < n))
                 e = hipEventRecord(pool.ev[slot], on);
         }
         int ok = (int)hipSuccess;
@@ -241,7 +259,7 @@ hipError_t host_slices_in(HostPool &pool, int device, hipStream_t s, size_t n, i
     for (int w = 1; w < HOST_WORKERS; w++)
         if (t[w].joinable())
             t[w].join();
-    const hipError_t e = hipStreamSynchronize(s), e2 = hipStreamSynchronize(odd);
+    const hipError_t e = hipStreamSynchronize(s), e2 = odd == s ? e : hipStreamSynchronize(odd);
     return err.load() != (int)hipSuccess ? (hipError_t)err.load() : e != hipSuccess ? e : e2;
 }
 
@@ -319,7 +337,7 @@ inline hipError_t host_copy(int device, hipStream_t s, const HostPart *parts, in
         total += parts[p].host ? parts[p].bytes : 0;
     for (int p = 0; p < nparts && total >= HOST_MIN; p++)
         known = known || (parts[p].host && runtime_array(parts[p].host));
-    const bool sliced = total >= HOST_MIN && !known;
+    const bool sliced = total >= HOST_MIN && !known && (down || total < HOST_UP_PLAIN || total >= HOST_UP_MANY);
     HostPool &pool = host_pool();
     std::unique_lock<std::mutex> lock(pool.mu, std::defer_lock);
     if (sliced) {
