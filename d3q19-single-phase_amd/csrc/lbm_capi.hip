@@ -863,9 +863,9 @@ int lbm_destroy(lbm_channel *h)
         (void)hipEventDestroy(h->ev[0]);
     if (h->ev[1])
         (void)hipEventDestroy(h->ev[1]);
+    host_pool().release(); // before the handle's own stream goes
     if (h->stream)
         (void)hipStreamDestroy(h->stream);
-    host_pool().release();
     delete h;
     return LBM_OK;
 }
@@ -2801,9 +2801,9 @@ int lbm_trainer_destroy(lbm_trainer *t)
         if (p)
             (void)hipFree(p);
     small_free(t->small, t->small_pinned);
+    host_pool().release(); // before the trainer's own stream goes
     if (t->stream)
         (void)hipStreamDestroy(t->stream);
-    host_pool().release();
     delete t;
     return LBM_OK;
 }

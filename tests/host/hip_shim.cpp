@@ -14,10 +14,13 @@ int shim_host_mallocs = 0;           // hipHostMalloc calls for 4 MiB and more s
 int shim_launches = 0;               // kernels launched so far
 int shim_copies = 0;                 // hipMemcpyAsync calls so far
 int shim_streams = 0;                // streams created so far
+int shim_last_gone = 0;              // number, in the order of creation, of the stream destroyed last
 int shim_fail_query = 0;             // hipStreamQuery: so many calls fail ...
 int shim_fail_query_from = 0;        // ... once so many kernels have been launched
 unsigned long long shim_fail_new = 0; // operator new of exactly so many bytes throws
 unsigned long long shim_malloc_bytes = 0; // bytes asked of hipMalloc so far
+
+static void *streams[64]; // the latest ones, by number
 
 static void *real(const char *name)
 {
@@ -61,9 +64,22 @@ int hipMemcpyAsync(void *dst, const void *src, size_t bytes, int kind, void *str
 
 int hipStreamCreateWithFlags(void **stream, unsigned flags)
 {
-    shim_streams++;
     static auto f = (int (*)(void **, unsigned))real("hipStreamCreateWithFlags");
-    return f(stream, flags);
+    const int rc = f(stream, flags);
+    if (rc == 0)
+        streams[shim_streams++ % 64] = *stream;
+    return rc;
+}
+
+int hipStreamDestroy(void *stream)
+{
+    for (int k = shim_streams - 1; k >= 0 && k > shim_streams - 64; k--)
+        if (streams[k % 64] == stream) {
+            shim_last_gone = k;
+            break;
+        }
+    static auto f = (int (*)(void *))real("hipStreamDestroy");
+    return f(stream);
 }
 
 struct Dim3 {
