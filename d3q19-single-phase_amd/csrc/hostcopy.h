@@ -53,8 +53,8 @@ constexpr size_t HOST_UP_ALL = 96u << 20;
 
 // Threads for a copy of `total` bytes: one (no thread is started) for downloads
 // below 8 MiB and uploads below 24 MiB.  Two keep up with the link where the
-// array's pages are there, as an upload's are (11.5 MB of samples 0.46 ms with
-// one, 0.52 with four); more share the faults of a new array (11.2 MB of fields
+// array's pages are there, as an upload's are (11.5 MB 0.46 ms with one, 0.52
+// with four); more share the faults of a new array (11.2 MB of fields
 // into one 1 570 us with two, 1 060 with four; 28 MB of viscosities 837 us with
 // three, 780 with six).
 inline int host_workers(size_t total, bool down)
@@ -331,9 +331,10 @@ struct HostPart {
     size_t bytes;
 };
 
-// The parts one after another, `down` from the device or up to it; returns
-// when the copy has finished.
-inline hipError_t host_copy(int device, hipStream_t s, const HostPart *parts, int nparts, bool down)
+// The parts one after another, `down` from the device or up to it, by at most
+// `most` threads; returns when the copy has finished.
+inline hipError_t host_copy(int device, hipStream_t s, const HostPart *parts, int nparts, bool down,
+                            int most = HOST_WORKERS)
 {
     size_t total = 0;
     bool known = false;
@@ -350,7 +351,7 @@ inline hipError_t host_copy(int device, hipStream_t s, const HostPart *parts, in
         if (e != hipSuccess)
             return e;
     }
-    const int workers = host_workers(total, down);
+    const int workers = std::min(most, host_workers(total, down));
     if (!sliced || !lock.try_lock() || !pool.ready(device, workers)) {
         for (int p = 0; p < nparts; p++)
             if (parts[p].host) {

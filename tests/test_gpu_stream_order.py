@@ -27,7 +27,7 @@ for life in range(4):
             tr.add_samples(x, y)
             fx, fy = tr.samples()  # 18.5 MB
             assert np.array_equal(fx, x) and np.array_equal(fy, y)
-    assert get("shim_streams") - first == 2
+    assert get("shim_streams") - first == (2 if life % 2 == 0 else 1)
     assert get("shim_last_gone") == first, "the handle's own stream did not go last"
 """
 
