@@ -60,7 +60,7 @@ struct StepArgs {
     const void *src; // P_k
     void *dst;       // P_{k+1}
     const double *rho, *ux, *uy, *uz;
-    const uint8_t *inside; // mode + 4: 1 at nodes inside a particle
+    const void *inside; // mode + 4: InsideFlag<P>, 1 at nodes inside a particle
     double rho_off;
     RatesD r;
     const float *mlp;  // learned closure parameters (mode bit 8), see mlp.h

@@ -395,7 +395,7 @@ __device__ __forceinline__ void step_node(const StepArgs &a)
     // a node inside a particle is computed like the others (its gather
     // issues with the flag load instead of waiting for it) but not stored
     if constexpr ((MODE & 4) != 0)
-        active = active && !a.inside[n];
+        active = active && !((const InsideFlag<P> *)a.inside)[n];
     const Nbr b = make_nbr(n, a.g);
     const S *__restrict__ src = (const S *)a.src;
     S *__restrict__ dst = (S *)a.dst;

@@ -2311,6 +2311,18 @@ static int part_alloc(Part *pt, void **p, size_t bytes)
     return LBM_OK;
 }
 
+// The collision's flags after beads_links.
+static int particles_inside(lbm_channel *h)
+{
+    const PartGeom &pg = h->part->pg;
+    const PartState &ps = h->part->ps;
+    const hipError_t e = h->prec == LBM_FP64   ? PartLaunch<0>::inside(pg, ps, h->stream)
+                         : h->prec == LBM_FP32 ? PartLaunch<1>::inside(pg, ps, h->stream)
+                         : h->prec == LBM_FP16 ? PartLaunch<2>::inside(pg, ps, h->stream)
+                                               : PartLaunch<3>::inside(pg, ps, h->stream);
+    return dispatch_err(e, "beads_links");
+}
+
 int lbm_particles_create(lbm_channel *h, const lbm_particle_config *pc, const double *pos, const double *vel,
                          const double *omg)
 {
@@ -2395,7 +2407,8 @@ int lbm_particles_create(lbm_channel *h, const lbm_particle_config *pc, const do
     A((void **)&ps.VWnew, 6 * np * sizeof(double));
     A((void **)&ps.nsteps_done, sizeof(int));
     A((void **)&ps.solid, h->g.N * sizeof(int));
-    A((void **)&ps.inside, h->g.N);
+    const size_t inside_bytes = h->g.N * (h->elem == 2 ? sizeof(InsideFlag<2>) : sizeof(InsideFlag<0>));
+    A((void **)&ps.inside, inside_bytes);
     A((void **)&ps.link_node, nl * sizeof(int));
     A((void **)&ps.link_dir, nl);
     A((void **)&ps.link_q, nl * sizeof(double));
@@ -2419,14 +2432,14 @@ int lbm_particles_create(lbm_channel *h, const lbm_particle_config *pc, const do
     HIP_TRY(hipMemsetAsync(ps.nsteps_done, 0, sizeof(int), h->stream));
     HIP_TRY(hipMemsetAsync(ps.overflow, 0, sizeof(int), h->stream));
     HIP_TRY(hipMemsetAsync(ps.solid, 0xff, h->g.N * sizeof(int), h->stream)); // -1: fluid
-    HIP_TRY(hipMemsetAsync(ps.inside, 0, h->g.N, h->stream));
+    HIP_TRY(hipMemsetAsync(ps.inside, 0, inside_bytes, h->stream));
     HIP_TRY(hipMemsetAsync(ps.fill_count, 0, np * sizeof(int), h->stream));
     HIP_TRY(hipMemsetAsync(ps.link_count, 0, np * sizeof(int), h->stream));
     h->part = pt;
     h->ave_pending = false;
     rc = dispatch_err(part_classify(pg, ps, 1, h->stream), "beads_links");
     if (!rc)
-        rc = dispatch_err(part_inside(pg, ps, h->stream), "beads_links");
+        rc = particles_inside(h);
     if (rc)
         return rc;
     int ovf = 0;
@@ -2468,7 +2481,7 @@ int lbm_beads_links(lbm_channel *h)
 {
     CHECK_P(h);
     const int rc = dispatch_err(part_classify(h->part->pg, h->part->ps, 0, h->stream), "beads_links");
-    return rc ? rc : dispatch_err(part_inside(h->part->pg, h->part->ps, h->stream), "beads_links");
+    return rc ? rc : particles_inside(h);
 }
 
 int lbm_beads_filling(lbm_channel *h)

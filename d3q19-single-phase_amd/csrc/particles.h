@@ -61,7 +61,7 @@ struct PartState {
     double *VWnew;                 // new velocities, then angular velocities, until committed (6*np)
     int *nsteps_done;              // 0 before the first move (Euler start)
     int *solid;                    // N: the particle at a node, -1 fluid, -2 - p uncovered by p and not refilled
-    uint8_t *inside;               // N: solid >= 0, the flags the collision reads (part_inside)
+    void *inside;                  // N InsideFlag: solid >= 0, the flags the collision reads (PartLaunch::inside)
     int *link_node;                // np*maxlink
     signed char *link_dir;         // np*maxlink
     double *link_q;                // np*maxlink
@@ -126,13 +126,13 @@ struct PartLaunch {
     // fractions and the settling of refilled nodes to the next bounce-back
     static hipError_t ibb(const PartGeom &pg, const PartState &ps, void *L, bool next, hipStream_t s);
     static hipError_t refill(const PartGeom &pg, const PartState &ps, void *L, hipStream_t s);
-    // the refill without its settling, and part_inside
+    // ps.inside after part_classify
+    static hipError_t inside(const PartGeom &pg, const PartState &ps, hipStream_t s);
+    // the refill without its settling, and inside
     static hipError_t refill_inside(const PartGeom &pg, const PartState &ps, void *L, hipStream_t s);
 };
 
 hipError_t part_classify(const PartGeom &pg, const PartState &ps, int first, hipStream_t s);
-// ps.inside after part_classify
-hipError_t part_inside(const PartGeom &pg, const PartState &ps, hipStream_t s);
 // macrovar's solid branch: fields at nodes inside particles
 hipError_t part_solid_fields(const PartGeom &pg, const PartState &ps, double rho_off, double *rho, double *ux,
                              double *uy, double *uz, hipStream_t s);

@@ -868,19 +868,25 @@ __global__ void __launch_bounds__(PBLOCK) k_p_refill(PartGeom pg, PartState ps, 
 
 // The collision's flags where the last classification can have changed the
 // sign of solid: particle p's box before it and its box now.
+template <int P>
 __device__ inline void inside_of(const PartGeom &pg, const PartState &ps, int p)
 {
+    InsideFlag<P> *const inside = (InsideFlag<P> *)ps.inside;
     for (int old = 0; old < 2; old++) {
         const BoxNodes box(sphere_box(pg, ps.X + 3 * ((size_t)old * pg.np + p), 0));
         for (int e = threadIdx.x; e < box.total; e += BOXBLOCK) {
             int ix, iy, iz;
             const uint32_t n = box.at(e, pg.g, ix, iy, iz);
-            ps.inside[n] = ps.solid[n] >= 0;
+            inside[n] = ps.solid[n] >= 0;
         }
     }
 }
 
-__global__ void __launch_bounds__(BOXBLOCK) k_p_inside(PartGeom pg, PartState ps) { inside_of(pg, ps, blockIdx.x); }
+template <int P>
+__global__ void __launch_bounds__(BOXBLOCK) k_p_inside(PartGeom pg, PartState ps)
+{
+    inside_of<P>(pg, ps, blockIdx.x);
+}
 
 // What the main loop does between two steps besides the bounce-back: the
 // refill and the collision's flags, neither of which reads what the other
@@ -891,14 +897,15 @@ __global__ void __launch_bounds__(BOXBLOCK) k_p_refill_inside(PartGeom pg, PartS
     if ((int)blockIdx.x < pg.np)
         refill_of<P, BOXBLOCK>(pg, ps, (typename Prec<P>::S *)Lv, blockIdx.x);
     else
-        inside_of(pg, ps, (int)blockIdx.x - pg.np);
+        inside_of<P>(pg, ps, (int)blockIdx.x - pg.np);
 }
 
 } // namespace
 
-hipError_t part_inside(const PartGeom &pg, const PartState &ps, hipStream_t s)
+template <int P>
+hipError_t PartLaunch<P>::inside(const PartGeom &pg, const PartState &ps, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_p_inside, dim3(pg.np), dim3(BOXBLOCK), 0, s, pg, ps);
+    hipLaunchKernelGGL((k_p_inside<P>), dim3(pg.np), dim3(BOXBLOCK), 0, s, pg, ps);
     return hipGetLastError();
 }
 
