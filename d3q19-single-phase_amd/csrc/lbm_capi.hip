@@ -2656,20 +2656,16 @@ int lbm_particles_links(lbm_channel *h, int *maxlink, int *counts, int *node, in
     if (maxlink)
         *maxlink = pg.maxlink;
     const size_t nl = (size_t)pg.np * pg.maxlink;
-    if (counts)
-        HIP_TRY(hipMemcpyAsync(counts, ps.link_count, pg.np * sizeof(int), hipMemcpyDeviceToHost, h->stream));
-    if (node)
-        HIP_TRY(hipMemcpyAsync(node, ps.link_node, nl * sizeof(int), hipMemcpyDeviceToHost, h->stream));
-    if (q)
-        HIP_TRY(hipMemcpyAsync(q, ps.link_q, nl * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    if (dir) {
-        std::vector<signed char> d(nl);
-        HIP_TRY(hipMemcpyAsync(d.data(), ps.link_dir, nl, hipMemcpyDeviceToHost, h->stream));
-        HIP_TRY(hipStreamSynchronize(h->stream));
-        for (size_t k = 0; k < nl; k++)
-            dir[k] = d[k];
-    }
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    std::vector<signed char> d(dir ? nl : 0);
+    const HostPart parts[4] = {{counts, ps.link_count, pg.np * sizeof(int)},
+                               {node, ps.link_node, nl * sizeof(int)},
+                               {q, ps.link_q, nl * sizeof(double)},
+                               {dir ? d.data() : nullptr, ps.link_dir, nl}};
+    const int rc = copy_parts(h, parts, 4, true, "lbm_particles_links");
+    if (rc)
+        return rc;
+    for (size_t k = 0; k < d.size(); k++)
+        dir[k] = d[k];
     return check_overflow(h, "lbm_particles_links");
 }
 
