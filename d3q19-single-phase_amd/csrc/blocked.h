@@ -191,20 +191,23 @@ constexpr long BLOCK_MAX_SLABS = 32;
 // Pairs of steps run as single steps when the lattice is small or the sweep's
 // chunks are.
 //
-// A lattice of up to BLOCK_MIN_LATTICE_BYTES, or most of one, stays in the
-// last-level cache anyway, and the sweep only adds launches and halo slabs.
-// us per step, sweep against single steps: FP64 10 MB (32x64x32) 11.7 / 6.1,
-// 53 MB 40 / 24, 184 MB (97x150x83) 81 / 74, 280 MB 106 / 107, 342 MB 126 /
-// 129, 478 MB 172 / 189; FP32 27 MB 28 / 13, 140 MB 60 / 56, 239 MB 93 /
-// 90-101, 294 MB 111 / 107, 538 MB 185 / 194.
+// A lattice of up to BLOCK_MIN_LATTICE_BYTES stays in the last-level cache
+// anyway, and the sweep only adds launches and halo slabs.  us per step, sweep
+// against single steps: FP64 10 MB (32x64x32) 11.7 / 6.1, 53 MB 40 / 24, 184 MB
+// (97x150x83) 81 / 57, 240 MB 84-91 / 75-85, 270 MB 92-101 / 85-98; 274 MB 94-
+// 101 / 87-108, 278 MB (seven shapes) 93-104 / 99-112, 286 MB 97-111 / 98-114, 294
+// MB 100-113 / 102-112, 342 MB 126 / 129, 478 MB 172 / 189.  FP32 27 MB 28 / 13,
+// 140 MB 60 / 47, 240 MB 89-106 / 77-88, 270 MB 92-116 / 85-102; 200x200 by 274 MB
+// 99 / 104, 278 MB 102 / 106, 286 MB 104 / 107, 294 MB 107 / 105, 538 MB 185 / 194.
 //
 // A chunk of K slabs of less than BLOCK_MIN_CHUNK_BYTES (K is at most 32) makes
 // launches too short to hide their start and end: FP64 66 MB (45x301x180) 150
 // / 135, 75 MB 198 / 190, 126 MB 207 / 217, 188 MB 292 / 325; FP32 33 MB
-// (45x301x180) 95 / 73, 63 MB 116 / 107, 81 MB 297 / 281, 94 MB 163 / 159-271 /
-// 274, 172 MB 464 / 475, 186 MB 502 / 529.
-constexpr uint64_t BLOCK_MIN_LATTICE_BYTES = 300000000ull;
-constexpr uint64_t BLOCK_MIN_CHUNK_BYTES = 90000000ull;
+// (45x301x180) 95 / 73, 63 MB 116 / 107, 81 MB 297 / 281, 87.8 MB (94x384x160) 161
+// / 157, 89.7 MB (96x384x192) 190 / 194, 94 MB 163 / 159-271 / 274, 172 MB 464 /
+// 475, 186 MB 502 / 529.
+constexpr uint64_t BLOCK_MIN_LATTICE_BYTES = 272000000ull;
+constexpr uint64_t BLOCK_MIN_CHUNK_BYTES = 88000000ull;
 
 // The sweep lbm_create chooses for a lattice of elem-byte values: axis 2 (z)
 // or 1 (y), K slabs per chunk (0: single steps only) and W rows per window

@@ -184,8 +184,8 @@ int lbm_avedensity(lbm_channel *h, double *rhomean);
  * the single-step path's bit for bit.  The environment variables
  * LBM_BLOCK_AXIS=z|y and LBM_BLOCK_PLANES (read by lbm_create) set the axis
  * and the slabs per chunk (at most 32), 0 turns the sweep off; lbm_block_info
- * and lbm_block_rows report the choice.  Lattices of at most 300 MB, and those whose
- * slabs are so small that a chunk holds less than 90 MB, run their steps one
+ * and lbm_block_rows report the choice.  Lattices of at most 272 MB, and those whose
+ * slabs are so small that a chunk holds less than 88 MB, run their steps one
  * by one, which measures faster there, unless one of the sweep's variables is
  * set; lbm_block_pairs tells which it is. */
 int lbm_run(lbm_channel *h, int nsteps);
