@@ -62,28 +62,32 @@ inline uint32_t block_ring_rows(const Geom &g, int axis, uint32_t W)
     return block_windowed(g, axis, W) ? W + 2 : block_geom(g, axis).nr;
 }
 
-// Nodes of a z slab modulo a wave (BlockArgs::res), 0 for y slabs and row
-// windows, whose rows are not contiguous in the lattice.
-inline uint32_t block_residue(const Geom &g, int axis, uint32_t W)
+// Nodes of a z slab modulo a wave (BlockArgs::res), 0 where slabs of elem-byte
+// values are whole cache lines as they are (130x200x200 in FP64: 283 us per step,
+// 287 shifted), and for y slabs and row windows, whose rows are not contiguous in
+// the lattice.
+inline uint32_t block_residue(const Geom &g, int axis, uint32_t W, size_t elem)
 {
-    return axis == 2 && !block_windowed(g, axis, W) ? g.lx * g.ly % WAVE_LANES : 0u;
+    if (axis != 2 || block_windowed(g, axis, W) || (uint64_t)g.lx * g.ly * elem % 128 == 0)
+        return 0u;
+    return g.lx * g.ly % WAVE_LANES;
 }
 
 // Ring slots, elements of one population of a ring slab (lx * ring rows nodes
 // and their shift, rounded up to whole waves so that slots start on cache
 // lines) and buffer sizes in elements.
 inline uint32_t block_ring_slots(uint32_t K) { return K + 2; }
-inline uint64_t block_ring_slab(const Geom &g, int axis, uint32_t W)
+inline uint64_t block_ring_slab(const Geom &g, int axis, uint32_t W, size_t elem)
 {
-    return slab_padded(g.lx * block_ring_rows(g, axis, W) + (block_residue(g, axis, W) ? WAVE_LANES - 1 : 0u));
+    return slab_padded(g.lx * block_ring_rows(g, axis, W) + (block_residue(g, axis, W, elem) ? WAVE_LANES - 1 : 0u));
 }
-inline uint64_t block_ring_elems(const Geom &g, int axis, uint32_t K, uint32_t W = 0)
+inline uint64_t block_ring_elems(const Geom &g, int axis, uint32_t K, uint32_t W = 0, size_t elem = 2)
 {
-    return 19ull * block_ring_slots(K) * block_ring_slab(g, axis, W);
+    return 19ull * block_ring_slots(K) * block_ring_slab(g, axis, W, elem);
 }
-inline uint64_t block_head_elems(const Geom &g, int axis, uint32_t W = 0)
+inline uint64_t block_head_elems(const Geom &g, int axis, uint32_t W = 0, size_t elem = 2)
 {
-    return 19ull * 2 * block_ring_slab(g, axis, W);
+    return 19ull * 2 * block_ring_slab(g, axis, W, elem);
 }
 
 // The force of one of the two steps of a pair: rates with the uniform force
@@ -97,17 +101,17 @@ struct StepForce {
 
 // Launch list of one pair: step t with force f0, step t+1 with force f1,
 // whole slabs (W = 0) or row windows of W rows; the lattices' population
-// stride (0: the node count).
+// stride (0: the node count) and the bytes of a value.
 inline std::vector<BlockArgs> block_schedule(const Geom &g, int axis, const StepForce &f0, const StepForce &f1,
                                              uint32_t K, uint32_t W, void *lat_in, void *lat_out, void *ring,
-                                             void *head, uint64_t lat_stride = 0)
+                                             void *head, uint64_t lat_stride = 0, size_t elem = 2)
 {
     const uint64_t ls = lat_stride ? lat_stride : g.N;
     const BlockGeom bg = block_geom(g, axis);
     const uint32_t ns = bg.ns, nr = bg.nr, slots = block_ring_slots(K);
     const bool win = block_windowed(g, axis, W);
-    const uint64_t rslab = block_ring_slab(g, axis, W);
-    const uint32_t res = block_residue(g, axis, W);
+    const uint64_t rslab = block_ring_slab(g, axis, W, elem);
+    const uint32_t res = block_residue(g, axis, W, elem);
     const PlaneStore full_in = {lat_in, ls, ns, make_fastdiv(ns), bg.lat_slab_stride, bg.lat_row_stride, nullptr, 0,
                                 0, 0, 0};
     const PlaneStore full_out = {lat_out, ls, ns, make_fastdiv(ns), bg.lat_slab_stride, bg.lat_row_stride, nullptr, 0,

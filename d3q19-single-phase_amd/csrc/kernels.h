@@ -170,31 +170,40 @@ __host__ __device__ inline uint32_t ring_slot(const PlaneStore &st, uint32_t s)
 constexpr uint32_t WAVE_LANES = 64;
 
 // Elements by which slab s starts past a multiple of WAVE_LANES.
-__host__ __device__ inline uint32_t slab_shift(uint32_t res, uint32_t s) { return (s * res) & (WAVE_LANES - 1); }
+template <bool RES = true>
+__host__ __device__ inline uint32_t slab_shift(uint32_t res, uint32_t s)
+{
+    return RES ? (s * res) & (WAVE_LANES - 1) : 0u;
+}
 
-// Slab s as a reader sees it.
+// Slab s as a reader sees it.  RES (here and below): whether the slabs may be
+// shifted; without, the sweep's scalar code before its loads is 22 instructions
+// and a branch shorter (us per FP32 step of 256^3: 405.8 with, 403.6 without).
+template <bool RES = true>
 __host__ __device__ inline PlaneRef plane_read(const PlaneStore &st, uint32_t s)
 {
     const uint32_t h = s - (uint32_t)st.head_lo; // wraps for s < head_lo
     if (st.head != nullptr && h < st.head_n)
-        return PlaneRef{st.head, st.head_stride, (uint64_t)h * st.slab_stride + slab_shift(st.res, s), st.row_stride};
-    return PlaneRef{st.ring, st.ring_stride, (uint64_t)ring_slot(st, s) * st.slab_stride + slab_shift(st.res, s),
+        return PlaneRef{st.head, st.head_stride, (uint64_t)h * st.slab_stride + slab_shift<RES>(st.res, s), st.row_stride};
+    return PlaneRef{st.ring, st.ring_stride, (uint64_t)ring_slot(st, s) * st.slab_stride + slab_shift<RES>(st.res, s),
                     st.row_stride};
 }
 
 // Slab s as a writer stores it: always its ring slot, and also the head copy
 // when s is a head slab (plane_write_head; buf = nullptr otherwise).
+template <bool RES = true>
 __host__ __device__ inline PlaneRef plane_write(const PlaneStore &st, uint32_t s)
 {
-    return PlaneRef{st.ring, st.ring_stride, (uint64_t)ring_slot(st, s) * st.slab_stride + slab_shift(st.res, s),
+    return PlaneRef{st.ring, st.ring_stride, (uint64_t)ring_slot(st, s) * st.slab_stride + slab_shift<RES>(st.res, s),
                     st.row_stride};
 }
 
+template <bool RES = true>
 __host__ __device__ inline PlaneRef plane_write_head(const PlaneStore &st, uint32_t s)
 {
     const uint32_t h = s - (uint32_t)st.head_lo;
     if (st.head != nullptr && h < st.head_n)
-        return PlaneRef{st.head, st.head_stride, (uint64_t)h * st.slab_stride + slab_shift(st.res, s), st.row_stride};
+        return PlaneRef{st.head, st.head_stride, (uint64_t)h * st.slab_stride + slab_shift<RES>(st.res, s), st.row_stride};
     return PlaneRef{nullptr, 0, 0, 0};
 }
 
@@ -204,11 +213,11 @@ __host__ __device__ inline PlaneRef plane_write_head(const PlaneStore &st, uint3
 // waves (slabp = slab rounded up to a multiple of 64), so every wave lies in
 // one slab and the slab's buffers and offsets are the same for all its lanes.
 // Thread t works on node t % slabt - slab_shift(res, s) of the launch's slab t /
-// slabt (block_thread_slab, block_thread_node).  When whole z slabs of lx * ly nodes do not fill cache lines, res is
-// that count modulo 64 and slabt leaves room for the shift: a wave's nodes
-// then start on a line of the lattice, and of the ring, whose slots hold each
-// slab at the same shift.  Without it every wave stored two partial lines a
-// population (us per step without / with, single steps: 191x401x255 FP64 1 160
+// slabt (block_thread_slab, block_thread_node).  When whole z slabs of lx * ly
+// nodes do not fill cache lines (block_residue), res is that count modulo 64 and
+// slabt leaves room for the shift: a wave's nodes then start on a line of the
+// lattice, and of the ring, whose slots hold each slab at the same shift.
+// Without it every wave stored two partial lines a population (us per step without / with, single steps: 191x401x255 FP64 1 160
 // / 964, 1 081; FP32 565 / 502, 529; 98x301x201 FP64 335 / 316, 337).
 // Otherwise res = 0 and slabt = slabp.
 // per_node: the body force is evaluated at every node as in step mode 16
@@ -259,18 +268,20 @@ __host__ __device__ inline uint32_t block_plane(const BlockArgs &a, uint32_t sl)
 // and its node of it, slab sb of the lattice: beyond a.slab, also below the
 // slab's shift, where the difference wraps, the thread has none.
 __host__ __device__ inline uint32_t block_thread_slab(const BlockArgs &a, uint32_t t) { return fdiv(t, a.dslabt); }
+template <bool RES = true>
 __host__ __device__ inline uint32_t block_thread_node(const BlockArgs &a, uint32_t t, uint32_t sl, uint32_t sb)
 {
-    return t - sl * a.slabt - slab_shift(a.res, sb);
+    return t - sl * a.slabt - slab_shift<RES>(a.res, sb);
 }
 
 // The source slabs of slab s: index c + 1 holds slab s - c, for the sweep-axis
 // component c of a velocity (slabs s + 1, s, s - 1).
+template <bool RES = true>
 __host__ __device__ inline void block_planes(const BlockArgs &a, uint32_t s, PlaneRef (&pl)[3])
 {
-    pl[0] = plane_read(a.src, s + 1 == a.ns ? 0 : s + 1);
-    pl[1] = plane_read(a.src, s);
-    pl[2] = plane_read(a.src, s == 0 ? a.ns - 1 : s - 1);
+    pl[0] = plane_read<RES>(a.src, s + 1 == a.ns ? 0 : s + 1);
+    pl[1] = plane_read<RES>(a.src, s);
+    pl[2] = plane_read<RES>(a.src, s == 0 ? a.ns - 1 : s - 1);
 }
 
 // A node's own part of its gather addresses: element offsets within a slab

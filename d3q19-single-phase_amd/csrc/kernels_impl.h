@@ -571,7 +571,8 @@ constexpr int plane_block() { return P == 1 ? 512 : (NT ? 512 : 256); }
 
 // FP: the body force per node (mode 16 of k_step: a.fc for the collision,
 // a.fm for the fused fields), with the same arithmetic as k_step<P, 16>.
-template <int P, int AXIS, int NT, int FP>
+// RES: z slabs shifted onto cache lines (a.res != 0).
+template <int P, int AXIS, int NT, int FP, bool RES>
 __global__ void __launch_bounds__((plane_block<P, NT>())) k_step_planes(BlockArgs a)
 {
     using T = typename Prec<P>::T;
@@ -579,16 +580,14 @@ __global__ void __launch_bounds__((plane_block<P, NT>())) k_step_planes(BlockArg
     // the wave's slab, uniform across its lanes (slabs are padded to whole
     // waves), so the slab buffers and offsets below stay in scalar registers
     const uint32_t sl = __builtin_amdgcn_readfirstlane(block_thread_slab(a, t));
-    if (sl >= a.count)
-        return;
-    const uint32_t sb = block_plane(a, sl);
-    const uint32_t w = block_thread_node(a, t, sl, sb);
-    if (w >= a.slab)
+    const uint32_t sb = block_plane(a, sl); // of no slab from a.count on
+    const uint32_t w = block_thread_node<RES>(a, t, sl, sb);
+    if (sl >= a.count || w >= a.slab)
         return;
     const BlockRow br = block_row(a, w);
     const uint32_t ix = br.ix;
     PlaneRef pl[3];
-    block_planes(a, sb, pl);
+    block_planes<RES>(a, sb, pl);
     const BlockLane l = block_lane(ix, br.rs, a.src_nr, (uint32_t)a.src.row_stride, a.g.lx);
 
     T f[19];
@@ -626,10 +625,10 @@ __global__ void __launch_bounds__((plane_block<P, NT>())) k_step_planes(BlockArg
         mrt_collide_delta(f, rho9, ux9, uy9, uz9, T(0), djx, djy, djz, rt);
     }
 
-    const PlaneRef d = plane_write(a.dst, sb);
+    const PlaneRef d = plane_write<RES>(a.dst, sb);
     const uint32_t e = (br.rl + a.dst_r0) * (uint32_t)d.row_stride + ix; // head and ring rows share the stride
     block_store<P, NT>(d, e, f, std::make_integer_sequence<int, 19>{});
-    const PlaneRef hd = plane_write_head(a.dst, sb);
+    const PlaneRef hd = plane_write_head<RES>(a.dst, sb);
     if (hd.buf != nullptr)
         block_store<P, 0>(hd, e, f, std::make_integer_sequence<int, 19>{});
 }
@@ -1582,18 +1581,25 @@ hipError_t Launch<P>::step_planes(const BlockArgs &a, int axis, hipStream_t s)
 {
     const uint32_t PB = a.nt ? plane_block<P, 1>() : plane_block<P, 0>();
     const dim3 grid((uint32_t)(((uint64_t)a.slabt * a.count + PB - 1) / PB)), blk(PB);
-    const int v = (axis == 2 ? 4 : axis == 1 ? 0 : -8) + (a.nt ? 2 : 0) + (a.per_node ? 1 : 0);
+    const int v = (axis == 2 ? (a.res ? 8 : 4) : axis == 1 ? 0 : -16) + (a.nt ? 2 : 0) + (a.per_node ? 1 : 0);
+#define PLANES_CASE(V, AXIS, NT, FP, RES) \
+    case V: hipLaunchKernelGGL((k_step_planes<P, AXIS, NT, FP, RES>), grid, blk, 0, s, a); break
     switch (v) {
-    case 0: hipLaunchKernelGGL((k_step_planes<P, 1, 0, 0>), grid, blk, 0, s, a); break;
-    case 1: hipLaunchKernelGGL((k_step_planes<P, 1, 0, 1>), grid, blk, 0, s, a); break;
-    case 2: hipLaunchKernelGGL((k_step_planes<P, 1, 1, 0>), grid, blk, 0, s, a); break;
-    case 3: hipLaunchKernelGGL((k_step_planes<P, 1, 1, 1>), grid, blk, 0, s, a); break;
-    case 4: hipLaunchKernelGGL((k_step_planes<P, 2, 0, 0>), grid, blk, 0, s, a); break;
-    case 5: hipLaunchKernelGGL((k_step_planes<P, 2, 0, 1>), grid, blk, 0, s, a); break;
-    case 6: hipLaunchKernelGGL((k_step_planes<P, 2, 1, 0>), grid, blk, 0, s, a); break;
-    case 7: hipLaunchKernelGGL((k_step_planes<P, 2, 1, 1>), grid, blk, 0, s, a); break;
+        PLANES_CASE(0, 1, 0, 0, false);
+        PLANES_CASE(1, 1, 0, 1, false);
+        PLANES_CASE(2, 1, 1, 0, false);
+        PLANES_CASE(3, 1, 1, 1, false);
+        PLANES_CASE(4, 2, 0, 0, false);
+        PLANES_CASE(5, 2, 0, 1, false);
+        PLANES_CASE(6, 2, 1, 0, false);
+        PLANES_CASE(7, 2, 1, 1, false);
+        PLANES_CASE(8, 2, 0, 0, true);
+        PLANES_CASE(9, 2, 0, 1, true);
+        PLANES_CASE(10, 2, 1, 0, true);
+        PLANES_CASE(11, 2, 1, 1, true);
     default: return hipErrorInvalidValue;
     }
+#undef PLANES_CASE
     return hipGetLastError();
 }
 

@@ -1572,8 +1572,8 @@ static StepForce step_force_of(const lbm_channel *h, const ForceSpec &fc, const 
 static int run_pair_with(lbm_channel *h, const StepForce &f0, const StepForce &f1)
 {
     if (!h->bring) {
-        const size_t rb = block_ring_elems(h->g, h->baxis, h->bK, h->bW) * h->elem,
-                     hb = block_head_elems(h->g, h->baxis, h->bW) * h->elem;
+        const size_t rb = block_ring_elems(h->g, h->baxis, h->bK, h->bW, h->elem) * h->elem,
+                     hb = block_head_elems(h->g, h->baxis, h->bW, h->elem) * h->elem;
         hipError_t e = hipMalloc(&h->bring, rb);
         if (e == hipSuccess)
             e = hipMalloc(&h->bhead, hb);
@@ -1587,7 +1587,7 @@ static int run_pair_with(lbm_channel *h, const StepForce &f0, const StepForce &f
     }
     const auto launches =
         block_schedule(h->g, h->baxis, f0, f1, h->bK, h->bW, h->lat[h->cur], h->lat[1 - h->cur], h->bring,
-                       h->bhead, h->g.S);
+                       h->bhead, h->g.S, h->elem);
     for (const BlockArgs &a : launches) {
         int rc = dispatch_err(PREC_CALL(h, step_planes, a, h->baxis, h->stream), "collision (blocked sweep)");
         if (rc)
@@ -2167,7 +2167,8 @@ int lbm_device_bytes(lbm_channel *h, size_t *bytes)
     if (h->stage)
         b += STAGE_BYTES;
     if (h->bring)
-        b += (block_ring_elems(h->g, h->baxis, h->bK, h->bW) + block_head_elems(h->g, h->baxis, h->bW)) * h->elem;
+        b += (block_ring_elems(h->g, h->baxis, h->bK, h->bW, h->elem) +
+              block_head_elems(h->g, h->baxis, h->bW, h->elem)) * h->elem;
     b += (2 * RED_BLOCKS + (size_t)PLANE_CHUNKS * NPLANE * h->g.lx + 2 + 2 * NPLANE * (size_t)h->g.lx) * sizeof(double) + ERR_BYTES;
     *bytes = b;
     return LBM_OK;

@@ -5,7 +5,7 @@
 // threads to nodes (block_thread_slab, block_thread_node: z slabs shifted so that
 // a wave's nodes start on a line) and with populations padded to whole lines in
 // buffers of exactly that size.  Also: a wave lies in one slab, its nodes start on
-// a multiple of a wave in the lattice and in the ring, and the padding keeps its
+// a cache line of the lattice and of the ring, and the padding keeps its
 // value.  Launches nothing on a GPU.
 #define main block_check_main
 #include "block_check.hip"
@@ -27,8 +27,8 @@ static bool check_threads(uint32_t lx, uint32_t ly, uint32_t lz, uint32_t K, int
     Buf in, out, ring, head;
     in.v.assign(19 * S, PAD);
     out.v.assign(19 * S, PAD);
-    ring.v.assign(block_ring_elems(g, axis, K, W), 0);
-    head.v.assign(block_head_elems(g, axis, W), 0);
+    ring.v.assign(block_ring_elems(g, axis, K, W, elem), 0);
+    head.v.assign(block_head_elems(g, axis, W, elem), 0);
     c.bufs[0] = &in;
     c.bufs[1] = &out;
     c.bufs[2] = &ring;
@@ -38,7 +38,7 @@ static bool check_threads(uint32_t lx, uint32_t ly, uint32_t lz, uint32_t K, int
             in.v[(uint64_t)i * S + n] = c.tag(0, n, i);
     const StepForce f = {};
     const auto launches =
-        block_schedule(g, axis, f, f, K, W, in.v.data(), out.v.data(), ring.v.data(), head.v.data(), S);
+        block_schedule(g, axis, f, f, K, W, in.v.data(), out.v.data(), ring.v.data(), head.v.data(), S, elem);
     uint64_t out_writes = 0;
     for (const BlockArgs &a : launches) {
         c.reads.clear();
@@ -73,7 +73,7 @@ static bool check_threads(uint32_t lx, uint32_t ly, uint32_t lz, uint32_t K, int
             const PlaneRef d = plane_write(a.dst, sb);
             if (axis == 2 && W == 0) { // contiguous slabs: lane k of a wave stores element k of a line
                 const uint64_t e = d.off + (uint64_t)(br.rl + a.dst_r0) * d.row_stride + br.ix;
-                if ((e - t) % WAVE_LANES != 0 || d.stride % (128 / elem) != 0)
+                if ((e - t) % (128 / elem) != 0 || d.stride % (128 / elem) != 0)
                     return fail_at(lx, ly, lz, "a wave's nodes do not start on a line");
                 shifted += a.res != 0;
             }
@@ -109,7 +109,7 @@ int main()
     // windows of every kind
     const uint32_t cases[][5] = {{4, 3, 1, 2, 0},  {4, 3, 2, 2, 0},   {5, 4, 3, 2, 0},   {8, 8, 9, 4, 0},  {13, 5, 9, 4, 0},
                                  {9, 7, 12, 5, 0}, {16, 6, 10, 3, 0}, {31, 4, 8, 4, 0},  {21, 9, 7, 2, 0}, {3, 21, 17, 16, 0},
-                                 {7, 5, 33, 8, 0}, {2, 1, 5, 2, 0},   {4, 37, 11, 6, 0}, {2, 5, 75, 32, 0},
+                                 {7, 5, 33, 8, 0}, {2, 1, 5, 2, 0},   {4, 37, 11, 6, 0}, {2, 5, 75, 32, 0}, {6, 8, 9, 4, 0}, {12, 8, 7, 3, 0}, {10, 16, 5, 2, 0},
                                  {4, 7, 9, 3, 2},  {5, 8, 6, 2, 3},   {3, 10, 4, 4, 1},  {13, 5, 7, 2, 4}, {3, 11, 3, 32, 5}};
     uint32_t shifted = 0;
     for (auto &k : cases)
